@@ -4,13 +4,9 @@
 // Kernels
 //   chol_factor_kernel  One workgroup factors a diagonal block (≤128×128) in
 //                       place.  The block is held as 16×16 MFMA accumulator
-//                       tiles; wave 0 holds the diagonal tiles, waves 1–3
-//                       the rest.  For each 16-wide column block the tiles
-//                       below the diagonal become X = A·L_kk⁻ᵀ, then wave 0
-//                       factors the next diagonal tile in registers column
-//                       by column as cholUnblocked! does (sqrt, reciprocal
-//                       scale, rank-1 update; DPP broadcasts move the column)
-//                       and inverts it while waves 1–3 apply the rank-16
+//                       tiles; waves 1–3 hold them, wave 0 factors and
+//                       inverts one diagonal tile after another
+//                       (tile_factor) while waves 1–3 apply the rank-16
 //                       update C -= X_i X_jᵀ on MFMA.  The tile inverses are
 //                       kept for the panel solve.
 //   chol_solve_kernel   rdiv!(A21, LowerTriangular(A11)') (src/cholesky.jl:28,
@@ -77,19 +73,6 @@ __device__ __forceinline__ T lane_bcast(T v, int src)
 }
 
 
-
-template <typename T>
-__device__ __forceinline__ void tile_factor_rows(T a[16], T rd[16], int nvalid, int *info,
-                                                 int64_t gbase)
-{
-    const int i = threadIdx.x & 15;
-    int fneg = 16;
-    TileFactorCols<0, T>::run(a, rd, i, fneg);
-    if (fneg < 16 && fneg < nvalid && (threadIdx.x & 63) == 0 && info)
-        atomicCAS(info, 0, (int)(gbase + fneg + 1));
-#pragma unroll
-    for (int j = 0; j < 16; ++j) a[j] = j <= i ? a[j] : T(0);
-}
 
 // w <- L⁻¹ for a lower 16×16 tile L (rd = reciprocals of its diagonal), in
 // the four-column layout (w[t] = W[i][g + 4t]).  Forward elimination of
@@ -163,76 +146,80 @@ constexpr bool oslots_cover()
 }
 static_assert(oslots_cover(), "the tile slots of waves 1-3 must cover the strictly-lower tiles once");
 
-// Cholesky tile factor: slot q of wave W (wave 0: diagonal tile q).
+// LDLᴴ and Cholesky tiles: slot q of wave W (LDLᴴ's wave 0: diagonal tile q).
 template <int W>
 __host__ __device__ constexpr int dslot_bi(int q) { return W == 0 ? q : oslot_bi(W, q); }
 template <int W>
 __host__ __device__ constexpr int dslot_bj(int q) { return W == 0 ? q : oslot_bj(W, q); }
 
-// d (a diagonal tile, transposed) -= X_j X_jᵀ for X_j = tile row j of X (LDS)
-template <typename T>
-__device__ __forceinline__ void diag_update(typename PanelMfma<T>::acc_t &d, const T *X, int j)
+// Tile rows of waves 1–3, whose diagonal tiles they keep up to date until
+// wave 0 factors them: row number d of wave W (0: none).
+template <int W>
+__host__ __device__ constexpr int row_of(int d)
 {
-    typedef PanelMfma<T> M;
-    const int lane = threadIdx.x & 63;
-    const int lc = lane & 15;
-#pragma unroll
-    for (int kq = 0; kq < 4; ++kq) {
-        const int kk = (lane >> 4) + 4 * kq;
-        const T x = X[(j * 16 + lc) * kXLD + kk];
-        d = M::mma(-x, x, d);
-    }
+    return W == 1 ? (d == 0 ? 7 : d == 1 ? 2 : 0)
+         : W == 2 ? (d == 0 ? 6 : d == 1 ? 3 : 0)
+                  : (d == 0 ? 5 : d == 1 ? 4 : 1);
 }
 
-// Wave 0: factors diagonal tile j (d, transposed) in row layout through the
-// wave's LDS tile D, inverts it, leaves L (transposed) in d, the inverse in Li
-// (row-major) and, when given, LinvG / Linv32.
-template <typename T>
-__device__ __forceinline__ void diag_factor(typename PanelMfma<T>::acc_t &d, int j, int nb,
-                                            int *info, int64_t info_base, T *D, T *Li,
-                                            T *__restrict__ LinvG, float *__restrict__ Linv32)
+// Tile (bi, bj) of A transposed (lane: row bi·16 + l % 16 at columns bj·16 +
+// row(l, r)); a diagonal tile symmetric, from its lower triangle.  Rows and
+// columns past nb continue as the identity.  TS: storage type of A.
+template <typename T, typename TS>
+__device__ __forceinline__ typename PanelMfma<T>::acc_t load_tile(int nb, const TS *__restrict__ A,
+                                                                 int64_t lda, int bi, int bj)
 {
     typedef PanelMfma<T> M;
-    const int lane = threadIdx.x & 63;
-    const int lc = lane & 15;
-    const int i = lane & 15, g = lane >> 4;
+    const int lane = threadIdx.x & 63, lc = lane & 15;
+    typename M::acc_t v;
 #pragma unroll
-    for (int r = 0; r < 4; ++r) D[lc * kXLD + M::row(lane, r)] = d[r];
-    wave_order();
-    T a[16], w[4], rd[16];
-#pragma unroll
-    for (int c = 0; c < 16; ++c) a[c] = c <= i ? D[i * kXLD + c] : T(0);
-    tile_factor_rows<T>(a, rd, nb - j * 16, info, info_base + j * 16);
-    tile_inverse_rows<T>(a, rd, w);
-    wave_order();
-    if (g == 0)
-#pragma unroll
-        for (int c = 0; c < 16; ++c) D[i * kXLD + c] = a[c];
-#pragma unroll
-    for (int t = 0; t < 4; ++t) {
-        Li[i * kXLD + g + 4 * t] = w[t];
-        if (LinvG) LinvG[j * 256 + i * 16 + g + 4 * t] = w[t];
-        if (Linv32) Linv32[j * 256 + i * 16 + g + 4 * t] = float(w[t]);
+    for (int r = 0; r < 4; ++r) {
+        const int a = bi * 16 + lc, b = bj * 16 + M::row(lane, r);
+        const int gi = a > b ? a : b, gj = a > b ? b : a;
+        v[r] = gi < nb ? T(A[gi + (int64_t)gj * lda]) : (gi == gj ? T(1) : T(0));
     }
-    wave_order();
+    return v;
+}
+
+// Stores tile (bi, bj) held transposed, its lower triangle only.
+template <typename T, typename TS>
+__device__ __forceinline__ void store_tile(int nb, TS *__restrict__ A, int64_t lda, int bi, int bj,
+                                           const typename PanelMfma<T>::acc_t &v)
+{
+    typedef PanelMfma<T> M;
+    const int lane = threadIdx.x & 63, lc = lane & 15;
 #pragma unroll
-    for (int r = 0; r < 4; ++r) d[r] = D[lc * kXLD + M::row(lane, r)];
+    for (int r = 0; r < 4; ++r) {
+        const int gi = bi * 16 + lc, gj = bj * 16 + M::row(lane, r);
+        if (gi < nb && gj <= gi) A[gi + (int64_t)gj * lda] = TS(v[r]);
+    }
 }
 
 // One workgroup factors the nb×nb (nb ≤ 128) diagonal block as 16×16 MFMA
-// tiles held transposed (lane: row bi·16 + l%16 of the tile, columns
-// bj·16 + row(l, r)).  Wave 0 holds the eight diagonal tiles, waves 1–3 the
-// strictly-lower ones.  Each 16-wide step kb takes two barriers: (A) waves
-// 1–3 form the panel tiles X = A_(i,kb) L_kk⁻ᵀ while wave 0 applies the
-// previous step's update to the diagonal tiles beyond kb + 1; (B) wave 0
-// updates, factors and inverts diagonal tile kb + 1 while waves 1–3 apply
-// the rank-16 update to theirs, so the serial tile factor overlaps the
-// trailing update.  Every product is formed from the same operands in the
-// same order as the right-looking sweep cholBlocked! describes
-// (src/cholesky.jl:17-35).
+// tiles.  Waves 1–3 own the tile rows below the first (row_of), diagonal
+// tiles included, held transposed; wave 0 factors and inverts the diagonal
+// tiles one after the other (tile_factor).  Step kb:
+//   (A) waves 1–3: the panel tiles X = A_(i,kb) L_kk⁻ᵀ (rdiv!), as
+//       Xᵀ = L_kk⁻¹ A_(i,kb)ᵀ with the B operand from registers; the owner of
+//       row kb + 1 first, which at once takes X Xᵀ off its diagonal tile
+//       (both operands in registers) and hands that tile to wave 0.  Wave 0
+//       stores the tile it has factored.
+//   (B) wave 0 factors diagonal tile kb + 1; waves 1–3 apply the rank-16
+//       update (rankUpdate!), C_ijᵀ -= X_j X_iᵀ, to their tiles, their later
+//       diagonal tiles among them, and store column block kb.
+// LDS tiles are kept as the lanes hold them (element r·64 + lane: the
+// accumulator layout of a tile is an MFMA operand of it with K permuted
+// alike on both sides), so every access is free of bank conflicts, and the
+// barriers leave global stores in flight.
+// Bound by the serial chain: 2,900 cycles of tile_factor and 1,500 of hand
+// over per step.  128×128 FP64: 17.5 µs; 31 µs when wave 0 also kept the
+// diagonal tiles up to date, moved each through a row layout (6,300 cycles
+// per tile) and every barrier waited for the stores of the tile inverse.
 // TS: storage type of A (T, or FP32 for the mixed-precision driver, which
 // factors its FP32 diagonal tiles in FP64); Linv32: optional FP32 copy of
 // the tile inverses.
+constexpr int kFactorX = 2 * (kPanelNB / 16) * 256;   // LDS elements: Xb,
+constexpr int kFactorLi = 2 * 16 * kXLD;              // Lib (Db: one tile, 256)
 template <typename T, int W, typename TS = T>
 __device__ __forceinline__ void factor_body(int nb, TS *__restrict__ A, int64_t lda, int *info,
                                              int64_t info_base, T *__restrict__ LinvG, T *Xb,
@@ -240,97 +227,99 @@ __device__ __forceinline__ void factor_body(int nb, TS *__restrict__ A, int64_t 
 {
     typedef PanelMfma<T> M;
     typedef typename M::acc_t acc_t;
-    constexpr int NQ = W == 0 ? 8 : 10;
     constexpr int NBLK = kPanelNB / 16;
-    constexpr int XS = kPanelNB * kXLD, LS = 16 * kXLD;
+    constexpr int XS = NBLK * 256, LS = 16 * kXLD;
     const int lane = threadIdx.x & 63;
-    const int lc = lane & 15;
+    const int lc = lane & 15, lg = lane >> 4;
     const int nkb = (nb + 15) / 16;
 
-    // tiles transposed: lane holds row bi*16 + lc at columns bj*16 + row(lane, r)
-    acc_t acc[NQ];
-#pragma unroll
-    for (int q = 0; q < NQ; ++q) {
-        const int bi = dslot_bi<W>(q), bj = dslot_bj<W>(q);
-        if (bi < 0) continue;
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-            const int gi = bi * 16 + lc, gj = bj * 16 + M::row(lane, r);
-            T v = T(0);
-            if (gj <= gi) v = gi < nb ? T(A[gi + (int64_t)gj * lda]) : (gi == gj ? T(1) : T(0));
-            acc[q][r] = v;
-        }
-    }
-    if constexpr (W == 0) diag_factor<T>(acc[0], 0, nb, info, info_base, Db, Lib, LinvG, Linv32);
-    __syncthreads();
-#pragma unroll
-    for (int kb = 0; kb < NBLK; ++kb) {
-        if (kb >= nkb) break;
-        T *X = Xb + (kb & 1) * XS;
-        // (A) waves 1-3: the panel tiles X = A_(i,kb) L_kk⁻ᵀ (rdiv!), as
-        //     Xᵀ = L_kk⁻¹ A_(i,kb)ᵀ with the B operand from registers, then to
-        //     LDS (row-major); wave 0: the diagonal tiles beyond kb + 1 take
-        //     the previous step's update
-        if constexpr (W == 0) {
+    if constexpr (W == 0) {
+        acc_t d = load_tile<T, TS>(nb, A, lda, 0, 0);
+#pragma unroll 1
+        for (int kb = 0; kb < nkb; ++kb) {
             if (kb > 0) {
-                const T *Xp = Xb + ((kb - 1) & 1) * XS;
 #pragma unroll
-                for (int j = kb + 1; j < NBLK; ++j) {
-                    if (j >= nkb) break;
-                    diag_update<T>(acc[j], Xp, j);
+                for (int r = 0; r < 4; ++r) d[r] = Db[r * 64 + lane];
+            }
+            T w[4];
+            tile_factor<T>(d, w, nb - kb * 16, info, info_base + kb * 16);
+            T *Li = Lib + (kb & 1) * LS;
+#pragma unroll
+            for (int t = 0; t < 4; ++t) Li[lc * kXLD + lg + 4 * t] = w[t];
+            lds_barrier();                                            // end of (B)
+#pragma unroll
+            for (int t = 0; t < 4; ++t) {
+                if (LinvG) LinvG[kb * 256 + lc * 16 + lg + 4 * t] = w[t];
+                if (Linv32) Linv32[kb * 256 + lc * 16 + lg + 4 * t] = float(w[t]);
+            }
+            store_tile<T, TS>(nb, A, lda, kb, kb, d);
+            lds_barrier();                                            // end of (A)
+        }
+    } else {
+        constexpr int NQ = W == 3 ? 10 : 9, ND = W == 3 ? 3 : 2;
+        acc_t acc[NQ], dg[ND];
+#pragma unroll
+        for (int q = 0; q < NQ; ++q)
+            acc[q] = load_tile<T, TS>(nb, A, lda, oslot_bi(W, q), oslot_bj(W, q));
+#pragma unroll
+        for (int d = 0; d < ND; ++d) dg[d] = load_tile<T, TS>(nb, A, lda, row_of<W>(d), row_of<W>(d));
+        lds_barrier();
+#pragma unroll
+        for (int kb = 0; kb < NBLK; ++kb) {
+            if (kb >= nkb) break;
+            T *X = Xb + (kb & 1) * XS;
+            const T *Lik = Lib + (kb & 1) * LS;
+            // (A), ascending tile rows: row kb + 1 is the first of its owner
+#pragma unroll
+            for (int bi = kb + 1; bi < NBLK; ++bi) {
+#pragma unroll
+                for (int q = 0; q < NQ; ++q) {
+                    if (oslot_bi(W, q) != bi || oslot_bj(W, q) != kb) continue;
+                    if (bi >= nkb) continue;
+                    acc_t x = {T(0), T(0), T(0), T(0)};
+#pragma unroll
+                    for (int kq = 0; kq < 4; ++kq)
+                        x = M::mma(Lik[lc * kXLD + M::row(lane, kq)], acc[q][kq], x);
+                    acc[q] = x;
+                    if (bi == kb + 1) {
+#pragma unroll
+                        for (int d = 0; d < ND; ++d) {
+                            if (row_of<W>(d) != bi) continue;
+#pragma unroll
+                            for (int kq = 0; kq < 4; ++kq) dg[d] = M::mma(-x[kq], x[kq], dg[d]);
+#pragma unroll
+                            for (int r = 0; r < 4; ++r) Db[r * 64 + lane] = dg[d][r];
+                        }
+                    }
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) X[bi * 256 + r * 64 + lane] = x[r];
                 }
             }
-        } else {
-            const T *Lik = Lib + (kb & 1) * LS;
+            lds_barrier();                                            // end of (A)
+            if (kb + 1 >= nkb) break;
+            // (B)
 #pragma unroll
             for (int q = 0; q < NQ; ++q) {
-                const int bi = dslot_bi<W>(q), bj = dslot_bj<W>(q);
-                if (bi < 0 || bj != kb) continue;
-                if (bi >= nkb) continue;
-                acc_t x = {T(0), T(0), T(0), T(0)};
+                const int bi = oslot_bi(W, q), bj = oslot_bj(W, q);
+                if (bj <= kb || bi >= nkb) continue;
 #pragma unroll
                 for (int kq = 0; kq < 4; ++kq)
-                    x = M::mma(Lik[lc * kXLD + M::row(lane, kq)], acc[q][kq], x);
-                acc[q] = x;
-#pragma unroll
-                for (int r = 0; r < 4; ++r) X[(bi * 16 + lc) * kXLD + M::row(lane, r)] = x[r];
+                    acc[q] = M::mma(-X[bj * 256 + kq * 64 + lane], X[bi * 256 + kq * 64 + lane],
+                                    acc[q]);
             }
-        }
-        __syncthreads();
-        // (B) wave 0: the next diagonal tile takes this step's update and is
-        //     factored and inverted; waves 1-3: rank-16 trailing update of
-        //     their tiles, C_ijᵀ -= X_j X_iᵀ (rankUpdate!)
-        if constexpr (W == 0) {
-            if (kb + 1 < nkb) {
-                diag_update<T>(acc[kb + 1], X, kb + 1);
-                diag_factor<T>(acc[kb + 1], kb + 1, nb, info, info_base, Db,
-                               Lib + ((kb + 1) & 1) * LS, LinvG, Linv32);
-            }
-        } else {
 #pragma unroll
             for (int q = 0; q < NQ; ++q) {
-                const int bi = dslot_bi<W>(q), bj = dslot_bj<W>(q);
-                if (bi < 0 || bj <= kb) continue;
-                if (bi >= nkb) continue;
+                const int bi = oslot_bi(W, q);
+                if (oslot_bj(W, q) != kb || bi >= nkb) continue;
 #pragma unroll
-                for (int kq = 0; kq < 4; ++kq) {
-                    const int kk = (lane >> 4) + 4 * kq;
-                    const T a = -X[(bj * 16 + lc) * kXLD + kk];
-                    const T b = X[(bi * 16 + lc) * kXLD + kk];
-                    acc[q] = M::mma(a, b, acc[q]);
+                for (int d = 0; d < ND; ++d) {
+                    if (row_of<W>(d) != bi || bi == kb + 1) continue;
+#pragma unroll
+                    for (int kq = 0; kq < 4; ++kq) dg[d] = M::mma(-acc[q][kq], acc[q][kq], dg[d]);
                 }
+                store_tile<T, TS>(nb, A, lda, bi, kb, acc[q]);
             }
-        }
-        __syncthreads();
-    }
-#pragma unroll
-    for (int q = 0; q < NQ; ++q) {
-        const int bi = dslot_bi<W>(q), bj = dslot_bj<W>(q);
-        if (bi < 0) continue;
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-            const int gi = bi * 16 + lc, gj = bj * 16 + M::row(lane, r);
-            if (gi < nb && gj <= gi) A[gi + (int64_t)gj * lda] = TS(acc[q][r]);
+            lds_barrier();                                            // end of (B)
         }
     }
 }
@@ -345,9 +334,9 @@ __global__ __launch_bounds__(kPanelThreads) void chol_factor_kernel(int nb, T *_
                                                                     int64_t info_base,
                                                                     T *__restrict__ LinvG)
 {
-    __shared__ T Xb[2 * kPanelNB * kXLD];
-    __shared__ T Db[2 * 16 * kXLD];
-    __shared__ T Lib[2 * 16 * kXLD];
+    __shared__ T Xb[kFactorX];
+    __shared__ T Db[256];
+    __shared__ T Lib[kFactorLi];
     switch (threadIdx.x >> 6) {
     case 0: factor_body<T, 0>(nb, A, lda, info, info_base, LinvG, Xb, Db, Lib); break;
     case 1: factor_body<T, 1>(nb, A, lda, info, info_base, LinvG, Xb, Db, Lib); break;
@@ -610,9 +599,9 @@ __global__ __launch_bounds__(kPanelThreads) void chol_factor_near_identity_kerne
     int nb, T *__restrict__ A, int64_t lda, int *info, int64_t info_base, T *__restrict__ LinvG,
     const int *flags)
 {
-    __shared__ T Xb[2 * kPanelNB * kXLD];
-    __shared__ T Db[2 * 16 * kXLD];
-    __shared__ T Lib[2 * 16 * kXLD];
+    __shared__ T Xb[kFactorX];
+    __shared__ T Db[256];
+    __shared__ T Lib[kFactorLi];
     if (flags[0] != 0) return;
     if (flags[1] == 0) {
         const int nt = (nb + 15) / 16;
@@ -647,9 +636,9 @@ __global__ __launch_bounds__(kPanelThreads) void chol_factor_f32io_kernel(int nb
                                                                           int64_t info_base,
                                                                           float *__restrict__ Linv32)
 {
-    __shared__ double Xb[2 * kPanelNB * kXLD];
-    __shared__ double Db[2 * 16 * kXLD];
-    __shared__ double Lib[2 * 16 * kXLD];
+    __shared__ double Xb[kFactorX];
+    __shared__ double Db[256];
+    __shared__ double Lib[kFactorLi];
     switch (threadIdx.x >> 6) {
     case 0: factor_body<double, 0, float>(nb, A, lda, info, info_base, nullptr, Xb, Db, Lib, Linv32); break;
     case 1: factor_body<double, 1, float>(nb, A, lda, info, info_base, nullptr, Xb, Db, Lib, Linv32); break;
@@ -668,9 +657,9 @@ __global__ __launch_bounds__(kPanelThreads) void chol_factor_batched_kernel(int 
                                                                             T *LinvG,
                                                                             int64_t sLinv)
 {
-    __shared__ T Xb[2 * kPanelNB * kXLD];
-    __shared__ T Db[2 * 16 * kXLD];
-    __shared__ T Lib[2 * 16 * kXLD];
+    __shared__ T Xb[kFactorX];
+    __shared__ T Db[256];
+    __shared__ T Lib[kFactorLi];
     const int64_t b = blockIdx.x;
     T *Ab = A + b * sA;
     T *Lg = LinvG + b * sLinv;

@@ -262,6 +262,176 @@ struct PanelMfma<float> {
 };
 
 
+// ------------------------------------------------- symmetric tile factor --
+// The other half of a lane pair at distance 16 / 32: permlane swaps of v
+// with itself.  even(): rows (0, 0, 2, 2) / (01, 01) of v; odd(): rows
+// (1, 1, 3, 3) / (23, 23).
+template <typename T>
+__device__ __forceinline__ void swap16(T v, T &even, T &odd)
+{
+    if constexpr (sizeof(T) == 8) {
+        const uint2 u = __builtin_bit_cast(uint2, v);
+        const auto a = __builtin_amdgcn_permlane16_swap(u.x, u.x, false, false);
+        const auto b = __builtin_amdgcn_permlane16_swap(u.y, u.y, false, false);
+        even = __builtin_bit_cast(T, uint2{a[0], b[0]});
+        odd = __builtin_bit_cast(T, uint2{a[1], b[1]});
+    } else {
+        const unsigned u = __builtin_bit_cast(unsigned, v);
+        const auto a = __builtin_amdgcn_permlane16_swap(u, u, false, false);
+        even = __builtin_bit_cast(T, (unsigned)a[0]);
+        odd = __builtin_bit_cast(T, (unsigned)a[1]);
+    }
+}
+template <typename T>
+__device__ __forceinline__ void swap32(T v, T &lo, T &hi)
+{
+    if constexpr (sizeof(T) == 8) {
+        const uint2 u = __builtin_bit_cast(uint2, v);
+        const auto a = __builtin_amdgcn_permlane32_swap(u.x, u.x, false, false);
+        const auto b = __builtin_amdgcn_permlane32_swap(u.y, u.y, false, false);
+        lo = __builtin_bit_cast(T, uint2{a[0], b[0]});
+        hi = __builtin_bit_cast(T, uint2{a[1], b[1]});
+    } else {
+        const unsigned u = __builtin_bit_cast(unsigned, v);
+        const auto a = __builtin_amdgcn_permlane32_swap(u, u, false, false);
+        lo = __builtin_bit_cast(T, (unsigned)a[0]);
+        hi = __builtin_bit_cast(T, (unsigned)a[1]);
+    }
+}
+
+// 1/√d: the hardware estimate (relative error 2^-23 or better) and, for
+// FP64, one third-order step y(1 + e/2 + 3e²/8), e = 1 − d y² (the rest is
+// 5e³/16 < 2^-70); FP32 takes one Newton step.  d = 0 gives ∞, d < 0 and
+// NaN give NaN: the min keeps e finite where d·y is 0·∞.
+__device__ __forceinline__ double rsqrt_step(double d)
+{
+    const double y = __builtin_amdgcn_rsq(d);
+    const double e = __builtin_fmin(__builtin_fma(-(d * y), y, 1.0), 0.5);
+    return __builtin_fma(y * e, __builtin_fma(e, 0.375, 0.5), y);
+}
+__device__ __forceinline__ float rsqrt_step(float d)
+{
+    const float y = __builtin_amdgcn_rsqf(d);
+    const float e = __builtin_fminf(__builtin_fmaf(-(d * y), y, 1.0f), 0.5f);
+    return __builtin_fmaf(y * e, 0.5f, y);
+}
+
+// Columns 4S … 4S+3 of the symmetric tile S (accumulator layout, both
+// triangles present), column t to c[t] with lane (i, g) holding row i in
+// every 16-lane group: by symmetry the columns are rows of the accumulator,
+// which sit in one register of the four groups (FP64) or in the four
+// registers of one group (FP32).
+template <int S>
+__device__ __forceinline__ void tile_columns(const d4 &a, double c[4])
+{
+    double e, o;
+    swap16<double>(a[S], e, o);
+    swap32<double>(e, c[0], c[2]);
+    swap32<double>(o, c[1], c[3]);
+}
+template <int S>
+__device__ __forceinline__ void tile_columns(const f4 &a, float c[4])
+{
+#pragma unroll
+    for (int t = 0; t < 4; ++t) {
+        float e, o, lo, hi;
+        swap16<float>(a[t], e, o);
+        swap32<float>(S & 1 ? o : e, lo, hi);
+        c[t] = S & 2 ? hi : lo;
+    }
+}
+
+// Column C = 4S + t of the factor, in every group: pivot, reciprocal square
+// root, scaling, the later columns of the group of four, and step C of the
+// inverse's forward elimination V[i] −= (l_i/l_C) V[C] (w[q] holds column
+// g + 4q of V, zero above row g + 4q, so columns past C need no step).
+template <int C, typename T>
+__device__ __forceinline__ void tile_column_step(T c[4], T w[4], T &dsel, T &ysel, int i)
+{
+    constexpr int t = C & 3;
+    const T d = row_bcast<C>(c[t]);
+    const T y = rsqrt_step(d);
+    const T l = c[t] * y;
+    c[t] = l;
+    dsel = i == C ? d : dsel;
+    ysel = i == C ? y : ysel;
+    if constexpr (t < 3) c[t + 1] = fma_t(-l, row_bcast<(C + 1) & 15>(l), c[t + 1]);
+    if constexpr (t < 2) c[t + 2] = fma_t(-l, row_bcast<(C + 2) & 15>(l), c[t + 2]);
+    if constexpr (t < 1) c[t + 3] = fma_t(-l, row_bcast<(C + 3) & 15>(l), c[t + 3]);
+    if constexpr (C < 15) {
+        const T m = i > C ? l * y : T(0);
+#pragma unroll
+        for (int q = 0; q <= C / 4; ++q) w[q] = fma_t(-m, row_bcast<C>(w[q]), w[q]);
+    }
+}
+
+template <int S, typename T>
+__device__ __forceinline__ void tile_four_columns(typename PanelMfma<T>::acc_t &a,
+                                                  typename PanelMfma<T>::acc_t &lt, T w[4],
+                                                  T &dsel, T &ysel, int i, int g)
+{
+    T c[4];
+    tile_columns<S>(a, c);
+    tile_column_step<4 * S, T>(c, w, dsel, ysel, i);
+    tile_column_step<4 * S + 1, T>(c, w, dsel, ysel, i);
+    tile_column_step<4 * S + 2, T>(c, w, dsel, ysel, i);
+    tile_column_step<4 * S + 3, T>(c, w, dsel, ysel, i);
+    // element (i, 4S + g): the MFMA operand of the rank-4 update
+    const T e = g < 2 ? (g == 0 ? c[0] : c[1]) : (g == 2 ? c[2] : c[3]);
+    if constexpr (S < 3) a = PanelMfma<T>::mma(-e, e, a);
+    if constexpr (sizeof(T) == 8) {
+        lt[S] = e;
+    } else {
+#pragma unroll
+        for (int t = 0; t < 4; ++t) lt[t] = g == S ? c[t] : lt[t];
+    }
+}
+
+// Factors a symmetric 16×16 tile on one wave.  a: the tile in accumulator
+// layout with both triangles (overwritten); on return a holds L transposed
+// (lane: row l % 16 at columns row(l, r); entries right of the diagonal are
+// meaningless) and w the inverse (w[q] = L⁻¹[i][g + 4q], lane (i, g)).
+// Right-looking by four-column groups: within a group column by column as
+// cholUnblocked! does (src/cholesky.jl:3-15; the products are (a_ic r)(a_jc
+// r), each factor rounded once), then one rank-4 MFMA for the rest of the
+// tile.  The inverse's elimination steps fill the pivot chain's latency.
+// The first pivot among the first `nvalid` whose square root is taken of a
+// negative number is recorded in *info as gbase + index + 1.
+template <typename T>
+__device__ __forceinline__ void tile_factor(typename PanelMfma<T>::acc_t &a, T w[4], int nvalid,
+                                            int *info, int64_t gbase)
+{
+    typedef PanelMfma<T> M;
+    const int lane = threadIdx.x & 63;
+    const int i = lane & 15, g = lane >> 4;
+    T dsel = T(1), ysel = T(1);
+    typename M::acc_t lt = {T(0), T(0), T(0), T(0)};
+#pragma unroll
+    for (int q = 0; q < 4; ++q) w[q] = (i == g + 4 * q) ? T(1) : T(0);
+    tile_four_columns<0, T>(a, lt, w, dsel, ysel, i, g);
+    tile_four_columns<1, T>(a, lt, w, dsel, ysel, i, g);
+    tile_four_columns<2, T>(a, lt, w, dsel, ysel, i, g);
+    tile_four_columns<3, T>(a, lt, w, dsel, ysel, i, g);
+    const unsigned neg = (unsigned)__ballot(dsel < T(0) && i < nvalid) & 0xffffu;
+    if (neg != 0 && lane == 0 && info) atomicCAS(info, 0, (int)(gbase + __builtin_ctz(neg) + 1));
+    // the diagonal: √d = d·y corrected once
+    T s = dsel * ysel;
+    s = fma_t(fma_t(-s, s, dsel), T(0.5) * ysel, s);
+    s = dsel == T(0) ? T(0) : s;
+#pragma unroll
+    for (int r = 0; r < 4; ++r) a[r] = M::row(lane, r) == i ? s : lt[r];
+#pragma unroll
+    for (int q = 0; q < 4; ++q) w[q] *= ysel;
+}
+
+// Barrier over the workgroup that orders LDS only: outstanding global
+// stores stay in flight (__syncthreads waits for them, about a memory round
+// trip per barrier).
+__device__ __forceinline__ void lds_barrier()
+{
+    asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+}
+
 // ------------------------------------------------------------------ handle --
 // Workspace slots carved out of one device allocation that only grows.
 struct Handle {
