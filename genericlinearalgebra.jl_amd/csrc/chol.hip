@@ -1399,6 +1399,9 @@ int chol_device(Handle *h, hipStream_t s, int64_t n, T *A, int64_t lda, int algo
     // cholRecursive!: the reference recurses to 1×1 (cutoff does not reach
     // the A11 branch, :46); on the device the recursion stops at a leaf of
     // at least 2048 (or `cutoff` if larger) that the blocked driver factors.
+    if (h->chol_block < 0 && n > kPanelNB && n <= h->chol_df &&
+        ensure_df(h, chol_df_bytes(n, n, sizeof(T))))
+        return chol_df<T>(h, s, n, n, A, lda, 0, nullptr);
     const int64_t NB = h->chol_block < 0 ? auto_chol_block(n) : h->chol_block;
     if (NB > kPanelNB) return chol_la_dev<T>(h, s, n, A, lda, (int)NB, 0, Linv);
     int64_t leaf = std::max<int64_t>(param, 2048);
@@ -1439,6 +1442,10 @@ int chol_entry(gla_handle_t hh, char uplo, int64_t n, T *A, int64_t lda, int alg
         int hv = 0;
         GLA_HIP_TRY(hipMemcpyAsync(&hv, h->dinfo, sizeof(int), hipMemcpyDeviceToHost, s));
         GLA_HIP_TRY(hipStreamSynchronize(s));
+        if (hv < 0) {
+            set_error("Cholesky: a device-side wait gave up after %u polls", h->spin_limit);
+            return GLA_ERR_TIMEOUT;
+        }
         *info = hv;
     }
     return GLA_OK;

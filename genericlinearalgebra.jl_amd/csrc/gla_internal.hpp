@@ -444,11 +444,16 @@ struct Handle {
     unsigned *dbar = nullptr;         // device: grid-barrier counters
     void *ws = nullptr;               // device workspace
     size_t ws_bytes = 0;
+    void *df = nullptr;               // packed tiles of the dataflow Cholesky
+    size_t df_bytes = 0;
     int num_cus = 256;
     // Tuning: block width of the look-ahead driver behind cholRecursive!
     // (0: the recursive-halving driver; −1: chosen from n).  Set with
     // gla_set_tuning.
     int64_t chol_block = -1;
+    // Factor whole matrices up to this order, and the look-ahead driver's
+    // diagonal blocks, by the dataflow kernel (0: never).
+    int64_t chol_df = 4096;
     // Solve the look-ahead Cholesky's panels in one launch each (1) or by the
     // recursive rdiv! (0).
     int chol_psolve = 1;
@@ -489,6 +494,9 @@ struct Handle {
 // Ensure the workspace holds at least `bytes` (grows with hipMalloc, which
 // synchronises the device; the first call of a given size pays for it).
 int ensure_workspace(Handle *h, size_t bytes);
+// The same for the dataflow Cholesky's buffer; false if it cannot be had
+// (the caller then takes a path without it).
+bool ensure_df(Handle *h, size_t bytes);
 
 // ------------------------------------------------------------------ GEMM --
 // C = alpha*op(A)*op(B) + beta*C  with op(A) M×K, op(B) K×N.
@@ -519,6 +527,15 @@ int gemm_batched(hipStream_t s, char ta, char tb, int mode, int64_t M, int64_t N
 template <typename T>
 int chol_device(Handle *h, hipStream_t s, int64_t n, T *A, int64_t lda, int algo,
                 int64_t param, T *Linv = nullptr);
+
+// Dataflow Cholesky (chol_df.hip) of the m×n block column at A (m ≥ n;
+// n a multiple of 64 unless m = n), the first n rows its diagonal block: L in
+// place, and the 16×16 diagonal-tile inverses in LinvG if given.  Bytes of
+// h->df it needs: chol_df_bytes.
+size_t chol_df_bytes(int64_t m, int64_t n, size_t esz);
+template <typename T>
+int chol_df(Handle *h, hipStream_t s, int64_t m, int64_t n, T *A, int64_t lda, int64_t info_base,
+            T *LinvG);
 
 // Cholesky building blocks (chol.hip): factor one ≤128 diagonal block in
 // place and store the inverses of its 16×16 diagonal tiles; solve rows

@@ -815,6 +815,10 @@ int mixed_attempt(Handle *h, hipStream_t s, char prec, int64_t n, const double *
     int hinfo = 0;
     GLA_HIP_TRY(hipMemcpyAsync(&hinfo, h->dinfo, sizeof(int), hipMemcpyDeviceToHost, s));
     GLA_HIP_TRY(hipStreamSynchronize(s));
+    if (hinfo < 0) {
+        set_error("Cholesky: a device-side wait gave up after %u polls", h->spin_limit);
+        return GLA_ERR_TIMEOUT;
+    }
     *info = hinfo;
     if (hinfo != 0) {
         *iters = 0;

@@ -37,6 +37,29 @@ int ensure_workspace(Handle *h, size_t bytes)
     return GLA_OK;
 }
 
+bool ensure_df(Handle *h, size_t bytes)
+{
+    if (bytes <= h->df_bytes) return true;
+    const size_t gran = size_t(16) << 20;
+    const size_t want = (bytes + gran - 1) / gran * gran;
+    if (h->df) {
+        // the old buffer may still be read by queued work
+        if (hipDeviceSynchronize() != hipSuccess || hipFree(h->df) != hipSuccess) {
+            (void)hipGetLastError();
+            return false;
+        }
+        h->df = nullptr;
+        h->df_bytes = 0;
+    }
+    if (hipMalloc(&h->df, want) != hipSuccess) {
+        (void)hipGetLastError();
+        h->df = nullptr;
+        return false;
+    }
+    h->df_bytes = want;
+    return true;
+}
+
 namespace {
 // (Re)creates the look-ahead Cholesky's stream pair: `masked`, limited to
 // every CU but the highest-numbered `reserve`, and `chain`, a non-blocking
@@ -80,6 +103,14 @@ int gla_set_tuning(gla_handle_t hh, const char *key, int64_t value)
             return -3;
         }
         h->chol_block = value;
+        return GLA_OK;
+    }
+    if (std::strcmp(key, "chol_df") == 0) {
+        if (value < 0 || value > 8192) {
+            gla::set_error("chol_df must be in [0, 8192]");
+            return -3;
+        }
+        h->chol_df = value;
         return GLA_OK;
     }
     if (std::strcmp(key, "ldlt_block") == 0) {
@@ -202,7 +233,7 @@ int gla_get_tuning(gla_handle_t hh, const char *key, int64_t *value)
         {"gemm_lds1", gla::get_gemm_lds1()}, {"qr_hr", h->qr_hr},
         {"chol_syrk_late", h->chol_syrk_late}, {"qr_lookahead", h->qr_lookahead},
         {"chol_psolve", h->chol_psolve},
-        {"spin_limit", (int64_t)h->spin_limit}, {"side_cu_reserve", h->side_cu_reserve},
+        {"spin_limit", (int64_t)h->spin_limit}, {"chol_df", h->chol_df}, {"side_cu_reserve", h->side_cu_reserve},
         {"qr_wait_test", h->qr_wait_test},
     };
     for (const auto &k : knobs)
@@ -248,6 +279,7 @@ int gla_handle_destroy(gla_handle_t hh)
     GLA_HIP_TRY(hipSetDevice(h->device));
     GLA_HIP_TRY(hipDeviceSynchronize());
     if (h->ws) (void)hipFree(h->ws);
+    if (h->df) (void)hipFree(h->df);
     if (h->dinfo) (void)hipFree(h->dinfo);
     if (h->dbar) (void)hipFree(h->dbar);
     (void)hipEventDestroy(h->ev_fork);
