@@ -23,9 +23,12 @@
 //              of the next block column runs on the caller's stream right
 //              after the panel, the rest of the trailing update runs on the
 //              handle's side stream and overlaps the next panel.
-//   look-ahead the same loop with wide blocks (NB = 512 by default): the
-//              diagonal block by the blocked driver, the panel by the
-//              recursive rdiv!, the trailing SYRK with K = NB.
+//   look-ahead the same loop with wide blocks: the block column by one
+//              dataflow launch (chol_df.hip), or the diagonal block by the
+//              blocked driver and the panel by one launch or the recursive
+//              rdiv!; the trailing SYRK with K = NB.
+//   dataflow   cholRecursive! up to h->chol_df: the whole matrix in one
+//              dataflow launch.
 //   recursive  halves n as cholRecursive! does; below a threshold the blocked
 //              driver factors the leaf.  rdiv! with a large L11 is itself
 //              recursive (two half solves and a GEMM); its leaves are
@@ -1139,16 +1142,19 @@ int trsm_rlt_dev(hipStream_t s, int64_t m, int64_t n, const T *L, int64_t ldl, c
 // diagonal factor and panel solve.
 template <typename T>
 int chol_la_dev(Handle *h, hipStream_t s0, int64_t n, T *A, int64_t lda, int NB,
-                int64_t info_base, T *Linv)
+                int64_t info_base, T *Linv, bool df = false)
 {
     if (n <= 0) return GLA_OK;
     if (NB <= kPanelNB || n <= NB) return chol_blocked_dev<T>(h, s0, n, A, lda, kPanelNB, info_base, Linv);
     const int64_t nsteps = cdiv(n, NB);
     const bool overlap = nsteps > 2;
-    // With CUs reserved from the SYRK, the chain runs on an internal stream
+    // df: each block column in one dataflow launch, which fills the chip, so
+    // the SYRK beside it runs on every CU (n = 16384 FP64, 2048-wide: 28.3
+    // ms; with 32 CUs kept from the SYRK 29.3 ms).
+    // Else, with CUs reserved from the SYRK, the chain runs on an internal stream
     // with every CU and the SYRK on the masked one, both forked from (and
     // joined back to) the caller's stream.
-    const bool masked = overlap && h->masked != nullptr;
+    const bool masked = overlap && !df && h->masked != nullptr;
     hipStream_t s = masked ? h->chain : s0;
     hipStream_t side = masked ? h->masked : h->side;
     if (overlap) {
@@ -1162,15 +1168,19 @@ int chol_la_dev(Handle *h, hipStream_t s0, int64_t n, T *A, int64_t lda, int NB,
         const int64_t below = n - k - kb;
         T *Akk = A + k + k * lda;
         T *A21 = Akk + kb;
-        // :27-28 rdiv! of the panel: one launch over all of it when the block
+        // :27-28 the diagonal block and rdiv! of the panel: one dataflow launch,
+        // or the 128-wide driver and one launch over the panel when the block
         // is a whole number of 128-wide tiles, else the recursive solve
         const bool fused = h->chol_psolve != 0 && kb % kPanelNB == 0 && kb <= kPsolveMaxNB;
-        GLA_TRY(chol_blocked_dev<T>(h, s, kb, Akk, lda, kPanelNB, info_base + k, Linv, false,
-                                    fused));
+        if (df)
+            GLA_TRY(chol_df<T>(h, s, n - k, kb, Akk, lda, info_base + k, nullptr));
+        else
+            GLA_TRY(chol_blocked_dev<T>(h, s, kb, Akk, lda, kPanelNB, info_base + k, Linv, false,
+                                        fused));
         if (below == 0) break;
-        if (fused) {
+        if (!df && fused) {
             GLA_TRY(launch_psolve<T>(s, (int)kb, Akk, lda, Linv, A21, lda, below));
-        } else {
+        } else if (!df) {
             GLA_TRY(launch_tile_inverse<T>(s, kb, Akk, lda, Linv));
             GLA_TRY(trsm_rlt_dev<T>(s, below, kb, Akk, lda, Linv, A21, lda));
         }
@@ -1364,19 +1374,27 @@ GLA_INST_BLOCKS(double)
 GLA_INST_BLOCKS(float)
 #undef GLA_INST_BLOCKS
 
-// algo: 0 unblocked, 1 blocked (param = blocksize), 2 recursive (param = cutoff)
-// Step width of the look-ahead driver for chol_block −1 (the default), from
-// n = 2048…16384 sweeps on MI355X: below 3072 the recursive driver (0), then
-// 256-wide steps while the chain of diagonal factor and panel solve sets the
-// pace, wider steps as the trailing SYRK grows to dominate.
-inline int64_t auto_chol_block(int64_t n)
+// Driver of cholRecursive! for chol_block −1 (the default), from sweeps on
+// MI355X (ms, copy of A included; FP64 | FP32):
+//                                       n = 1000   5001       8192       12288      16384
+//   whole matrix in one dataflow launch  0.21|0.18  1.50|1.01  4.65|2.59
+//   look-ahead, 3072-wide dataflow                             4.81|2.87  12.9|7.33  28.4|15.9
+//   look-ahead, 2048-wide dataflow                             4.89|2.99  13.3|7.55  27.6|15.5
+//   a launch per 128-wide step           0.53|0.49  3.37|3.05  7.38|5.65  16.9|11.7  33.2|21.9
+// so: one launch up to h->chol_df (8192: its packed tiles take 266 MB in
+// FP64), then 3072-wide steps, then 2048.  Without the dataflow buffer
+// (chol_df 0, or no memory for it) the step width is 0 (recursive halving)
+// below 3072, then 256, 512 and 1024.
+inline int64_t auto_chol_block(int64_t n, bool df)
 {
+    if (df) return n < 14336 ? 3072 : 2048;
     if (n < 3072) return 0;
     if (n < 10240) return 256;
     if (n < 14336) return 512;
     return 1024;
 }
 
+// algo: 0 unblocked, 1 blocked (param = blocksize), 2 recursive (param = cutoff)
 template <typename T>
 int chol_device(Handle *h, hipStream_t s, int64_t n, T *A, int64_t lda, int algo, int64_t param,
                 T *Linv)
@@ -1399,11 +1417,14 @@ int chol_device(Handle *h, hipStream_t s, int64_t n, T *A, int64_t lda, int algo
     // cholRecursive!: the reference recurses to 1×1 (cutoff does not reach
     // the A11 branch, :46); on the device the recursion stops at a leaf of
     // at least 2048 (or `cutoff` if larger) that the blocked driver factors.
-    if (h->chol_block < 0 && n > kPanelNB && n <= h->chol_df &&
-        ensure_df(h, chol_df_bytes(n, n, sizeof(T))))
-        return chol_df<T>(h, s, n, n, A, lda, 0, nullptr);
-    const int64_t NB = h->chol_block < 0 ? auto_chol_block(n) : h->chol_block;
-    if (NB > kPanelNB) return chol_la_dev<T>(h, s, n, A, lda, (int)NB, 0, Linv);
+    bool df = false;
+    if (h->chol_block < 0 && h->chol_df > 0 && n > kPanelNB) {
+        const int64_t w = n <= h->chol_df ? n : auto_chol_block(n, true);
+        df = ensure_df(h, chol_df_bytes(n, w, sizeof(T)));
+        if (df && w == n) return chol_df<T>(h, s, n, n, A, lda, 0, nullptr);
+    }
+    const int64_t NB = h->chol_block < 0 ? auto_chol_block(n, df) : h->chol_block;
+    if (NB > kPanelNB) return chol_la_dev<T>(h, s, n, A, lda, (int)NB, 0, Linv, df);
     int64_t leaf = std::max<int64_t>(param, 2048);
     return chol_recursive_dev<T>(h, s, n, A, lda, leaf, 0, Linv);
 }

@@ -22,8 +22,16 @@
 //
 // Bound: for small n the chain along the diagonal, per 64 columns the tile
 // factor of four 16×16 tiles (≈7 µs), one flag and tile exchange between
-// workgroups (≈2 µs) and the 64-wide solve and update (≈2 µs); a launch per
-// factor, solve and update took about twice as long.
+// workgroups (≈2 µs) and the 64-wide solve and update (≈2 µs): FP64 n = 1000
+// takes 0.21 ms (0.53 ms with a launch per factor, solve and update of 128
+// columns).  For large n the products, at about half the MFMA rate (n = 8192
+// FP64: 4.65 ms, 39 TFLOP/s): three workgroups per CU cover each other's
+// waits, which is why a slab is 16 columns (53 KB of LDS); with 32-column
+// slabs and two workgroups per CU n = 8192 took 5.07 ms.  Coherent or plain
+// operand loads took the same time, so the coherent ones stay.
+// Accuracy: sums are formed from zero over 256 columns at a time, as the
+// launch-per-step driver's; FP64 n = 1000 is 1.5e-16 from an 80-bit
+// evaluation (2.1e-16 that driver).
 #include <algorithm>
 
 #include "gla_coherent.hpp"
@@ -242,7 +250,7 @@ __device__ __forceinline__ void factor_diag(const DfP<T> &p, int j, int w,
 #pragma unroll
         for (int kb = 0; kb < 4; ++kb) {
             if (kb >= nkb) break;
-            T *X = Xs + (kb & 1) * 1024;
+            T *X = Xs + (kb & 1) * 768;           // tile rows 1–3
             acc_t x = {T(0), T(0), T(0), T(0)};
             if (w > kb && w < nkb) {
                 const T *Li = Lib + (kb & 1) * LS;
@@ -254,7 +262,7 @@ __device__ __forceinline__ void factor_diag(const DfP<T> &p, int j, int w,
                     for (int kq = 0; kq < 4; ++kq) dg = M::mma(-x[kq], x[kq], dg);
                     put16(Db, dg);
                 }
-                put16(X + w * 256, x);
+                put16(X + (w - 1) * 256, x);
             }
             lds_barrier();                                            // end of (A)
             if (kb + 1 >= nkb) break;
@@ -263,7 +271,7 @@ __device__ __forceinline__ void factor_diag(const DfP<T> &p, int j, int w,
 #pragma unroll
                     for (int b = kb + 1; b < 3; ++b)
                         if (b < w) {
-                            const acc_t xb = get16(X + b * 256);
+                            const acc_t xb = get16(X + (b - 1) * 256);
 #pragma unroll
                             for (int kq = 0; kq < 4; ++kq) c[b] = M::mma(-xb[kq], x[kq], c[b]);
                         }
@@ -283,12 +291,15 @@ __device__ __forceinline__ void factor_diag(const DfP<T> &p, int j, int w,
 }
 
 template <typename T>
-__global__ __launch_bounds__(kDThreads, 2) void chol_df_kernel(DfP<T> p)
+__global__ __launch_bounds__(kDThreads, sizeof(T) == 8 ? 3 : 4) void chol_df_kernel(DfP<T> p)
 {
     typedef PanelMfma<T> M;
     typedef typename M::acc_t acc_t;
-    constexpr int H = kTE / 2;                        // half a tile: 32 columns
-    __shared__ __align__(16) T buf[4 * H];            // two slabs of two operands
+    constexpr int H = kTE / 4;                        // a quarter tile: 16 columns
+    // a ring of three slabs of two operands; then the packed L and the solved
+    // tile.  53 KB in FP64: three workgroups per CU
+    __shared__ __align__(16) T buf[kLE + kTE];
+    static_assert(3 * 2 * H <= kLE + kTE, "slab ring");
     const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
 
     // this workgroup's tile: column j, then the diagonal tile or row i
@@ -325,69 +336,88 @@ __global__ __launch_bounds__(kDThreads, 2) void chol_df_kernel(DfP<T> p)
         for (int r = 0; r < 4; ++r) dg[r] = elem(16 * w + lc, 16 * w + M::row(lane, r));
     }
 
-    // the products, in slabs of 32 columns: slab s of X(i, ·) and X(jo, ·) at
-    // buf + (s % 2)·2H and + H, loaded while slab s − 1 is multiplied
-    const int ns = 2 * nk;
-    int av = 0;                                       // 64-column products available
-    auto issue = [&](int s) {
-        T *d = buf + (s & 1) * 2 * H;
-        stage<T>(x_tile<T>(p, i, s >> 1) + (s & 1) * H, d, H);
-        stage<T>(x_tile<T>(p, jo, s >> 1) + (s & 1) * H, d + H, H);
+    // the products, in slabs of 16 columns: slab s of X(i, ·) and X(jo, ·) in
+    // place s % 3 of a ring, two slabs in flight while one is multiplied
+    const int ns = 4 * nk;
+    // products are summed from zero and taken off the tile every kFold slabs:
+    // a sum that runs through the tile rounds every product at the tile's own
+    // magnitude (FP32 n = 5001: 4x the error)
+    constexpr int kFold = 16;
+    const acc_t zero = {T(0), T(0), T(0), T(0)};
+    acc_t sa[4], sc[3], sd = zero;
+#pragma unroll
+    for (int b = 0; b < 4; ++b) sa[b] = zero;
+#pragma unroll
+    for (int b = 0; b < 3; ++b) sc[b] = zero;
+    int av = 0, next = 0;                             // products available, next slab to load
+    auto issue = [&]() {
+        T *d = buf + (next % 3) * 2 * H;
+        stage<T>(x_tile<T>(p, i, next >> 2) + (next & 3) * H, d, H);
+        stage<T>(x_tile<T>(p, jo, next >> 2) + (next & 3) * H, d + H, H);
+        ++next;
     };
-    auto available = [&](int need) {
-        const int a = wait_ge(p.prog + i, need, p.spin_limit, p.info);
-        const int b = wait_ge(p.prog + jo, need, p.spin_limit, p.info);
-        av = a < b ? a : b;
-    };
-    if (ns > 0) {
-        available(1);
-        issue(0);
-    }
     for (int s = 0; s < ns; ++s) {
-        stores_done();      // vmcnt(0): this wave's loads of slab s have landed
+        if (next <= s) {
+            const int a = wait_ge(p.prog + i, (s >> 2) + 1, p.spin_limit, p.info);
+            const int b = wait_ge(p.prog + jo, (s >> 2) + 1, p.spin_limit, p.info);
+            av = a < b ? a : b;
+            issue();
+        }
+        // this wave's loads of slab s have landed, those of later ones may not
+        constexpr int PER = 2 * H * sizeof(T) / 4096;
+        const int later = next - s - 1;
+        if (later == 0) __builtin_amdgcn_s_waitcnt(0x0F70);
+        else if (later == 1) __builtin_amdgcn_s_waitcnt(0x0F70 | PER);
+        else __builtin_amdgcn_s_waitcnt(0x0F70 | (2 * PER));
         lds_barrier();      // everyone's have, and slab s − 1 has been read
-        const int need = ((s + 1) >> 1) + 1;
-        bool ahead = false;
-        if (s + 1 < ns) {
-            if (av < need) {
+        while (next < ns && next <= s + 2) {
+            if (av < (next >> 2) + 1) {
                 const int a = load_coherent(p.prog + i), b = load_coherent(p.prog + jo);
                 av = __builtin_amdgcn_readfirstlane(a < b ? a : b);
+                if (av < (next >> 2) + 1) break;
             }
-            ahead = av >= need;
-            if (ahead) issue(s + 1);
+            issue();
         }
-        const T *bi = buf + (s & 1) * 2 * H, *bj = bi + H;
+        const T *bi = buf + (s % 3) * 2 * H, *bj = bi + H;
+        const acc_t xi = get16(bi + w * 256);
 #pragma unroll
-        for (int bk = 0; bk < 2; ++bk) {
-            const acc_t xi = get16(bi + (bk * 4 + w) * 256);
+        for (int b = 0; b < 4; ++b) {
+            const acc_t xj = get16(bj + b * 256);
+#pragma unroll
+            for (int kq = 0; kq < 4; ++kq) sa[b] = M::mma(xj[kq], xi[kq], sa[b]);
+        }
+        if (diag) {
+#pragma unroll
+            for (int b = 0; b < 3; ++b)
+                if (b < w) {
+                    const acc_t xb = get16(bi + b * 256);
+#pragma unroll
+                    for (int kq = 0; kq < 4; ++kq) sc[b] = M::mma(xb[kq], xi[kq], sc[b]);
+                }
+#pragma unroll
+            for (int kq = 0; kq < 4; ++kq) sd = M::mma(xi[kq], xi[kq], sd);
+        }
+        if ((s & (kFold - 1)) == kFold - 1 || s + 1 == ns) {
 #pragma unroll
             for (int b = 0; b < 4; ++b) {
-                const acc_t xj = get16(bj + (bk * 4 + b) * 256);
-#pragma unroll
-                for (int kq = 0; kq < 4; ++kq) acc[b] = M::mma(-xj[kq], xi[kq], acc[b]);
+                acc[b] -= sa[b];
+                sa[b] = zero;
             }
             if (diag) {
 #pragma unroll
-                for (int b = 0; b < 3; ++b)
-                    if (b < w) {
-                        const acc_t xb = get16(bi + (bk * 4 + b) * 256);
-#pragma unroll
-                        for (int kq = 0; kq < 4; ++kq) c[b] = M::mma(-xb[kq], xi[kq], c[b]);
-                    }
-#pragma unroll
-                for (int kq = 0; kq < 4; ++kq) dg = M::mma(-xi[kq], xi[kq], dg);
+                for (int b = 0; b < 3; ++b) {
+                    c[b] -= sc[b];
+                    sc[b] = zero;
+                }
+                dg -= sd;
+                sd = zero;
             }
-        }
-        if (s + 1 < ns && !ahead) {
-            available(need);
-            issue(s + 1);
         }
     }
 
     // X = acc L(jo, jo)⁻ᵀ
     T *Ls = buf;                                      // 2560 elements
     T *Xr = buf + kLE;                                // 4096: the solved tile
-    static_assert(kLE + kTE + 256 + 2 * 16 * kXLD <= 4 * H, "LDS regions");
     if (jo >= 0) {
         wait_ge(p.ldone + jo, 1, p.spin_limit, p.info);
         lds_barrier();                                // the last slab has been read
@@ -414,10 +444,10 @@ __global__ __launch_bounds__(kDThreads, 2) void chol_df_kernel(DfP<T> p)
             for (int b = 0; b < 4; ++b) put16(Xr + (b * 4 + w) * 256, acc[b]);
             lds_barrier();
 #pragma unroll
-            for (int bk = 0; bk < 4; ++bk) {
+            for (int bk = 0; bk < 4; ++bk)
 #pragma unroll
-                for (int kq = 0; kq < 4; ++kq) dg = M::mma(-acc[bk][kq], acc[bk][kq], dg);
-            }
+                for (int kq = 0; kq < 4; ++kq) sd = M::mma(acc[bk][kq], acc[bk][kq], sd);
+            dg -= sd;
 #pragma unroll
             for (int b = 0; b < 3; ++b)
                 if (b < w) {
@@ -425,12 +455,14 @@ __global__ __launch_bounds__(kDThreads, 2) void chol_df_kernel(DfP<T> p)
                     for (int bk = 0; bk < 4; ++bk) {
                         const acc_t xb = get16(Xr + (bk * 4 + b) * 256);
 #pragma unroll
-                        for (int kq = 0; kq < 4; ++kq) c[b] = M::mma(-xb[kq], acc[bk][kq], c[b]);
+                        for (int kq = 0; kq < 4; ++kq) sc[b] = M::mma(xb[kq], acc[bk][kq], sc[b]);
                     }
+                    c[b] -= sc[b];
                 }
         }
         // Ls is free: every wave is past its solve (the barrier above; j = 0 has none)
-        factor_diag<T>(p, j, w, c, dg, Xr + kTE, Xr + kTE + 256, buf);
+        static_assert(256 + 2 * 16 * kXLD + 2 * 768 <= kLE, "LDS regions");
+        factor_diag<T>(p, j, w, c, dg, buf, buf + 256, buf + 256 + 2 * 16 * kXLD);
     }
     if (jo >= 0) store_strip<T>(p, i, jo, w, acc);
 }

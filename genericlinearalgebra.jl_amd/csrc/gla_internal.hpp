@@ -451,9 +451,9 @@ struct Handle {
     // (0: the recursive-halving driver; −1: chosen from n).  Set with
     // gla_set_tuning.
     int64_t chol_block = -1;
-    // Factor whole matrices up to this order, and the look-ahead driver's
-    // diagonal blocks, by the dataflow kernel (0: never).
-    int64_t chol_df = 4096;
+    // cholRecursive! factors matrices up to this order in one dataflow launch
+    // and the look-ahead driver's block columns likewise (0: neither).
+    int64_t chol_df = 8192;
     // Solve the look-ahead Cholesky's panels in one launch each (1) or by the
     // recursive rdiv! (0).
     int chol_psolve = 1;

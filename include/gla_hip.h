@@ -66,9 +66,14 @@ const char *gla_version(void);
 /* Tuning knobs of a handle (no reference counterpart).  "chol_block": a
  * multiple of 128 runs cholRecursive! as a right-looking blocked
  * factorisation with blocks of that width and depth-1 look-ahead; 0 runs it
- * as recursive halving down to 2048-wide leaves; −1 (default) picks from n
- * (0 below 3072, then 256, 512 from 10240, 1024 from 14336).  All compute
- * the same factor up to rounding.  "chol_psolve": 1 (default) solves each
+ * as recursive halving down to 2048-wide leaves; −1 (default) takes the
+ * dataflow driver ("chol_df"), or without its buffer picks from n (0 below
+ * 3072, then 256, 512 from 10240, 1024 from 14336).  All compute the same
+ * factor up to rounding.  "chol_df": largest order (default 8192, at most
+ * 8192) that cholRecursive! factors in one dataflow launch; larger ones take
+ * 3072- or 2048-wide block columns of one such launch each; 0 turns both
+ * off.  The handle keeps the launch's tile buffer (266 MB at n = 8192 in
+ * FP64), which only grows; if it cannot be allocated the other drivers run.  "chol_psolve": 1 (default) solves each
  * look-ahead panel up to 768 wide in one launch (every 64 rows sweep the
  * 128-wide column blocks), 0 by the recursive rdiv!.  "chol_syrk_late": 1 (default) starts the look-ahead
  * driver's trailing SYRK on the side stream after the next block column's
@@ -102,7 +107,7 @@ const char *gla_version(void);
  * 8/8/16-wide K slabs, 0 to the register-staged kernel; "gemm_lds1" (process-wide): 1 (default) stages
  * FP64 128×128 tiles through one LDS buffer, 0 through two.  Same results
  * bit for bit in every setting.  "spin_limit": polls (default 2^25, about a
- * second) before a grid-wide wait of the QR panel gives up and the call
+ * second) before a wait of the dataflow Cholesky or a grid-wide wait of the QR panel gives up and the call
  * returns GLA_ERR_TIMEOUT.  "qr_wait_test": 1 makes every such wait target
  * an arrival count that never comes (a test of the timeout report; the
  * kernels still finish, after spin_limit polls per wait). */
