@@ -612,6 +612,11 @@ size_t symv_scratch(int64_t n);
 
 // QR building blocks (qr.hip): T of the first k reflectors of F (m×k), and
 // A (mA×nA) <- op(Q) A, trans 'N' or 'T', Q from the first b reflectors.
+// V (m×n, ld ldv) = the reflectors stored in F with their unit diagonal and
+// zeros above.
+template <typename T>
+int unit_lower_explicit(hipStream_t s, int64_t m, int64_t n, const T *F, int64_t ldf, T *V,
+                        int64_t ldv);
 size_t qr_tblock_scratch(int64_t m, int64_t k);
 size_t qr_apply_scratch(int64_t mA, int64_t nA, int64_t b);
 template <typename T>

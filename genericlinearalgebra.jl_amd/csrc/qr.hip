@@ -1798,7 +1798,16 @@ int qr_apply_dev(hipStream_t s, char trans, int64_t mA, int64_t nA, int64_t b, c
                         8 * (size_t)b * nA);
 }
 
+template <typename T>
+int unit_lower_explicit(hipStream_t s, int64_t m, int64_t n, const T *F, int64_t ldf, T *V,
+                        int64_t ldv)
+{
+    return unit_lower_copy<T>(s, m, n, F, ldf, V, ldv);
+}
+
 #define GLA_INST_QR(T)                                                                           \
+    template int unit_lower_explicit<T>(hipStream_t, int64_t, int64_t, const T *, int64_t, T *,  \
+                                        int64_t);                                                \
     template int qr_tblock_dev<T>(hipStream_t, int64_t, int64_t, const T *, int64_t, const T *, \
                                   T *, int64_t, T *);                                            \
     template int qr_apply_dev<T>(hipStream_t, char, int64_t, int64_t, int64_t, const T *,        \
@@ -1831,7 +1840,12 @@ int qr_entry(gla_handle_t hh, int64_t m, int64_t n, T *A, int64_t lda, int64_t b
     if (lda < std::max<int64_t>(1, m)) { set_error("lda < max(1,m)"); return -5; }
     if (!unblocked && bs < 1) { set_error("blocksize < 1"); return -6; }
     if (!tau && std::min(m, n) > 0) { set_error("tau is null"); return -7; }
-    const int nb = (int)std::min<int64_t>(unblocked ? kQrNB : bs, kQrNB);
+    // The factors do not depend on the block size; only `work` shows it.  So
+    // without `work` every matrix wider than its block size runs in 128-wide
+    // block columns: a panel costs about as much at any width, and the
+    // trailing products have K = block width (1501×700 FP64: block size 12
+    // took 59 panels and 9.8 ms with the least-squares solve, 128 takes six and 2.5 ms).
+    const int nb = (int)std::min<int64_t>(unblocked || !work ? kQrNB : bs, kQrNB);
     if (work && ldwork < std::max<int64_t>(1, std::min<int64_t>(m, nb))) {
         set_error("ldwork < min(m, blocksize)");
         return -9;

@@ -135,6 +135,24 @@ __global__ void div_rows_k(int64_t n, int64_t nrhs, const T *F, int64_t ldf, T *
     if (k < nrhs) Y[k + i * nrhs] = Y[k + i * nrhs] / F[i + i * ldf];
 }
 
+// G <- I + stril(G) D, D = diag(d); the upper triangle is left alone.
+template <typename T>
+__global__ void unit_scale_k(int64_t n, T *G, const T *d)
+{
+    GLA_ROW(i);
+    GLA_COLS(j, n)
+    if (i < n && i >= j) G[i + j * n] = i == j ? T(1) : G[i + j * n] * d[j];
+}
+
+// W (n×nrhs) = D Zᵀ for Z nrhs×n.
+template <typename T>
+__global__ void scaled_cols_k(int64_t n, int64_t nrhs, const T *Z, const T *d, T *W)
+{
+    GLA_ROW(i);
+    GLA_COLS(k, nrhs)
+    if (i < n) W[i + k * n] = d[i] * Z[k + i * nrhs];
+}
+
 #undef GLA_COLS
 #undef GLA_ROW
 
@@ -240,34 +258,49 @@ int ldlt_lmul_dev(hipStream_t s, char uplo, int64_t n, int64_t nrhs, const T *F,
     return gemm<T>(s, 'N', 'N', 0, n, nrhs, n, T(1), Lx, n, Y, n, T(0), B, ldb, 0);
 }
 
-// Scratch elements of the QR solve.
+// Scratch elements of the QR solve: explicit V, G = VᵀV (then J Rᵀ J), tile
+// inverses, three nrhs×n blocks, split-K partials.
 size_t qr_solve_scratch(int64_t m, int64_t n, int64_t nrhs)
 {
-    return (size_t)n * n + std::max(qr_tblock_scratch(m, n), qr_apply_scratch(m, nrhs, n)) +
-           (size_t)n * n + tile_inverse_elems(n) + (size_t)nrhs * n + 256;
+    return (size_t)m * n + (size_t)n * n + tile_inverse_elems(n) + 3 * (size_t)nrhs * n +
+           8 * (size_t)nrhs * n + 256;
 }
 
 // Least squares for m ≥ n: B (m×nrhs) <- Qᵀ B, then B[0:n] <- R⁻¹ B[0:n],
 // with (F, τ) as stored by qrBlocked!/qrUnblocked!.  info: 1 + the first
 // zero diagonal entry of R (device int), n + 1 when R is nonsingular.
+// Qᵀ B = B − V Tᵀ Vᵀ B with T = (I + D striu(VᵀV))⁻¹ D, D = diag(τ)
+// (src/qr.jl:64-83, src/householder.jl:119-157), so TᵀW = D L⁻¹ W for the
+// unit lower L = I + stril(VᵀV) D: a solve with nrhs rows instead of T's
+// explicit inverse (1501×700: 1.0 ms of 128-wide inverses).
 template <typename T>
 int qr_solve_dev(hipStream_t s, int64_t m, int64_t n, int64_t nrhs, const T *F, int64_t ldf,
                  const T *tau, T *B, int64_t ldb, int *info, T *scratch)
 {
     if (n <= 0 || nrhs <= 0) return GLA_OK;
-    const size_t nn = (size_t)n * n;
-    T *Tm = scratch;
-    T *rest = Tm + nn;
-    T *Kr = rest + std::max(qr_tblock_scratch(m, n), qr_apply_scratch(m, nrhs, n));
-    T *Kri = Kr + nn, *Z = Kri + tile_inverse_elems(n);
+    const size_t nr = (size_t)nrhs * n;
+    T *Vw = scratch, *G = Vw + (size_t)m * n, *Gi = G + (size_t)n * n,
+      *W = Gi + tile_inverse_elems(n), *Z = W + nr, *W2 = Z + nr, *split = W2 + nr;
     hipLaunchKernelGGL(set_int_k, dim3(1), dim3(1), 0, s, info, (int)(n + 1));
     GLA_LAUNCH_CHECK();
     hipLaunchKernelGGL((first_zero_diag_k<T>), dim3((unsigned)cdiv(n, 256)), dim3(256), 0, s, n, F,
                        ldf, info);
     GLA_LAUNCH_CHECK();
-    GLA_TRY(qr_tblock_dev<T>(s, m, n, F, ldf, tau, Tm, n, rest));                // :64-83
-    GLA_TRY(qr_apply_dev<T>(s, 'T', m, nrhs, n, F, ldf, Tm, n, B, ldb, rest));   // lmul!(Hᴴ, B)
+    GLA_TRY(unit_lower_explicit<T>(s, m, n, F, ldf, Vw, m));
+    GLA_TRY(gemm<T>(s, 'T', 'N', 0, n, n, m, T(1), Vw, m, Vw, m, T(0), G, n));
+    hipLaunchKernelGGL((unit_scale_k<T>), g2(n, n), dim3(256), 0, s, n, G, tau);
+    GLA_LAUNCH_CHECK();
+    // W = VᵀB, Z = (L⁻¹ W)ᵀ, W2 = D Zᵀ, B -= V W2
+    GLA_TRY(gemm<T>(s, 'T', 'N', 0, n, nrhs, m, T(1), Vw, m, B, ldb, T(0), W, n, 0, split, 8 * nr));
+    hipLaunchKernelGGL((to_rows_k<T>), g2(n, nrhs), dim3(256), 0, s, n, nrhs, W, n, Z, 0);
+    GLA_LAUNCH_CHECK();
+    GLA_TRY(tile_inverses<T>(s, n, G, n, Gi));
+    GLA_TRY(trsm_rlt<T>(s, nrhs, n, G, n, Gi, Z, nrhs));
+    hipLaunchKernelGGL((scaled_cols_k<T>), g2(n, nrhs), dim3(256), 0, s, n, nrhs, Z, tau, W2);
+    GLA_LAUNCH_CHECK();
+    GLA_TRY(gemm<T>(s, 'N', 'N', 0, m, nrhs, n, T(-1), Vw, m, W2, n, T(1), B, ldb));
     // R x = y: Z = yᵀ J, Z <- Z Kr⁻ᵀ, x = (Z J)ᵀ
+    T *Kr = G, *Kri = Gi;
     hipLaunchKernelGGL((to_rows_k<T>), g2(n, nrhs), dim3(256), 0, s, n, nrhs, B, ldb, Z, 1);
     GLA_LAUNCH_CHECK();
     hipLaunchKernelGGL((rev_lower_k<T>), g2(n, n), dim3(256), 0, s, n, F, ldf, Kr, n, 0);
