@@ -20,6 +20,7 @@
 // reference's to rounding for any step width.
 #include <algorithm>
 
+#include "gla_coherent.hpp"
 #include "gla_internal.hpp"
 
 namespace gla {
@@ -70,9 +71,10 @@ __global__ __launch_bounds__(256) void zgemm_kernel(int64_t M, int64_t N, int64_
             accr[i][j] = acc_t{0, 0, 0, 0};
             acci[i][j] = acc_t{0, 0, 0, 0};
         }
-    for (int64_t k0 = k_begin; k0 < k_end; k0 += kZK) {
-        T ar[4], ai[4], br[4], bi[4];
-        // op(A) (x, k): N — A[x + k·lda]; C — conj(A[k + x·lda])
+    // slab at k0 of op(A) (x, k): N — A[x + k·lda]; C — conj(A[k + x·lda]);
+    // and of op(B) (k, y): N — B[k + y·ldb]; C — conj(B[y + k·ldb])
+    T ar[4], ai[4], br[4], bi[4];
+    auto fetch = [&](int64_t k0) {
 #pragma unroll
         for (int l = 0; l < 4; ++l) {
             int x, k;
@@ -87,7 +89,6 @@ __global__ __launch_bounds__(256) void zgemm_kernel(int64_t M, int64_t N, int64_
                 ai[l] = TA ? -p[1] : p[1];
             }
         }
-        // op(B) (k, y): N — B[k + y·ldb]; C — conj(B[y + k·ldb])
 #pragma unroll
         for (int l = 0; l < 4; ++l) {
             int y, k;
@@ -102,6 +103,11 @@ __global__ __launch_bounds__(256) void zgemm_kernel(int64_t M, int64_t N, int64_
                 bi[l] = TB ? -p[1] : p[1];
             }
         }
+    };
+    // one slab ahead: VᴴA 64×64, K = 4096 in splits of 128: 48 µs (100 in
+    // splits of 256 with every load waited for)
+    fetch(k_begin);
+    for (int64_t k0 = k_begin; k0 < k_end; k0 += kZK) {
         __syncthreads();   // the previous slab is consumed
 #pragma unroll
         for (int l = 0; l < 4; ++l) {
@@ -117,6 +123,7 @@ __global__ __launch_bounds__(256) void zgemm_kernel(int64_t M, int64_t N, int64_
             Bi[kb * LD + y] = bi[l];
         }
         __syncthreads();
+        if (k0 + kZK < k_end) fetch(k0 + kZK);   // in flight behind this slab's products
 #pragma unroll
         for (int kk = 0; kk < kZK / 4; ++kk) {
             const int kr = kk * 4 + (lane >> 4);
@@ -181,6 +188,7 @@ __global__ void zsplit_reduce_kernel(int64_t M, int64_t N, int S, const T *__res
     if (e >= M * N) return;
     const int64_t r = e % M, c = e / M;
     T re = T(0), im = T(0);
+#pragma unroll 8
     for (int z = 0; z < S; ++z) {
         re += part[2 * ((int64_t)z * M * N + e)];
         im += part[2 * ((int64_t)z * M * N + e) + 1];
@@ -207,7 +215,7 @@ int zgemm_launch(hipStream_t s, int64_t M, int64_t N, int64_t K, T alpha, const 
     const int64_t tiles = cdiv(M, kZB) * cdiv(N, kZB);
     int64_t S = 1;
     if (MODE == 0 && !HERM && ws && tiles < 128 && K >= 1024) {
-        S = std::min<int64_t>(std::min<int64_t>(cdiv(K, 256), std::max<int64_t>(1, 256 / tiles)),
+        S = std::min<int64_t>(std::min<int64_t>(cdiv(K, 128), std::max<int64_t>(1, 512 / tiles)),
                               64);
         while (S > 1 && 2 * S * M * N > ws_elems) --S;
     }
@@ -763,6 +771,368 @@ int zqr_panel(hipStream_t s, int64_t m, int w, T *A, int64_t lda, T *tau, T *ws)
     return GLA_OK;
 }
 
+// ---- one launch per block column ----
+// qrUnblocked! of the m×w block column (w ≤ 64) over P workgroups that hold
+// 128 rows each in registers: wave v columns 8v…8v+7, lane l rows l + 64q.
+// Per column j: its owner puts it in LDS; every lane forms its rows' share of
+// xᴴ a_c (rows > j) for its wave's columns, summed over the wave; the
+// workgroup publishes the sums and workgroup 0 also row j, tagged; every
+// workgroup gathers all of them in a fixed order (so all hold the same
+// totals), forms reflector!'s scalars and applies them to its registers.
+// One more workgroup holds no rows: it follows the exchange and builds T from
+// the totals of the finished columns (v_iᴴ v_j = conj(a_ji) + conj(d_i)/ξ).
+// Every column has an exchange slot of its own, so nobody waits for it.
+// Bound: latency.  4096×64 FP64: 315 µs, 4.9 µs a column, of which the round
+// trip through the device-coherent level takes about 2 (3700 cycles for one
+// batch of loads) and the chain of sums, square root and update the rest; the
+// two launches per column it replaced took 14.6 µs.
+constexpr int kZP = 64;                 // panel width
+constexpr int kZPThreads = 512;
+constexpr int kZPRPL = 2;               // rows per lane
+constexpr int kZPRows = 64 * kZPRPL;    // rows per workgroup
+constexpr int kZPMaxP = 127;            // workgroups with rows: beyond, the launches per column
+
+template <typename T>
+struct ZPanelP {
+    int64_t m;
+    int w, kmax;
+    T *A;
+    int64_t lda;
+    T *tau, *V, *Tm;
+    int64_t ldv;
+    uint4 *xch;          // [kZP columns][P + 1][kZP] tagged complex values
+    unsigned tag0;       // tags tag0 + 1 … tag0 + kmax
+    unsigned spin_limit;
+};
+
+// Sums of v[0…15] over the wave: lane l returns, for its group of eight
+// lanes, the totals of v[8·bit5 + 4·bit4 + 2·bit3] and the one after it.
+template <typename T>
+__device__ __forceinline__ void wave_reduce16(const T v[16], T &z0, T &z1)
+{
+    const bool b3 = threadIdx.x & 8;
+    T u[8], w[4];
+#pragma unroll
+    for (int k = 0; k < 8; ++k) u[k] = pair_sum32<T>(v[k], v[k + 8]);
+#pragma unroll
+    for (int k = 0; k < 4; ++k) w[k] = pair_sum16<T>(u[k], u[k + 4]);
+    z0 = (b3 ? w[2] : w[0]) + dppmov<0x128>(b3 ? w[0] : w[2]);   // row_ror:8
+    z1 = (b3 ? w[3] : w[1]) + dppmov<0x128>(b3 ? w[1] : w[3]);
+    z0 += dppmov<0xB1>(z0);
+    z1 += dppmov<0xB1>(z1);
+    z0 += dppmov<0x4E>(z0);
+    z1 += dppmov<0x4E>(z1);
+    z0 += dppmov<0x141>(z0);
+    z1 += dppmov<0x141>(z1);
+}
+
+template <typename T>
+__global__ __launch_bounds__(kZPThreads) void zqr_panel_kernel(ZPanelP<T> p)
+{
+    constexpr int RPL = kZPRPL, NB = kZP, H = kZPThreads / NB;   // H = waves = 8
+    constexpr int EW = sizeof(T) / 4;                            // uint4 per complex value
+    __shared__ T xs[2][kZPRows][2];
+    __shared__ T red[H][NB][2];
+    __shared__ T tot[NB][2], rowj[NB][2], rows[NB][2], scal[5];
+    __shared__ T Ts[2 * NB * NB];                                // T, column-major
+    const int t = threadIdx.x, lane = t & 63;
+    const int wv = __builtin_amdgcn_readfirstlane(t >> 6);
+    const int wg = blockIdx.x, P = gridDim.x - 1;
+    const bool tw = wg == P;                                     // the one that builds T
+    const int64_t row0 = (int64_t)wg * kZPRows;
+    const int c0 = 8 * wv;
+
+    T ar[8][RPL], ai[8][RPL];
+#pragma unroll
+    for (int c = 0; c < 8; ++c)
+#pragma unroll
+        for (int q = 0; q < RPL; ++q) {
+            const int64_t r = row0 + lane + 64 * q;
+            const bool ok = !tw && r < p.m && c0 + c < p.w;
+            const T *src = p.A + 2 * ((ok ? r : 0) + (int64_t)(ok ? c0 + c : 0) * p.lda);
+            const T re = src[0], im = src[1];
+            ar[c][q] = ok ? re : T(0);
+            ai[c][q] = ok ? im : T(0);
+        }
+    if (tw)
+        for (int e = t; e < 2 * NB * NB; e += kZPThreads) Ts[e] = T(0);
+
+    for (int j = 0; j < p.kmax; ++j) {
+        const unsigned tag = p.tag0 + (unsigned)j + 1;
+        uint4 *xb = p.xch + (size_t)j * (P + 1) * NB * EW;
+        T xr[RPL], xi[RPL];
+        if (!tw) {
+            // (1) column j to LDS
+            const int buf = j & 1;
+            if (wv == j / 8) {
+                auto put = [&](const T (&re)[RPL], const T (&im)[RPL]) {
+#pragma unroll
+                    for (int q = 0; q < RPL; ++q) {
+                        xs[buf][lane + 64 * q][0] = re[q];
+                        xs[buf][lane + 64 * q][1] = im[q];
+                    }
+                };
+                switch (j % 8) {
+                case 0: put(ar[0], ai[0]); break;
+                case 1: put(ar[1], ai[1]); break;
+                case 2: put(ar[2], ai[2]); break;
+                case 3: put(ar[3], ai[3]); break;
+                case 4: put(ar[4], ai[4]); break;
+                case 5: put(ar[5], ai[5]); break;
+                case 6: put(ar[6], ai[6]); break;
+                default: put(ar[7], ai[7]); break;
+                }
+            }
+            lds_barrier();
+            // (2) xᴴ a_c over this workgroup's rows > j
+#pragma unroll
+            for (int q = 0; q < RPL; ++q) {
+                const bool below = row0 + lane + 64 * q > j;
+                const T a = xs[buf][lane + 64 * q][0], b = xs[buf][lane + 64 * q][1];
+                xr[q] = below ? a : T(0);
+                xi[q] = below ? b : T(0);
+            }
+            T d[16];
+#pragma unroll
+            for (int c = 0; c < 8; ++c) {
+                T dr = T(0), di = T(0);
+#pragma unroll
+                for (int q = 0; q < RPL; ++q) {
+                    dr = fma_t(xi[q], ai[c][q], fma_t(xr[q], ar[c][q], dr));
+                    di = fma_t(-xi[q], ar[c][q], fma_t(xr[q], ai[c][q], di));
+                }
+                d[c] = dr;
+                d[8 + c] = di;
+            }
+            T z0, z1;
+            wave_reduce16<T>(d, z0, z1);
+            auto put = [&](int pp, int c, int cp, T v) {
+                uint4 *e = xb + ((size_t)pp * NB + c) * EW;
+                if constexpr (sizeof(T) == 8) tagged_store(e + cp, v, tag);
+                else tagged_store(reinterpret_cast<uint2 *>(e) + cp, v, tag);
+            };
+            if ((lane & 7) < 2)
+                put(wg, c0 + 4 * ((lane >> 4) & 1) + 2 * ((lane >> 3) & 1) + (lane & 1), lane >> 5,
+                    lane & 1 ? z1 : z0);
+            if (wg == 0) {                // row j < 64 is workgroup 0's, q = 0
+                if (lane == j) {
+#pragma unroll
+                    for (int c = 0; c < 8; ++c) {
+                        rows[c0 + c][0] = ar[c][0];
+                        rows[c0 + c][1] = ai[c][0];
+                    }
+                }
+                __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
+                if (lane < 16) put(P, c0 + lane / 2, lane & 1, rows[c0 + lane / 2][lane & 1]);
+            }
+        }
+        // (3) wave h sums column `lane` over the workgroups ≡ h (mod 8); row j
+        // travels with wave 7's first batch
+        {
+            const int h = wv;
+            const int cnt = h < P ? (P - h + H - 1) / H : 0;
+            T sr = T(0), si = T(0);
+            constexpr int EB = 8 / EW;            // entries per batch of eight loads
+            bool lost = false;
+            for (int i0 = 0; i0 == 0 || i0 < cnt; i0 += EB) {
+                const tagged4 *ptr[10];
+                tagged4 v[10];
+                const bool row = h == H - 1 && i0 == 0;
+                auto entry = [&](int pp) {
+                    return reinterpret_cast<const tagged4 *>(xb + ((size_t)pp * NB + lane) * EW);
+                };
+                // past the last: row j, whose words arrive as well
+#pragma unroll
+                for (int u = 0; u < 8; ++u)
+                    ptr[u] = entry(i0 + u / EW < cnt ? h + (i0 + u / EW) * H : P) + u % EW;
+                ptr[8] = row ? entry(P) : ptr[0];
+                ptr[9] = row ? entry(P) + (EW - 1) : ptr[0];
+                unsigned spins = 0;
+                for (;;) {
+                    tagged_load10(ptr, v);
+                    bool ok = true;
+#pragma unroll
+                    for (int u = 0; u < 10; ++u) ok = ok && v[u][1] == tag && v[u][3] == tag;
+                    if (__all(ok)) break;
+                    if (++spins > p.spin_limit) {
+                        lost = true;
+                        break;
+                    }
+                }
+                auto value = [&](int e, T &re, T &im) {
+                    if constexpr (sizeof(T) == 8) {
+                        re = tagged_value(v[e]);
+                        im = tagged_value(v[e + 1]);
+                    } else {
+                        re = __builtin_bit_cast(float, (unsigned)v[e][0]);
+                        im = __builtin_bit_cast(float, (unsigned)v[e][2]);
+                    }
+                };
+#pragma unroll
+                for (int e = 0; e < EB; ++e) {
+                    T re, im;
+                    value(e * EW, re, im);
+                    if (i0 + e < cnt) {
+                        sr += re;
+                        si += im;
+                    }
+                }
+                if (row) {
+                    T re, im;
+                    value(8, re, im);
+                    rowj[lane][0] = re;
+                    rowj[lane][1] = im;
+                }
+            }
+            // a wait that gave up makes the results NaN
+            if (lost) sr = si = T(__builtin_nan(""));
+            red[h][lane][0] = sr;
+            red[h][lane][1] = si;
+            lds_barrier();
+        }
+        // (4) wave 0, lane c: the total of column c and the reflector from
+        // column j's: ν = copysign(‖x‖, Re x_j), ξ = x_j + ν, τ = ξ/ν, the
+        // divisions by ξ and ν as products with their reciprocals; then the
+        // column's coefficient τ̄ (a_jc + d_c/ξ̄), or for a finished column
+        // g_c = v_cᴴ v_j
+        if (wv == 0) {
+            T dr = T(0), di = T(0);
+#pragma unroll
+            for (int hh = 0; hh < H; ++hh) {
+                dr += red[hh][lane][0];
+                di += red[hh][lane][1];
+            }
+            const T br = rowj[lane][0], bi = rowj[lane][1];
+            const T xjr = lane_value(br, j), xji = lane_value(bi, j), s = lane_value(dr, j);
+            T nrm, rn;
+            sqrt_and_rsqrt(xjr * xjr + xji * xji + s, nrm, rn);
+            const bool alive = nrm != T(0);
+            const T nv = copysign(nrm, xjr), rnu = copysign(rn, xjr);
+            const T er = xjr + nv, ei = xji;
+            const T den = recip_step(er * er + ei * ei);                // 1/ξ = ξ̄/|ξ|²
+            const T f_r = alive ? er * den : T(0), f_i = alive ? -ei * den : T(0);
+            const T tr = alive ? er * rnu : T(0), ti = alive ? ei * rnu : T(0);
+            T kr, ki;
+            if (lane < j) {
+                kr = br + (dr * f_r + di * f_i);        // conj(a_jc) + conj(d_c)/ξ
+                ki = -bi + (dr * f_i - di * f_r);
+            } else {
+                const T gr = br + (dr * f_r + di * f_i), gi = bi + (di * f_r - dr * f_i);
+                kr = tr * gr + ti * gi;
+                ki = tr * gi - ti * gr;
+            }
+            tot[lane][0] = kr;
+            tot[lane][1] = ki;
+            if (lane == 0) {
+                scal[0] = f_r;
+                scal[1] = f_i;
+                scal[2] = tr;
+                scal[3] = ti;
+                scal[4] = nv;
+            }
+        }
+        lds_barrier();
+        const T fr = scal[0], fi = scal[1], taur = scal[2], taui = scal[3], nu = scal[4];
+        const bool live = nu != T(0);
+        if (tw) {
+            // T[0:j, j] = −τ T[0:j, 0:j] g
+            const int i = t % NB, h = t / NB;
+            T sr = T(0), si = T(0);
+            for (int l = i + h; l < j; l += H) {
+                const T a = Ts[2 * (i + l * NB)], b = Ts[2 * (i + l * NB) + 1];
+                sr += a * tot[l][0] - b * tot[l][1];
+                si += a * tot[l][1] + b * tot[l][0];
+            }
+            red[h][i][0] = sr;
+            red[h][i][1] = si;
+            __syncthreads();
+            if (t < j) {
+                T a = T(0), b = T(0);
+#pragma unroll
+                for (int hh = 0; hh < H; ++hh) {
+                    a += red[hh][t][0];
+                    b += red[hh][t][1];
+                }
+                Ts[2 * (t + j * NB)] = -(taur * a - taui * b);
+                Ts[2 * (t + j * NB) + 1] = -(taur * b + taui * a);
+            }
+            if (t == j) {
+                Ts[2 * (j + j * NB)] = taur;
+                Ts[2 * (j + j * NB) + 1] = taui;
+            }
+            if (t == 0) {
+                p.tau[2 * j] = taur;
+                p.tau[2 * j + 1] = taui;
+            }
+            __syncthreads();
+        } else if (live) {
+            // (5) a_c −= v τ̄ (a_jc + d_c/ξ̄) right of column j; column j
+            // becomes (β, v)
+            T vr[RPL], vi[RPL];
+#pragma unroll
+            for (int q = 0; q < RPL; ++q) {
+                const int64_t r = row0 + lane + 64 * q;
+                vr[q] = r == j ? T(1) : xr[q] * fr - xi[q] * fi;
+                vi[q] = r == j ? T(0) : xr[q] * fi + xi[q] * fr;
+            }
+#pragma unroll
+            for (int c = 0; c < 8; ++c) {
+                const int cg = c0 + c;
+                if (cg > j && cg < p.w) {
+                    const T kr = tot[cg][0], ki = tot[cg][1];
+#pragma unroll
+                    for (int q = 0; q < RPL; ++q) {
+                        ar[c][q] = fma_t(vi[q], ki, fma_t(-vr[q], kr, ar[c][q]));
+                        ai[c][q] = fma_t(-vi[q], kr, fma_t(-vr[q], ki, ai[c][q]));
+                    }
+                } else if (cg == j) {
+#pragma unroll
+                    for (int q = 0; q < RPL; ++q) {
+                        const int64_t r = row0 + lane + 64 * q;
+                        ar[c][q] = r > j ? vr[q] : (r == j ? -nu : ar[c][q]);
+                        ai[c][q] = r > j ? vi[q] : (r == j ? T(0) : ai[c][q]);
+                    }
+                }
+            }
+        }
+    }
+
+    // the factored columns and the explicit V; T
+    if (tw) {
+        for (int e = t; e < p.kmax * p.kmax; e += kZPThreads) {
+            const int i = e % p.kmax, jj = e / p.kmax;
+            p.Tm[2 * (i + (int64_t)jj * NB)] = Ts[2 * (i + jj * NB)];
+            p.Tm[2 * (i + (int64_t)jj * NB) + 1] = Ts[2 * (i + jj * NB) + 1];
+        }
+        return;
+    }
+#pragma unroll
+    for (int c = 0; c < 8; ++c) {
+        const int cg = c0 + c;
+        if (cg >= p.w) continue;
+#pragma unroll
+        for (int q = 0; q < RPL; ++q) {
+            const int64_t r = row0 + lane + 64 * q;
+            if (r >= p.m) continue;
+            T *a = p.A + 2 * (r + (int64_t)cg * p.lda);
+            a[0] = ar[c][q];
+            a[1] = ai[c][q];
+            if (cg < p.kmax) {
+                T *v = p.V + 2 * (r + (int64_t)cg * p.ldv);
+                v[0] = r < cg ? T(0) : (r == cg ? T(1) : ar[c][q]);
+                v[1] = r <= cg ? T(0) : ai[c][q];
+            }
+        }
+    }
+}
+
+// Clears the tagged words of the exchange.
+__global__ void zqr_clear_kernel(uint4 *x, int64_t n)
+{
+    const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (i < n) x[i] = uint4{0u, 0u, 0u, 0u};
+}
+
 // V (m×k, ld ldv): the unit lower reflectors of F explicitly (ones on the
 // diagonal, zeros above).
 template <typename T>
@@ -919,11 +1289,118 @@ int zwy_apply_dev(hipStream_t s, char trans, int64_t mA, int64_t nA, int64_t b, 
 // products of a 32-row panel by n columns (or of a 32×32 Gram matrix).
 inline int64_t zqr_part_elems(int64_t n) { return 2 * 16 * (int64_t)kZQ * std::max<int64_t>(n, kZQ); }
 
-// qrBlocked! (src/qr.jl:113-146) for complex A: block columns w =
-// min(blocksize, 32) wide, each factored by zqr_panel, its T formed and
-// Hᴴ applied to the columns right of it.
+// Workspace of zqr_blocked_dev in elements of T, every part on 32 elements:
+// two (V, T) panel sets and two (W1, W2, split-K) update sets, since the side
+// stream updates with one while the next panel fills the other; the tagged
+// exchange.
 template <typename T>
-int zqr_blocked_dev(hipStream_t s, int64_t m, int64_t n, T *A, int64_t lda, int64_t bs, T *tau,
+struct ZqrWS {
+    T *V[2], *Tm[2], *W1[2], *W2[2], *part[2];
+    uint4 *xch;
+    int64_t part_elems, xch_words;
+    size_t elems;
+    ZqrWS(T *base, int64_t m, int64_t n)
+    {
+        size_t off = 0;
+        auto take = [&](size_t c) {
+            T *q = base ? base + off : nullptr;
+            off += (c + 31) / 32 * 32;
+            return q;
+        };
+        const int64_t P = cdiv(m, kZPRows);
+        part_elems = 2 * 16 * (int64_t)kZP * std::max<int64_t>(n, kZP);
+        for (int q = 0; q < 2; ++q) {
+            V[q] = take(2 * (size_t)m * kZP);
+            Tm[q] = take(2 * kZP * kZP);
+            W1[q] = take(2 * (size_t)kZP * n);
+            W2[q] = take(2 * (size_t)kZP * n);
+            part[q] = take((size_t)part_elems);
+        }
+        xch_words = kZP * (P + 1) * kZP * (int64_t)(sizeof(T) / 4);
+        xch = reinterpret_cast<uint4 *>(take((size_t)xch_words * (16 / sizeof(T))));
+        elems = off;
+    }
+};
+
+// qrBlocked! (src/qr.jl:113-146) for complex A, in 64-wide block columns
+// whatever the block size (the factors do not depend on it): the panel and
+// its T by one launch, then Hᴴ on the next block column, on which the next
+// panel starts while the side stream applies Hᴴ to the rest (depth-1
+// look-ahead, as qr_blocked_dev).  4096×2048 ComplexF64: 13.8 ms (45.8 with
+// 32-wide block columns, two launches per column and no look-ahead); the
+// chain of panels and next-block updates is what it takes.
+template <typename T>
+int zqr_blocked_dev(Handle *h, hipStream_t s0, int64_t m, int64_t n, T *A, int64_t lda, T *tau)
+{
+    const int64_t k = std::min(m, n);
+    GLA_TRY(ensure_workspace(h, ZqrWS<T>(nullptr, m, n).elems * sizeof(T)));
+    const ZqrWS<T> ws(reinterpret_cast<T *>(h->ws), m, n);
+    const bool la = h->qr_lookahead && cdiv(k, (int64_t)kZP) > 2;
+    const bool masked = la && h->masked != nullptr;
+    hipStream_t s = masked ? h->chain : s0, side = masked ? h->masked : h->side;
+    hipLaunchKernelGGL(zqr_clear_kernel, dim3((unsigned)cdiv(ws.xch_words, 256)), dim3(256), 0, s0,
+                       ws.xch, ws.xch_words);
+    GLA_LAUNCH_CHECK();
+    if (la) {
+        GLA_HIP_TRY(hipEventRecord(h->ev_fork, s0));
+        GLA_HIP_TRY(hipStreamWaitEvent(side, h->ev_fork, 0));
+        if (masked) GLA_HIP_TRY(hipStreamWaitEvent(s, h->ev_fork, 0));
+    }
+    int64_t step = 0;
+    for (int64_t off = 0; off < k; off += kZP, ++step) {
+        const int64_t mm = m - off, right = n - off;
+        const int q = (int)(step & 1);
+        ZPanelP<T> p;
+        p.m = mm;
+        p.w = (int)std::min<int64_t>(kZP, right);
+        p.kmax = (int)std::min<int64_t>(mm, p.w);
+        p.A = A + 2 * (off + off * lda);
+        p.lda = lda;
+        p.tau = tau + 2 * off;
+        p.V = ws.V[q];
+        p.ldv = mm;
+        p.Tm = ws.Tm[q];
+        p.xch = ws.xch;
+        p.tag0 = (unsigned)off;
+        p.spin_limit = h->spin_limit;
+        hipLaunchKernelGGL((zqr_panel_kernel<T>), dim3((unsigned)cdiv(mm, kZPRows) + 1),
+                           dim3(kZPThreads), 0, s, p);
+        GLA_LAUNCH_CHECK();
+        const int64_t n2 = right - p.w;
+        if (n2 <= 0) break;
+        T *A2 = p.A + 2 * p.w * lda;
+        if (!la) {
+            GLA_TRY(zwy_apply_dev<T>(s, 'C', mm, n2, p.kmax, p.V, mm, p.Tm, kZP, A2, lda, ws.W1[0],
+                                     ws.W2[0], ws.part[0], ws.part_elems));
+            continue;
+        }
+        const int64_t w2 = std::min<int64_t>(kZP, n2), rest = n2 - w2;
+        if (step > 0) GLA_HIP_TRY(hipStreamWaitEvent(s, h->ev_step[1], 0));
+        GLA_HIP_TRY(hipEventRecord(h->ev_step[0], s));
+        GLA_TRY(zwy_apply_dev<T>(s, 'C', mm, w2, p.kmax, p.V, mm, p.Tm, kZP, A2, lda, ws.W1[0],
+                                 ws.W2[0], ws.part[0], ws.part_elems));
+        GLA_HIP_TRY(hipStreamWaitEvent(side, h->ev_step[0], 0));
+        if (rest > 0)
+            GLA_TRY(zwy_apply_dev<T>(side, 'C', mm, rest, p.kmax, p.V, mm, p.Tm, kZP,
+                                     A2 + 2 * w2 * lda, lda, ws.W1[1], ws.W2[1], ws.part[1],
+                                     ws.part_elems));
+        GLA_HIP_TRY(hipEventRecord(h->ev_step[1], side));
+    }
+    if (la) {
+        GLA_HIP_TRY(hipEventRecord(h->ev_join, side));
+        GLA_HIP_TRY(hipStreamWaitEvent(s0, h->ev_join, 0));
+        if (masked) {
+            GLA_HIP_TRY(hipEventRecord(h->ev_fork, s));
+            GLA_HIP_TRY(hipStreamWaitEvent(s0, h->ev_fork, 0));
+        }
+    }
+    return GLA_OK;
+}
+
+// The same for matrices too tall for the panel's registers: block columns of
+// min(blocksize, 32), two launches per column (zqr_panel).
+template <typename T>
+int zqr_tall_dev(hipStream_t s, int64_t m, int64_t n, T *A, int64_t lda, int64_t bs, T *tau,
                     T *ws)
 {
     const int64_t k = std::min(m, n);
@@ -980,9 +1457,13 @@ int zqr_entry(gla_handle_t hh, int64_t m, int64_t n, void *Av, int64_t lda, int6
     if (!tau && std::min(m, n) > 0) { set_error("tau is null"); return -7; }
     if (std::min(m, n) == 0) return GLA_OK;
     GLA_HIP_TRY(hipSetDevice(h->device));
+    // the panel's workgroups must all be resident, and every one gathers from
+    // all; up to 127 of them (16256 rows) hold rows
+    if (cdiv(m, kZPRows) <= std::min(kZPMaxP, h->num_cus / 2))
+        return zqr_blocked_dev<T>(h, reinterpret_cast<hipStream_t>(stream), m, n, A, lda, tau);
     GLA_TRY(ensure_workspace(h, zqr_scratch(m, n) * sizeof(T)));
-    return zqr_blocked_dev<T>(reinterpret_cast<hipStream_t>(stream), m, n, A, lda, bs, tau,
-                              reinterpret_cast<T *>(h->ws));
+    return zqr_tall_dev<T>(reinterpret_cast<hipStream_t>(stream), m, n, A, lda, bs, tau,
+                           reinterpret_cast<T *>(h->ws));
 }
 
 template <typename T>

@@ -299,6 +299,52 @@ __device__ __forceinline__ void swap32(T v, T &lo, T &hi)
     }
 }
 
+// Lanes below 32 (even rows): a summed over the lane pair at distance 32
+// (16); the other lanes: b likewise.
+template <typename T>
+__device__ __forceinline__ T pair_sum32(T a, T b)
+{
+    if constexpr (sizeof(T) == 8) {
+        const uint2 u = __builtin_bit_cast(uint2, a), v = __builtin_bit_cast(uint2, b);
+        const auto x = __builtin_amdgcn_permlane32_swap(u.x, v.x, false, false);
+        const auto y = __builtin_amdgcn_permlane32_swap(u.y, v.y, false, false);
+        return __builtin_bit_cast(T, uint2{x[0], y[0]}) + __builtin_bit_cast(T, uint2{x[1], y[1]});
+    } else {
+        const auto x = __builtin_amdgcn_permlane32_swap(__builtin_bit_cast(unsigned, a),
+                                                        __builtin_bit_cast(unsigned, b), false, false);
+        return __builtin_bit_cast(T, (unsigned)x[0]) + __builtin_bit_cast(T, (unsigned)x[1]);
+    }
+}
+template <typename T>
+__device__ __forceinline__ T pair_sum16(T a, T b)
+{
+    if constexpr (sizeof(T) == 8) {
+        const uint2 u = __builtin_bit_cast(uint2, a), v = __builtin_bit_cast(uint2, b);
+        const auto x = __builtin_amdgcn_permlane16_swap(u.x, v.x, false, false);
+        const auto y = __builtin_amdgcn_permlane16_swap(u.y, v.y, false, false);
+        return __builtin_bit_cast(T, uint2{x[0], y[0]}) + __builtin_bit_cast(T, uint2{x[1], y[1]});
+    } else {
+        const auto x = __builtin_amdgcn_permlane16_swap(__builtin_bit_cast(unsigned, a),
+                                                        __builtin_bit_cast(unsigned, b), false, false);
+        return __builtin_bit_cast(T, (unsigned)x[0]) + __builtin_bit_cast(T, (unsigned)x[1]);
+    }
+}
+
+// 1/a to about an ulp: the hardware estimate (relative error 2^-23 or better)
+// and one third-order step (FP64) or Newton step (FP32).  For finite a with a
+// finite reciprocal.
+__device__ __forceinline__ double recip_step(double a)
+{
+    const double y = __builtin_amdgcn_rcp(a);
+    const double e = __builtin_fma(-a, y, 1.0);
+    return __builtin_fma(y, __builtin_fma(e, e, e), y);
+}
+__device__ __forceinline__ float recip_step(float a)
+{
+    const float y = __builtin_amdgcn_rcpf(a);
+    return __builtin_fmaf(y, __builtin_fmaf(-a, y, 1.0f), y);
+}
+
 // 1/√d: the hardware estimate (relative error 2^-23 or better) and, for
 // FP64, one third-order step y(1 + e/2 + 3e²/8), e = 1 − d y² (the rest is
 // 5e³/16 < 2^-70); FP32 takes one Newton step.  d = 0 gives ∞, d < 0 and
