@@ -544,6 +544,17 @@ int ensure_workspace(Handle *h, size_t bytes);
 // (the caller then takes a path without it).
 bool ensure_df(Handle *h, size_t bytes);
 
+// Launches whose workgroups wait for each other and take most of the chip
+// must not share it with another such launch: each could hold places the
+// other waits for.  resident_begin makes stream s wait for the last of them on
+// the handle's device, from any stream and thread of the process;
+// resident_end marks the new one.  Between the two the caller queues its
+// launch; a lock is held meanwhile, so every begin is followed by its end.
+// False (nothing held): the stream is being captured, where another stream's
+// launch cannot be waited for, or an event failed.
+bool resident_begin(Handle *h, hipStream_t s);
+int resident_end(Handle *h, hipStream_t s);
+
 // ------------------------------------------------------------------ GEMM --
 // C = alpha*op(A)*op(B) + beta*C  with op(A) M×K, op(B) K×N.
 // mode 0: every element; mode 1: only elements with (row + diag_off) >= col

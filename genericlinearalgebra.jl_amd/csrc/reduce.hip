@@ -28,6 +28,7 @@
 // Panel end: Ã[k+nb:, k+nb:] −= V Wᵀ + W Vᵀ (two lower-triangle GEMMs).
 #include <algorithm>
 
+#include "gla_coherent.hpp"
 #include "gla_internal.hpp"
 
 namespace gla {
@@ -379,6 +380,346 @@ __global__ __launch_bounds__(256) void tri_w_kernel(int64_t n, int64_t c, int j,
     if ((t & 63) == 0) sh[t >> 6] = vu;
     __syncthreads();
     if (t == 0) qpart[blockIdx.x] = (sh[0] + sh[1]) + (sh[2] + sh[3]);
+}
+
+// ---- symtriLower! with the matrix in registers ----
+// One launch for orders up to 2048.  Workgroup g of P = ⌈n/8⌉ holds the eight
+// rows g + P k of the full symmetric matrix; thread 2g' + f of every workgroup
+// holds the four columns g' + P (4f + u).  Every workgroup keeps the current
+// column x and the vectors v, p, w of the whole order, spread over its threads
+// like the columns.  Per column c:
+//   the workgroup that holds row c + 1 publishes it (by symmetry the column
+//   c + 1 as it stands);  the reflector's scalars from x, v;  p = Ã v for the
+//   own rows (both triangles are held, so a row's sum is complete), published;
+//   all workgroups gather p and the row;  w = τ p − (τ² vᵀp / 2) v;  the next
+//   column x = Ã[:, c+1] − v w[c+1] − w v[c+1] in every workgroup alike, and
+//   Ã −= v wᵀ + w vᵀ on the own rows (src/eigenSelfAdjoint.jl:466-491).
+// So one exchange per column, and nothing but two vectors moves, in the order
+// [g][k] in which a workgroup writes one line and a thread reads 32 bytes.
+// Each column has an exchange region of its own, filled beforehand with a
+// signalling-NaN pattern no arithmetic produces: a value is its own arrival
+// mark.  All workgroups must be resident: such launches follow one another on
+// a device (resident_begin) and take no more than half of a CU's registers,
+// so that the panel kernels, which wait within a launch too, keep their place
+// beside them.  A wait that gives up makes the result NaN.
+// Bound: latency.  n = 2048 FP64: 10.4 ms, 5.1 µs a column (3.2 at n = 512),
+// about half of it the exchange; the three launches per column of the
+// deferred form took 38 ms.  With p and the row in index order (eight
+// scattered loads a thread, every one polled) 16.8 ms.
+// Accuracy: over 224 matrices of order 17…80 the error against a __float128
+// evaluation is 0.62 of the FP64 oracle's (0.63 the deferred form; 0.76 with
+// the two products of the update subtracted one after the other).
+constexpr int kTRRows = 8;           // rows per workgroup
+constexpr int kTRMax = 2048;         // largest order: 256 workgroups of 512 threads
+
+template <typename T>
+struct NaNMark;
+template <>
+struct NaNMark<double> {
+    typedef unsigned long long bits;
+    static constexpr bits value = 0xFFF4C0DEC0DEC0DEull;
+};
+template <>
+struct NaNMark<float> {
+    typedef unsigned bits;
+    static constexpr bits value = 0xFFA5C0DEu;
+};
+template <typename T>
+__device__ __forceinline__ bool is_mark(T v)
+{
+    return __builtin_bit_cast(typename NaNMark<T>::bits, v) == NaNMark<T>::value;
+}
+
+template <typename T>
+__global__ void mark_kernel(int64_t cnt, T *p)
+{
+    const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
+    typedef typename NaNMark<T>::bits B;
+    if (i < cnt) reinterpret_cast<B *>(p)[i] = NaNMark<T>::value;
+}
+
+// Sums of v[0…7] over the wave: the lanes with l % 8 = 0 hold the total of
+// v[4·bit5 + 2·bit4 + bit3].
+template <typename T>
+__device__ __forceinline__ T wave_rows8(const T v[8])
+{
+    const bool b3 = threadIdx.x & 8;
+    T u[4], w[2];
+#pragma unroll
+    for (int k = 0; k < 4; ++k) u[k] = pair_sum32<T>(v[k], v[k + 4]);
+#pragma unroll
+    for (int k = 0; k < 2; ++k) w[k] = pair_sum16<T>(u[k], u[k + 2]);
+    T z = (b3 ? w[1] : w[0]) + dppmov<0x128>(b3 ? w[0] : w[1]);   // row_ror:8
+    z += dppmov<0xB1>(z);
+    z += dppmov<0x4E>(z);
+    z += dppmov<0x141>(z);
+    return z;
+}
+
+// Four consecutive values, device-coherent.
+__device__ __forceinline__ void store4_coherent(double *p, const double v[4])
+{
+    typedef double d2 __attribute__((ext_vector_type(2)));
+    const d2 a = {v[0], v[1]}, b = {v[2], v[3]};
+    asm volatile("global_store_dwordx4 %0, %1, off sc1\n\t"
+                 "global_store_dwordx4 %0, %2, off offset:16 sc1\n\ts_nop 1" ::"v"(p), "v"(a), "v"(b)
+                 : "memory");
+}
+__device__ __forceinline__ void store4_coherent(float *p, const float v[4])
+{
+    const f4 a = {v[0], v[1], v[2], v[3]};
+    asm volatile("global_store_dwordx4 %0, %1, off sc1\n\ts_nop 1" ::"v"(p), "v"(a) : "memory");
+}
+__device__ __forceinline__ void load4_coherent(const double *p, double v[4])
+{
+    typedef double d2 __attribute__((ext_vector_type(2)));
+    d2 a, b;
+    asm volatile("global_load_dwordx4 %0, %2, off sc1\n\t"
+                 "global_load_dwordx4 %1, %2, off offset:16 sc1\n\ts_waitcnt vmcnt(0)"
+                 : "=&v"(a), "=&v"(b)
+                 : "v"(p)
+                 : "memory");
+    v[0] = a[0]; v[1] = a[1]; v[2] = b[0]; v[3] = b[1];
+}
+__device__ __forceinline__ void load4_coherent(const float *p, float v[4])
+{
+    f4 a;
+    asm volatile("global_load_dwordx4 %0, %1, off sc1\n\ts_waitcnt vmcnt(0)"
+                 : "=&v"(a)
+                 : "v"(p)
+                 : "memory");
+    v[0] = a[0]; v[1] = a[1]; v[2] = a[2]; v[3] = a[3];
+}
+// The same from two places, in one round trip.
+__device__ __forceinline__ void load4x2_coherent(const double *p, const double *q, double v[4],
+                                                 double w[4])
+{
+    typedef double d2 __attribute__((ext_vector_type(2)));
+    d2 a, b, c, d;
+    asm volatile("global_load_dwordx4 %0, %4, off sc1\n\t"
+                 "global_load_dwordx4 %1, %4, off offset:16 sc1\n\t"
+                 "global_load_dwordx4 %2, %5, off sc1\n\t"
+                 "global_load_dwordx4 %3, %5, off offset:16 sc1\n\ts_waitcnt vmcnt(0)"
+                 : "=&v"(a), "=&v"(b), "=&v"(c), "=&v"(d)
+                 : "v"(p), "v"(q)
+                 : "memory");
+    v[0] = a[0]; v[1] = a[1]; v[2] = b[0]; v[3] = b[1];
+    w[0] = c[0]; w[1] = c[1]; w[2] = d[0]; w[3] = d[1];
+}
+__device__ __forceinline__ void load4x2_coherent(const float *p, const float *q, float v[4],
+                                                 float w[4])
+{
+    f4 a, b;
+    asm volatile("global_load_dwordx4 %0, %2, off sc1\n\t"
+                 "global_load_dwordx4 %1, %3, off sc1\n\ts_waitcnt vmcnt(0)"
+                 : "=&v"(a), "=&v"(b)
+                 : "v"(p), "v"(q)
+                 : "memory");
+    v[0] = a[0]; v[1] = a[1]; v[2] = a[2]; v[3] = a[3];
+    w[0] = b[0]; w[1] = b[1]; w[2] = b[2]; w[3] = b[3];
+}
+
+template <typename T>
+struct TriResP {
+    T *A;
+    int64_t lda;
+    int n;
+    T *tau;
+    T *xch;              // [n columns][2][P][8]
+    unsigned spin_limit;
+};
+
+template <typename T>
+__global__ __launch_bounds__(512, 4) void tri_resident_kernel(TriResP<T> q)
+{
+    constexpr int R = kTRRows, U = 4;
+    __shared__ T nred[8], vred[8], red[8][R], prow[R], vrow[R], x1s, p1s;
+    const int t = threadIdx.x, lane = t & 63, wv = t >> 6, nw = blockDim.x >> 6;
+    const int g = blockIdx.x, P = gridDim.x, n = q.n;
+    const int64_t lda = q.lda;
+    // this thread's columns i0 + P u; threads past 2P hold none
+    const int gi = t >> 1, f = t & 1;
+    const bool act = gi < P;
+    const int i0 = act ? gi + 4 * P * f : n;
+    const int eo = act ? gi * R + 4 * f : 0;          // its place in an exchanged vector
+
+    T a[R][U], x[U];
+#pragma unroll
+    for (int k = 0; k < R; ++k)
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            const int r = g + P * k, i = i0 + P * u;
+            const bool in = r < n && i < n;
+            const int hi = r > i ? r : i, lo = r > i ? i : r;
+            const T v = q.A[in ? hi + (int64_t)lo * lda : 0];
+            a[k][u] = in ? v : T(0);
+        }
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+        const int i = i0 + P * u;
+        const T v = q.A[i < n ? i : 0];
+        x[u] = i < n ? v : T(0);
+    }
+    bool lost = false;
+    int gc = 0, kc = 0;                               // c = gc + P kc
+    for (int c = 0; c < n - 2; ++c) {
+        T *pc = q.xch + (int64_t)c * 2 * P * R, *yc = pc + P * R;
+        const int c1 = c + 1;
+        const int g1 = gc + 1 < P ? gc + 1 : 0, k1 = gc + 1 < P ? kc : kc + 1;   // c + 1
+        // row c + 1, by the workgroup that holds it
+        if (g1 == g && act) {
+            T y[U];
+#pragma unroll
+            for (int u = 0; u < U; ++u) {
+                y[u] = a[0][u];
+#pragma unroll
+                for (int k = 1; k < R; ++k) y[u] = k == k1 ? a[k][u] : y[u];
+            }
+            store4_coherent(yc + eo, y);
+        }
+        // ‖x[c+1:]‖² and x[c+1]
+        T sq = T(0);
+#pragma unroll
+        for (int u = 0; u < U; ++u) sq = i0 + P * u > c ? fma_t(x[u], x[u], sq) : sq;
+        sq = wave_sum(sq);
+        if (lane == 0) nred[wv] = sq;
+        const bool own1 = t == 2 * g1 + (k1 >> 2);
+        if (own1) x1s = (k1 & 2) ? ((k1 & 1) ? x[3] : x[2]) : ((k1 & 1) ? x[1] : x[0]);
+        lds_barrier();
+        T nrm2 = T(0);
+        for (int w = 0; w < nw; ++w) nrm2 += nred[w];
+        const T nrm = sqrt(nrm2);
+        const T x1 = x1s;
+        const bool live = nrm != T(0);
+        const T nu = copysign(nrm, x1), xi = x1 + nu;
+        const T tau = live ? xi / nu : T(0);
+        const T rxi = live ? T(1) / xi : T(1);
+        T v[U];
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            const int i = i0 + P * u;
+            v[u] = i > c1 ? x[u] * rxi : (i == c1 ? T(1) : T(0));
+        }
+        if (gi == g)
+#pragma unroll
+            for (int u = 0; u < U; ++u) vrow[4 * f + u] = v[u];
+        // p for the own rows
+        T s[R];
+#pragma unroll
+        for (int k = 0; k < R; ++k) {
+            T acc = T(0);
+#pragma unroll
+            for (int u = 0; u < U; ++u) acc = fma_t(a[k][u], v[u], acc);
+            s[k] = acc;
+        }
+        const T z = wave_rows8<T>(s);
+        if ((lane & 7) == 0) red[wv][4 * (lane >> 5) + 2 * ((lane >> 4) & 1) + ((lane >> 3) & 1)] = z;
+        lds_barrier();
+        if (wv == 0 && lane < R) {
+            typedef typename NaNMark<T>::bits B;
+            T p = T(0);
+            for (int w = 0; w < nw; ++w) p += red[w][lane];
+            // rows at or before column c: nobody uses them, but their place
+            // must not keep the mark
+            const int r = g + P * lane;
+            p = r > c && r < n ? p : T(0);
+            store_coherent(reinterpret_cast<B *>(pc + g * R + lane), __builtin_bit_cast(B, p));
+            prow[lane] = p;
+        }
+        // gather p and row c + 1
+        T p[U], y[U];
+        {
+            auto marked = [](const T (&m)[U]) {
+                return is_mark(m[0]) || is_mark(m[1]) || is_mark(m[2]) || is_mark(m[3]);
+            };
+            unsigned spins = 0;
+            load4x2_coherent(pc + eo, yc + eo, p, y);
+            while (!lost && __any(marked(p))) {
+                load4_coherent(pc + eo, p);
+                if (++spins > q.spin_limit) lost = true;
+            }
+            while (!lost && __any(marked(y))) {
+                load4_coherent(yc + eo, y);
+                if (++spins > q.spin_limit) lost = true;
+            }
+        }
+        T vp = T(0);
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            const int i = i0 + P * u;
+            const bool in = i > c && i < n;
+            p[u] = in ? p[u] : T(0);
+            y[u] = in ? y[u] : T(0);
+            vp = fma_t(v[u], p[u], vp);
+        }
+        vp = wave_sum(vp);
+        if (lane == 0) vred[wv] = vp;
+        if (own1) p1s = (k1 & 2) ? ((k1 & 1) ? p[3] : p[2]) : ((k1 & 1) ? p[1] : p[0]);
+        lds_barrier();
+        // column c: the diagonal, β, v.  Only now: the waves of this workgroup
+        // have between them gathered every row, so every workgroup has loaded
+        // its part of A
+        if (gc == g) {
+#pragma unroll
+            for (int u = 0; u < U; ++u) {
+                const int i = i0 + P * u;
+                if (i >= c && i < n)
+                    q.A[i + c * lda] = i == c || !live ? x[u] : (i == c1 ? -nu : v[u]);
+            }
+            if (t == 0) q.tau[c] = tau;
+        }
+        vp = T(0);
+        for (int w = 0; w < nw; ++w) vp += vred[w];
+        const T gam = T(0.5) * tau * (tau * vp);
+        const T w1 = tau * p1s - gam;
+        T w[U];
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            w[u] = tau * p[u] - gam * v[u];
+            x[u] = y[u] - fma_t(v[u], w1, w[u]);
+        }
+#pragma unroll
+        for (int k = 0; k < R; ++k) {
+            const T vk = vrow[k], wk = tau * prow[k] - gam * vk;
+            // both products first: one rounding at the element's own magnitude
+#pragma unroll
+            for (int u = 0; u < U; ++u) a[k][u] -= fma_t(wk, v[u], vk * w[u]);
+        }
+        gc = g1;
+        kc = k1;
+    }
+    // the last 2×2 block
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+        const int i = i0 + P * u;
+        if (g == 0 && i >= n - 2 && i < n) q.A[i + (int64_t)(n - 2) * lda] = x[u];
+#pragma unroll
+        for (int k = 0; k < R; ++k)
+            if (g + P * k == n - 1 && i == n - 1) q.A[(n - 1) * (lda + 1)] = a[k][u];
+    }
+}
+
+// Orders the resident kernel takes.
+inline bool tri_resident_fits(int64_t n, int num_cus)
+{
+    return n >= 3 && n <= kTRMax && cdiv(n, kTRRows) <= num_cus;
+}
+
+// symtriLower! by the resident kernel; *done = false (and nothing queued) if
+// it cannot run here (resident_begin).
+template <typename T>
+int tri_resident(Handle *h, hipStream_t s, int64_t n, T *A, int64_t lda, T *tau, T *xch, bool *done)
+{
+    *done = resident_begin(h, s);
+    if (!*done) return GLA_OK;
+    const int64_t P = cdiv(n, kTRRows), cnt = n * 2 * P * kTRRows;
+    hipLaunchKernelGGL((mark_kernel<T>), dim3((unsigned)cdiv(cnt, 256)), dim3(256), 0, s, cnt, xch);
+    const TriResP<T> q{A, lda, (int)n, tau, xch, h->spin_limit};
+    hipLaunchKernelGGL((tri_resident_kernel<T>), dim3((unsigned)P), dim3((unsigned)cdiv(2 * P, 64) * 64),
+                       0, s, q);
+    const int rc = resident_end(h, s);
+    GLA_LAUNCH_CHECK();
+    return rc;
 }
 
 // A[i, j] <-> A[n−1−i, n−1−j] over the whole matrix (J A J in place).
@@ -801,12 +1142,16 @@ size_t symtri_scratch(int64_t n)
     const int64_t ldv = (n + 3) / 4 * 4;
     const int64_t nbk = cdiv(n, kTB);
     const int64_t g = cdiv(n, kRPB);
-    return 2 * (size_t)ldv * kPanel + (size_t)nbk * n + 2 * (size_t)nbk * kPanel + 2 * g + 64;
+    const int64_t nr = std::min<int64_t>(n, kTRMax);   // the resident kernel's exchange
+    return 2 * (size_t)ldv * kPanel +
+           std::max((size_t)nbk * n + 2 * (size_t)nbk * kPanel + 2 * g, 2 * (size_t)nr * (nr + 8)) + 64;
 }
 
-// symtriLower! on the lower triangle of A (n×n); τ (n − 1 entries, device).
+// symtriLower! on the lower triangle of A (n×n); τ (n − 1 entries, device):
+// panels of deferred updates until the trailing block fits the resident
+// kernel, which takes the rest.
 template <typename T>
-int symtri_lower_dev(hipStream_t s, int64_t n, T *A, int64_t lda, T *tau, T *ws)
+int symtri_lower_dev(Handle *h, hipStream_t s, int64_t n, T *A, int64_t lda, T *tau, T *ws)
 {
     if (n < 1) return GLA_OK;
     if (n > 1) {
@@ -818,11 +1163,17 @@ int symtri_lower_dev(hipStream_t s, int64_t n, T *A, int64_t lda, T *tau, T *ws)
     const int64_t ldv = (n + 3) / 4 * 4;
     const int64_t nbk_max = cdiv(n, kTB);
     const int64_t gmax = cdiv(n, kRPB);
+    // (P starts on 16 bytes: ldv is a multiple of 4)
     T *V = ws, *W = V + ldv * kPanel, *P = W + ldv * kPanel, *Y1 = P + nbk_max * n,
       *Y2 = Y1 + nbk_max * kPanel, *npart = Y2 + nbk_max * kPanel, *qpart = npart + gmax,
       *scal = qpart + gmax;
     const int64_t ncols = n - 2;   // columns with a reflector (:462)
     for (int64_t k = 0; k < ncols; k += kPanel) {
+        if (tri_resident_fits(n - k, h->num_cus)) {
+            bool done = false;
+            GLA_TRY(tri_resident<T>(h, s, n - k, A + k * (lda + 1), lda, tau + k, P, &done));
+            if (done) break;
+        }
         const int w = (int)std::min<int64_t>(kPanel, ncols - k);
         for (int j = 0; j < w; ++j) {
             const int64_t c = k + j;
@@ -862,14 +1213,14 @@ int symtri_lower_dev(hipStream_t s, int64_t n, T *A, int64_t lda, T *tau, T *ws)
 }
 
 template <typename T>
-int symtri_dev(hipStream_t s, char uplo, int64_t n, T *A, int64_t lda, T *tau, T *ws)
+int symtri_dev(Handle *h, hipStream_t s, char uplo, int64_t n, T *A, int64_t lda, T *tau, T *ws)
 {
     const dim3 rg((unsigned)cdiv(n, 16), (unsigned)cdiv(n, 16));
     if (uplo == 'U') {
         hipLaunchKernelGGL((reverse_kernel<T>), rg, dim3(16, 16), 0, s, n, A, lda);
         GLA_LAUNCH_CHECK();
     }
-    GLA_TRY(symtri_lower_dev<T>(s, n, A, lda, tau, ws));
+    GLA_TRY(symtri_lower_dev<T>(h, s, n, A, lda, tau, ws));
     if (uplo == 'U') {
         hipLaunchKernelGGL((reverse_kernel<T>), rg, dim3(16, 16), 0, s, n, A, lda);
         GLA_LAUNCH_CHECK();
@@ -877,8 +1228,8 @@ int symtri_dev(hipStream_t s, char uplo, int64_t n, T *A, int64_t lda, T *tau, T
     return GLA_OK;
 }
 
-template int symtri_dev<double>(hipStream_t, char, int64_t, double *, int64_t, double *, double *);
-template int symtri_dev<float>(hipStream_t, char, int64_t, float *, int64_t, float *, float *);
+template int symtri_dev<double>(Handle *, hipStream_t, char, int64_t, double *, int64_t, double *, double *);
+template int symtri_dev<float>(Handle *, hipStream_t, char, int64_t, float *, int64_t, float *, float *);
 
 // Workspace elements of bidiagonalize! for m×n.
 size_t bidiag_scratch(int64_t m, int64_t n)
@@ -995,7 +1346,7 @@ int symtri_entry(gla_handle_t hh, char uplo, int64_t n, T *A, int64_t lda, T *ta
     if (n == 0) return GLA_OK;
     GLA_HIP_TRY(hipSetDevice(h->device));
     GLA_TRY(gla::ensure_workspace(h, gla::symtri_scratch(n) * sizeof(T)));
-    return gla::symtri_dev<T>(reinterpret_cast<hipStream_t>(stream), uplo, n, A, lda, tau,
+    return gla::symtri_dev<T>(h, reinterpret_cast<hipStream_t>(stream), uplo, n, A, lda, tau,
                               reinterpret_cast<T *>(h->ws));
 }
 

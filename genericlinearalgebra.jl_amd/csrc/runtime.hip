@@ -1,6 +1,7 @@
 // Handle, workspace and error reporting of libgla_hip.so.
 #include <cstdarg>
 #include <cstring>
+#include <mutex>
 
 #include "gla_internal.hpp"
 
@@ -58,6 +59,49 @@ bool ensure_df(Handle *h, size_t bytes)
     }
     h->df_bytes = want;
     return true;
+}
+
+namespace {
+constexpr int kMaxDevices = 64;
+struct ResidentChain {
+    std::mutex lock;
+    hipEvent_t last = nullptr;   // the last resident launch, once recorded
+};
+ResidentChain g_resident[kMaxDevices];
+}  // namespace
+
+bool resident_begin(Handle *h, hipStream_t s)
+{
+    if (h->device < 0 || h->device >= kMaxDevices) return false;
+    hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(s, &cap) != hipSuccess || cap != hipStreamCaptureStatusNone) {
+        (void)hipGetLastError();
+        return false;
+    }
+    ResidentChain &c = g_resident[h->device];
+    c.lock.lock();
+    hipError_t e = hipSuccess;
+    if (!c.last) {
+        e = hipEventCreateWithFlags(&c.last, hipEventDisableTiming);
+        if (e != hipSuccess) c.last = nullptr;
+    } else {
+        e = hipStreamWaitEvent(s, c.last, 0);
+    }
+    if (e != hipSuccess) {
+        (void)hipGetLastError();
+        c.lock.unlock();
+        return false;
+    }
+    return true;
+}
+
+int resident_end(Handle *h, hipStream_t s)
+{
+    ResidentChain &c = g_resident[h->device];
+    const hipError_t e = hipEventRecord(c.last, s);
+    c.lock.unlock();
+    GLA_HIP_TRY(e);
+    return GLA_OK;
 }
 
 namespace {
