@@ -59,6 +59,45 @@ __device__ __forceinline__ void load8_coherent(const float *const p[8], float v[
         : "memory");
 }
 
+// The same from byte offsets to one wave-uniform base (below 4 GiB): half the
+// address registers.
+__device__ __forceinline__ void load8_coherent(const double *base, const unsigned off[8], double v[8])
+{
+    asm volatile(
+        "global_load_dwordx2 %0, %8, %16 sc1\n\t"
+        "global_load_dwordx2 %1, %9, %16 sc1\n\t"
+        "global_load_dwordx2 %2, %10, %16 sc1\n\t"
+        "global_load_dwordx2 %3, %11, %16 sc1\n\t"
+        "global_load_dwordx2 %4, %12, %16 sc1\n\t"
+        "global_load_dwordx2 %5, %13, %16 sc1\n\t"
+        "global_load_dwordx2 %6, %14, %16 sc1\n\t"
+        "global_load_dwordx2 %7, %15, %16 sc1\n\t"
+        "s_waitcnt vmcnt(0)"
+        : "=&v"(v[0]), "=&v"(v[1]), "=&v"(v[2]), "=&v"(v[3]), "=&v"(v[4]), "=&v"(v[5]),
+          "=&v"(v[6]), "=&v"(v[7])
+        : "v"(off[0]), "v"(off[1]), "v"(off[2]), "v"(off[3]), "v"(off[4]), "v"(off[5]),
+          "v"(off[6]), "v"(off[7]), "s"(base)
+        : "memory");
+}
+__device__ __forceinline__ void load8_coherent(const float *base, const unsigned off[8], float v[8])
+{
+    asm volatile(
+        "global_load_dword %0, %8, %16 sc1\n\t"
+        "global_load_dword %1, %9, %16 sc1\n\t"
+        "global_load_dword %2, %10, %16 sc1\n\t"
+        "global_load_dword %3, %11, %16 sc1\n\t"
+        "global_load_dword %4, %12, %16 sc1\n\t"
+        "global_load_dword %5, %13, %16 sc1\n\t"
+        "global_load_dword %6, %14, %16 sc1\n\t"
+        "global_load_dword %7, %15, %16 sc1\n\t"
+        "s_waitcnt vmcnt(0)"
+        : "=&v"(v[0]), "=&v"(v[1]), "=&v"(v[2]), "=&v"(v[3]), "=&v"(v[4]), "=&v"(v[5]),
+          "=&v"(v[6]), "=&v"(v[7])
+        : "v"(off[0]), "v"(off[1]), "v"(off[2]), "v"(off[3]), "v"(off[4]), "v"(off[5]),
+          "v"(off[6]), "v"(off[7]), "s"(base)
+        : "memory");
+}
+
 // load8_coherent plus a ninth agent-coherent load in the same round trip.
 __device__ __forceinline__ void load9_coherent(const double *const p[8], double v[8],
                                                const double *p9, double &v9)

@@ -430,6 +430,11 @@ __device__ __forceinline__ bool is_mark(T v)
     return __builtin_bit_cast(typename NaNMark<T>::bits, v) == NaNMark<T>::value;
 }
 
+// v with a signalling NaN made quiet: an element that happens to have the
+// mark's bits is no mark.
+__device__ __forceinline__ double quiet(double v) { return __builtin_canonicalize(v); }
+__device__ __forceinline__ float quiet(float v) { return __builtin_canonicalizef(v); }
+
 template <typename T>
 __global__ void mark_kernel(int64_t cnt, T *p)
 {
@@ -552,7 +557,7 @@ __global__ __launch_bounds__(512, 4) void tri_resident_kernel(TriResP<T> q)
             const bool in = r < n && i < n;
             const int hi = r > i ? r : i, lo = r > i ? i : r;
             const T v = q.A[in ? hi + (int64_t)lo * lda : 0];
-            a[k][u] = in ? v : T(0);
+            a[k][u] = in ? quiet(v) : T(0);
         }
 #pragma unroll
     for (int u = 0; u < U; ++u) {
@@ -573,7 +578,7 @@ __global__ __launch_bounds__(512, 4) void tri_resident_kernel(TriResP<T> q)
             for (int u = 0; u < U; ++u) {
                 y[u] = a[0][u];
 #pragma unroll
-                for (int k = 1; k < R; ++k) y[u] = k == k1 ? a[k][u] : y[u];
+                for (int k = 1; k < R; ++k) y[u] = k == k1 ? T(a[k][u]) : T(y[u]);
             }
             store4_coherent(yc + eo, y);
         }
@@ -1122,6 +1127,388 @@ __global__ __launch_bounds__(256) void bd_x_kernel(int64_t m, int64_t n, int64_t
     if (t == 0) npart[blockIdx.x] = (sh[0] + sh[1]) + (sh[2] + sh[3]);
 }
 
+// ---- bidiagonalize! with the matrix in registers ----
+// One launch for a tall matrix that fits 128×128 elements per workgroup on
+// ⌈m/128⌉ × ⌈n/128⌉ ≤ 256 of them.  Workgroup (gr, gc) of the PR × PC grid
+// holds rows ≡ gr (mod PR) and columns ≡ gc (mod PC): thread (row group rg,
+// column group cg) rows 4 rg + k, columns 8 cg + q of the block.  It also
+// keeps, for its own rows or columns, the column x to be reflected and the
+// vectors v, w and y, z, u.  Column i (src/svd.jl:333-345), A as it stands:
+//   L  publish d = Σ_{r>i} x_r A[r, ·] over the own rows, Σ x_r², row i and
+//      x_i;  gather over the grid column;  ‖x‖, ξ, τ;  y = A[i, ·] + d/ξ
+//      (= Aᵀv), z = A[i, ·] − τ y;  A −= τ v yᵀ;
+//   R  publish e = Σ_{c>i+1} z_c A[·, c] over the own columns, Σ z_c², column
+//      i + 1 and z_{i+1};  gather over the grid row;  w = A[·, i+1] + e/ξ
+//      (= A u);  the next column x = A[·, i+1] − τ w;  A −= τ w uᵀ.
+// Two exchanges per column; the sums travel before the norm is known, since
+// they are formed with the unscaled vector.  Arrival marks as in the
+// tridiagonal kernel; the partial sums go through a ring of three slots,
+// marked again by their owner one step after they were gathered: a
+// workgroup that gathers step i + 1 knows that its peers are done with step
+// i, and its publication of step i + 2, after which the slot's next use can
+// begin, follows the new mark.  All workgroups must be resident, as there.
+// The grid is two-dimensional since a workgroup then exchanges with a row or
+// a column of it (20 of 240 for 2500×1501) and not with all.
+// Bound: latency, two exchanges and six barriers a column.  2500×1501 FP64
+// 10.2 ms, 6.8 µs a column; the four launches per column of the deferred form
+// took 50.0 ms.  The same kernel with some of the block spilled to memory
+// took 24.4 ms: no wide stores of the block, no exit inside the loop, places
+// worked out anew per column.
+// Line: wherever the block fits.  Deferred form -> this, FP64 ms: 2×2
+// 0.072 -> 0.063, 64×64 1.28 -> 0.36, 8192×20 0.67 -> 0.18, 8192×512
+// 22.2 -> 4.3, 2048² 65.9 -> 14.9, 3000×2000 (panels first) 72.7 -> 32.3;
+// FP32 64×64 1.15 -> 0.28, 2048² 57.0 -> 14.7.
+// Accuracy: over 84 matrices of 17×17…140×64 the error against a __float128
+// evaluation is 0.69 of the FP64 oracle's (1.03 the deferred form), in FP32
+// 0.70 of the FP32 oracle's (0.84).
+constexpr int kBRLoc = 128;                 // rows and columns per workgroup
+constexpr int kBRBlk = 136;                 // an exchanged vector with its scalar
+constexpr int kBRMaxPR = 64;
+
+template <typename T>
+struct BdResP {
+    T *A;
+    int64_t lda;
+    int m, n, PR, PC;
+    T *taul, *taur;
+    T *e1, *e2;          // [3][P][kBRBlk], grid column and grid row major; e1 starts the
+                         // workspace, which ends below 4 GiB
+    T *rowb, *colb;      // [n][PC][kBRBlk], [n][PR][kBRBlk]
+    unsigned spin_limit;
+};
+
+template <typename T>
+__global__ __launch_bounds__(512, 4) void bd_resident_kernel(BdResP<T> q)
+{
+    typedef typename NaNMark<T>::bits B;
+    __shared__ T red[8][kBRLoc], gsum[4][kBRLoc];
+    __shared__ T X[kBRLoc], V[kBRLoc], Wv[kBRLoc], Y[kBRLoc], Z[kBRLoc], Uv[kBRLoc];
+    __shared__ T sp[2], ss[2], xpiv, piv;
+    const int PR = q.PR, PC = q.PC, m = q.m, n = q.n;
+    const int gr = blockIdx.x % PR, gc = blockIdx.x / PR;
+    const int64_t lda = q.lda, slot = (int64_t)PR * PC * kBRBlk;
+
+    auto mark = [](T *p) {
+        store_coherent(reinterpret_cast<B *>(p), NaNMark<T>::value);
+    };
+    auto publish = [](T *p, T v) {
+        store_coherent(reinterpret_cast<B *>(p), __builtin_bit_cast(B, v));
+    };
+
+    T a[4][8];
+    {
+        const int t = threadIdx.x, lane = t & 63, cg = lane & 15, rg = 4 * (t >> 6) + (lane >> 4);
+#pragma unroll
+        for (int k = 0; k < 4; ++k)
+#pragma unroll
+            for (int c = 0; c < 8; ++c) {
+                const int r = gr + PR * (4 * rg + k), cc = gc + PC * (8 * cg + c);
+                const bool in = r < m && cc < n;
+                const T v = q.A[in ? r + (int64_t)cc * lda : 0];
+                a[k][c] = in ? quiet(v) : T(0);
+            }
+        if (t < kBRLoc) {
+            const int r = gr + PR * t;
+            const T v = q.A[r < m ? r : 0];
+            const T x = r < m && r > 0 ? v : T(0);
+            X[t] = x;
+            if (r == 0) xpiv = v;
+            const T sq = wave_sum(x * x);
+            if (lane == 0) ss[t >> 6] = sq;
+        }
+    }
+    bool lost = false;
+
+    // Sum over the cnt partial vectors at base + e·kBRBlk (element tl, those
+    // ≡ h mod 4) into gsum, and with them the scalar parts: quarter 0 returns
+    // `line`'s element, quarter 1 sums the partials' scalars into sp, one
+    // thread of quarter 2 takes line's scalar into piv.
+    auto gather = [&](const T *base, int cnt, const T *line, int t) -> T {
+        const int tl = t & (kBRLoc - 1), h = t >> 7, lane = t & 63, wv = t >> 6;
+        T s = T(0), extra = T(0);
+        // places in the workspace, in elements
+        const unsigned b0 = (unsigned)(base - q.e1), l0 = (unsigned)(line - q.e1);
+        unsigned xo = b0;
+        if (h == 0) xo = l0 + tl;
+        else if (h == 1 && tl < cnt) xo = b0 + tl * kBRBlk + kBRLoc;
+        else if (h == 2) xo = l0 + kBRLoc;
+        for (int e0 = h; e0 == h || e0 < cnt; e0 += 28) {
+            unsigned off[8];
+            T v[8];
+#pragma unroll
+            for (int u = 0; u < 7; ++u) {
+                const int e = e0 + 4 * u;
+                off[u] = (b0 + (e < cnt ? e : 0) * kBRBlk + tl) * (unsigned)sizeof(T);
+            }
+            off[7] = xo * (unsigned)sizeof(T);
+            for (unsigned spins = 0;; ++spins) {
+                load8_coherent(q.e1, off, v);
+                bool ok = true;
+#pragma unroll
+                for (int u = 0; u < 8; ++u) ok = ok && !is_mark(v[u]);
+                if (__all(ok) || lost) break;
+                if (spins >= q.spin_limit) lost = true;
+            }
+#pragma unroll
+            for (int u = 0; u < 7; ++u)
+                if (e0 + 4 * u < cnt) s += v[u];
+            extra = v[7];
+        }
+        gsum[h][tl] = s;
+        if (h == 1) {
+            const T sc = wave_sum(tl < cnt ? extra : T(0));
+            if (lane == 0) sp[wv - 2] = sc;
+        }
+        if (t == 2 * kBRLoc) piv = extra;
+        return extra;
+    };
+
+    lds_barrier();
+    for (int i = 0; i < n; ++i) {
+        // the thread's places are worked out anew for every column: kept over
+        // the loop, they and what follows from them push the block out of the
+        // registers
+        int t = threadIdx.x;
+        asm volatile("" : "+v"(t));
+        const int lane = t & 63, wv = t >> 6, cg = lane & 15, rg = 4 * wv + (lane >> 4);
+        const int tl = t & (kBRLoc - 1);                  // element of an exchanged vector
+        T *e1 = q.e1 + (i % 3) * slot + ((int64_t)gc * PR) * kBRBlk;   // this grid column
+        T *e2 = q.e2 + (i % 3) * slot + ((int64_t)gr * PC) * kBRBlk;   // this grid row
+        T *rowi = q.rowb + ((int64_t)i * PC + gc) * kBRBlk;
+        T *coli = q.colb + ((int64_t)i * PR + gr) * kBRBlk;
+        const int li = i / PR, lc1 = (i + 1) / PC;
+        const bool has_row = i % PR == gr, has_col = i + 1 < n && (i + 1) % PC == gc;
+        // ---- L: row i, d
+        if (has_row) {
+            if (rg == li >> 2) {
+                // (one value per store: wider ones would tie the block's
+                // registers together)
+                auto put = [&](const T (&r)[8]) {
+#pragma unroll
+                    for (int c = 0; c < 8; ++c) publish(rowi + 8 * cg + c, r[c]);
+                };
+                switch (li & 3) {
+                case 0: put(a[0]); break;
+                case 1: put(a[1]); break;
+                case 2: put(a[2]); break;
+                default: put(a[3]); break;
+                }
+            }
+            if (t == 0) publish(rowi + kBRLoc, xpiv);
+        }
+        {
+            T d[8];
+            const T x0 = X[4 * rg], x1 = X[4 * rg + 1], x2 = X[4 * rg + 2], x3 = X[4 * rg + 3];
+#pragma unroll
+            for (int c = 0; c < 8; ++c)
+                d[c] = fma_t(x3, a[3][c], fma_t(x2, a[2][c], fma_t(x1, a[1][c], x0 * a[0][c])));
+            // over the wave's four row groups: lanes keep columns
+            // 4·bit5 + 2·bit4 and the next of their eight
+            T u[4], w[2];
+#pragma unroll
+            for (int k = 0; k < 4; ++k) u[k] = pair_sum32<T>(d[k], d[k + 4]);
+#pragma unroll
+            for (int k = 0; k < 2; ++k) w[k] = pair_sum16<T>(u[k], u[k + 2]);
+            const int c = 8 * cg + 4 * (lane >> 5) + 2 * ((lane >> 4) & 1);
+            red[wv][c] = w[0];
+            red[wv][c + 1] = w[1];
+        }
+        lds_barrier();
+        if (t < kBRLoc) {
+            T s = T(0);
+#pragma unroll
+            for (int w = 0; w < 8; ++w) s += red[w][t];
+            publish(e1 + gr * kBRBlk + t, s);
+            if (t == 0) publish(e1 + gr * kBRBlk + kBRLoc, ss[0] + ss[1]);
+        }
+        T line = gather(e1, PR, rowi, t);
+        lds_barrier();
+        // the left reflector
+        const T xi_ = piv;
+        const T nrm = sqrt(fma_t(xi_, xi_, sp[0] + sp[1]));
+        const bool live = nrm != T(0);
+        const T nu = copysign(nrm, xi_), xi = xi_ + nu;
+        const T tau = live ? xi / nu : T(0), rxi = live ? T(1) / xi : T(1);
+        if (t < kBRLoc) {
+            // the grid column's peers are done with the previous step's sums
+            if (i > 0) {
+                T *old = q.e1 + ((i + 2) % 3) * slot + ((int64_t)gc * PR + gr) * kBRBlk;
+                mark(old + t);
+                if (t == 0) mark(old + kBRLoc);
+            }
+            const int c = gc + PC * t;
+            const T d = (gsum[0][t] + gsum[1][t]) + (gsum[2][t] + gsum[3][t]);
+            const bool in = c > i && c < n;
+            const T y = in ? fma_t(d, rxi, line) : T(0);
+            const T z = in ? fma_t(-tau, y, line) : T(0);
+            Y[t] = y;
+            Z[t] = c > i + 1 ? z : T(0);
+            if (c == i + 1) xpiv = z;                     // z's first element
+            const T sq = wave_sum(c > i + 1 ? z * z : T(0));
+            if (lane == 0) ss[wv] = sq;
+        } else if (t < 2 * kBRLoc) {
+            const int r = gr + PR * tl;
+            V[tl] = r > i ? X[tl] * rxi : (r == i ? T(1) : T(0));
+        }
+        if (blockIdx.x == 0 && t == 0) q.taul[i] = tau;
+        const T beta_l = live ? -nu : xi_;
+        lds_barrier();
+        if (i + 1 < n) {     // the last column has no right reflector (src/svd.jl:339)
+            // A −= τ v yᵀ, then e
+            {
+                T tv[4], e[4];
+#pragma unroll
+                for (int k = 0; k < 4; ++k) {
+                    tv[k] = -tau * V[4 * rg + k];
+                    e[k] = T(0);
+                }
+                // two columns at a time: the block leaves no more registers
+#pragma unroll
+                for (int c = 0; c < 8; c += 2) {
+                    const T y0 = Y[8 * cg + c], y1 = Y[8 * cg + c + 1];
+                    const T z0 = Z[8 * cg + c], z1 = Z[8 * cg + c + 1];
+#pragma unroll
+                    for (int k = 0; k < 4; ++k) {
+                        a[k][c] = fma_t(tv[k], y0, a[k][c]);
+                        a[k][c + 1] = fma_t(tv[k], y1, a[k][c + 1]);
+                        e[k] = fma_t(z1, a[k][c + 1], fma_t(z0, a[k][c], e[k]));
+                    }
+                    __builtin_amdgcn_sched_barrier(0);
+                }
+                // over the row's 16 lanes: lane keeps row 2·bit3 + bit2 of its four
+                const bool b3 = lane & 8, b2 = lane & 4;
+                T w0 = (b3 ? e[2] : e[0]) + dppmov<0x128>(b3 ? e[0] : e[2]);   // row_ror:8
+                T w1 = (b3 ? e[3] : e[1]) + dppmov<0x128>(b3 ? e[1] : e[3]);
+                T s = (b2 ? w1 : w0) + dppmov<0x141>(b2 ? w0 : w1);            // half mirror
+                s += dppmov<0xB1>(s);
+                s += dppmov<0x4E>(s);
+                if ((lane & 3) == 0)
+                    publish(e2 + gc * kBRBlk + 4 * rg + 2 * ((lane >> 3) & 1) + ((lane >> 2) & 1), s);
+            }
+            if (has_col && cg == lc1 >> 3) {
+                auto put = [&](T r0, T r1, T r2, T r3) {
+                    publish(coli + 4 * rg, r0);
+                    publish(coli + 4 * rg + 1, r1);
+                    publish(coli + 4 * rg + 2, r2);
+                    publish(coli + 4 * rg + 3, r3);
+                };
+                switch (lc1 & 7) {
+                case 0: put(a[0][0], a[1][0], a[2][0], a[3][0]); break;
+                case 1: put(a[0][1], a[1][1], a[2][1], a[3][1]); break;
+                case 2: put(a[0][2], a[1][2], a[2][2], a[3][2]); break;
+                case 3: put(a[0][3], a[1][3], a[2][3], a[3][3]); break;
+                case 4: put(a[0][4], a[1][4], a[2][4], a[3][4]); break;
+                case 5: put(a[0][5], a[1][5], a[2][5], a[3][5]); break;
+                case 6: put(a[0][6], a[1][6], a[2][6], a[3][6]); break;
+                default: put(a[0][7], a[1][7], a[2][7], a[3][7]); break;
+                }
+            }
+            if (t == 0) {
+                publish(e2 + gc * kBRBlk + kBRLoc, ss[0] + ss[1]);
+                if (has_col) publish(coli + kBRLoc, xpiv);
+            }
+            // ---- R
+            line = gather(e2, PC, coli, t);
+            lds_barrier();
+            const T zi = piv;
+            const T nrmr = sqrt(fma_t(zi, zi, sp[0] + sp[1]));
+            const bool liver = nrmr != T(0);
+            const T nur = copysign(nrmr, zi), xir = zi + nur;
+            const T taur = liver ? xir / nur : T(0), rxir = liver ? T(1) / xir : T(1);
+            if (t < kBRLoc) {
+                if (i > 0) {
+                    T *old = q.e2 + ((i + 2) % 3) * slot + ((int64_t)gr * PC + gc) * kBRBlk;
+                    mark(old + t);
+                    if (t == 0) mark(old + kBRLoc);
+                }
+                const int r = gr + PR * t;
+                const T e = (gsum[0][t] + gsum[1][t]) + (gsum[2][t] + gsum[3][t]);
+                const bool in = r > i && r < m;
+                const T w = in ? fma_t(e, rxir, line) : T(0);
+                const T x = in ? fma_t(-taur, w, line) : T(0);
+                Wv[t] = w;
+                X[t] = r > i + 1 ? x : T(0);
+                if (r == i + 1) xpiv = x;
+                const T sq = wave_sum(r > i + 1 ? x * x : T(0));
+                if (lane == 0) ss[wv] = sq;
+            } else if (t < 2 * kBRLoc) {
+                const int c = gc + PC * tl;
+                Uv[tl] = c > i + 1 ? Z[tl] * rxir : (c == i + 1 ? T(1) : T(0));
+            }
+            if (blockIdx.x == 0 && t == 0) q.taur[i] = taur;
+            lds_barrier();
+            {
+                T tw[4];
+#pragma unroll
+                for (int k = 0; k < 4; ++k) tw[k] = -taur * Wv[4 * rg + k];
+#pragma unroll
+                for (int c = 0; c < 8; c += 2) {
+                    const T u0 = Uv[8 * cg + c], u1 = Uv[8 * cg + c + 1];
+#pragma unroll
+                    for (int k = 0; k < 4; ++k) {
+                        a[k][c] = fma_t(tw[k], u0, a[k][c]);
+                        a[k][c + 1] = fma_t(tw[k], u1, a[k][c + 1]);
+                    }
+                    __builtin_amdgcn_sched_barrier(0);
+                }
+            }
+            // row i of the result, by its holders
+            if (has_row && t >= kBRLoc && t < 2 * kBRLoc) {
+                const int c = gc + PC * tl;
+                if (c > i && c < n)
+                    q.A[i + (int64_t)c * lda] = c == i + 1 ? (liver ? -nur : zi) : Uv[tl];
+            }
+        }
+        // column i of the result, by its holders.  Only now: the grid row's
+        // peers have published e, so they have read x
+        if (i % PC == gc && t < kBRLoc) {
+            const int r = gr + PR * t;
+            if (r >= i && r < m) q.A[r + (int64_t)i * lda] = r == i ? beta_l : V[t];
+        }
+    }
+}
+
+// Shapes the resident kernel takes (m ≥ n), and its workspace in elements.
+inline bool bd_resident_fits(int64_t m, int64_t n, int num_cus)
+{
+    const int64_t PR = cdiv(m, kBRLoc), PC = cdiv(n, kBRLoc);
+    return n >= 2 && m >= n && PR <= kBRMaxPR && PR * PC <= std::min(256, num_cus);
+}
+inline size_t bd_resident_elems(int64_t m, int64_t n)
+{
+    const int64_t PR = cdiv(m, kBRLoc), PC = cdiv(n, kBRLoc);
+    return (size_t)(6 * PR * PC + n * (PR + PC)) * kBRBlk;
+}
+
+template <typename T>
+int bd_resident(Handle *h, hipStream_t s, int64_t m, int64_t n, T *A, int64_t lda, T *taul, T *taur,
+                T *ws, bool *done)
+{
+    *done = resident_begin(h, s);
+    if (!*done) return GLA_OK;
+    BdResP<T> q;
+    q.A = A;
+    q.lda = lda;
+    q.m = (int)m;
+    q.n = (int)n;
+    q.PR = (int)cdiv(m, kBRLoc);
+    q.PC = (int)cdiv(n, kBRLoc);
+    q.taul = taul;
+    q.taur = taur;
+    const size_t ring = 3 * (size_t)q.PR * q.PC * kBRBlk;
+    q.e1 = ws;
+    q.e2 = q.e1 + ring;
+    q.rowb = q.e2 + ring;
+    q.colb = q.rowb + (size_t)n * q.PC * kBRBlk;
+    q.spin_limit = h->spin_limit;
+    const int64_t cnt = (int64_t)bd_resident_elems(m, n);
+    hipLaunchKernelGGL((mark_kernel<T>), dim3((unsigned)cdiv(cnt, 256)), dim3(256), 0, s, cnt, ws);
+    hipLaunchKernelGGL((bd_resident_kernel<T>), dim3((unsigned)(q.PR * q.PC)), dim3(512), 0, s, q);
+    const int rc = resident_end(h, s);
+    GLA_LAUNCH_CHECK();
+    return rc;
+}
+
 // B (n×m, ld ldb) = Aᵀ for A m×n.
 template <typename T>
 __global__ void transpose_kernel(int64_t m, int64_t n, const T *A, int64_t lda, T *B, int64_t ldb)
@@ -1237,15 +1624,24 @@ size_t bidiag_scratch(int64_t m, int64_t n)
     const int64_t M = std::max(m, n), N = std::min(m, n);   // the tall problem
     const int64_t ldm = (M + 3) / 4 * 4, ldn = (N + 3) / 4 * 4;
     const int64_t nrb = cdiv(M, kTB), ncb = cdiv(N, kTB), g = cdiv(M, kRPB) + 1;
-    const size_t pe = std::max((size_t)nrb * N, (size_t)ncb * M);
+    // the GEMVs' partials, or the resident kernel's exchange for the largest
+    // trailing block that fits it
+    size_t pe = std::max((size_t)nrb * N, (size_t)ncb * M), re = 0;
+    for (int64_t k = 0; k < N; k += kPanel)
+        if (bd_resident_fits(M - k, N - k, 256)) {
+            re = bd_resident_elems(M - k, N - k);
+            break;
+        }
+    pe = std::max(pe, re);
     const size_t tr = m < n ? (size_t)ldm * N : 0;   // Aᵀ for the wide case
     return 2 * (size_t)ldm * kPanel + 2 * (size_t)ldn * kPanel + pe +
            2 * (size_t)nrb * kPanel + 2 * (size_t)ncb * kPanel + 2 * (size_t)g + 16 + tr;
 }
 
-// bidiagonalize! of a tall A (m ≥ n).
+// bidiagonalize! of a tall A (m ≥ n): panels of deferred updates until the
+// trailing block fits the resident kernel, which takes the rest.
 template <typename T>
-int bidiag_tall_dev(hipStream_t s, int64_t m, int64_t n, T *A, int64_t lda, T *taul, T *taur,
+int bidiag_tall_dev(Handle *h, hipStream_t s, int64_t m, int64_t n, T *A, int64_t lda, T *taul, T *taur,
                     T *ws)
 {
     const int64_t ldm = (m + 3) / 4 * 4, ldn = (n + 3) / 4 * 4;
@@ -1256,6 +1652,12 @@ int bidiag_tall_dev(hipStream_t s, int64_t m, int64_t n, T *A, int64_t lda, T *t
     T *Cu1 = Cv2 + nrb_max * kPanel, *Cu2 = Cu1 + ncb_max * kPanel;
     T *npart = Cu2 + ncb_max * kPanel, *npart2 = npart + gmax, *scal = npart2 + gmax;
     for (int64_t k = 0; k < n; k += kPanel) {
+        if (bd_resident_fits(m - k, n - k, h->num_cus)) {
+            bool done = false;
+            GLA_TRY(bd_resident<T>(h, s, m - k, n - k, A + k * (lda + 1), lda, taul + k, taur + k, P,
+                                   &done));
+            if (done) break;
+        }
         const int w = (int)std::min<int64_t>(kPanel, n - k);
         int ncnt = (int)cdiv(m - k, 256);
         hipLaunchKernelGGL((bd_col0_kernel<T>), dim3((unsigned)ncnt), dim3(256), 0, s, m, k,
@@ -1306,26 +1708,27 @@ int bidiag_tall_dev(hipStream_t s, int64_t m, int64_t n, T *A, int64_t lda, T *t
 // (its left reflectors are A's right ones, src/svd.jl:356-375 mirrors
 // :332-349), transposed back.
 template <typename T>
-int bidiag_dev(hipStream_t s, int64_t m, int64_t n, T *A, int64_t lda, T *taul, T *taur, T *ws)
+int bidiag_dev(Handle *h, hipStream_t s, int64_t m, int64_t n, T *A, int64_t lda, T *taul, T *taur,
+               T *ws)
 {
     if (m == 0 || n == 0) return GLA_OK;
-    if (m >= n) return bidiag_tall_dev<T>(s, m, n, A, lda, taul, taur, ws);
+    if (m >= n) return bidiag_tall_dev<T>(h, s, m, n, A, lda, taul, taur, ws);
     const int64_t ldt = (n + 3) / 4 * 4;
     T *At = ws;
     T *rest = ws + (size_t)ldt * m;
     hipLaunchKernelGGL((transpose_kernel<T>), dim3((unsigned)cdiv(m, 16), (unsigned)cdiv(n, 16)),
                        dim3(16, 16), 0, s, m, n, (const T *)A, lda, At, ldt);
     GLA_LAUNCH_CHECK();
-    GLA_TRY(bidiag_tall_dev<T>(s, n, m, At, ldt, taur, taul, rest));
+    GLA_TRY(bidiag_tall_dev<T>(h, s, n, m, At, ldt, taur, taul, rest));
     hipLaunchKernelGGL((transpose_kernel<T>), dim3((unsigned)cdiv(n, 16), (unsigned)cdiv(m, 16)),
                        dim3(16, 16), 0, s, n, m, (const T *)At, ldt, A, lda);
     GLA_LAUNCH_CHECK();
     return GLA_OK;
 }
 
-template int bidiag_dev<double>(hipStream_t, int64_t, int64_t, double *, int64_t, double *,
+template int bidiag_dev<double>(Handle *, hipStream_t, int64_t, int64_t, double *, int64_t, double *,
                                 double *, double *);
-template int bidiag_dev<float>(hipStream_t, int64_t, int64_t, float *, int64_t, float *, float *,
+template int bidiag_dev<float>(Handle *, hipStream_t, int64_t, int64_t, float *, int64_t, float *, float *,
                                float *);
 
 }  // namespace gla
@@ -1368,7 +1771,7 @@ int bidiag_entry(gla_handle_t hh, int64_t m, int64_t n, T *A, int64_t lda, T *ta
     if (k == 0) return GLA_OK;
     GLA_HIP_TRY(hipSetDevice(h->device));
     GLA_TRY(gla::ensure_workspace(h, gla::bidiag_scratch(m, n) * sizeof(T)));
-    return gla::bidiag_dev<T>(reinterpret_cast<hipStream_t>(stream), m, n, A, lda, taul, taur,
+    return gla::bidiag_dev<T>(h, reinterpret_cast<hipStream_t>(stream), m, n, A, lda, taul, taur,
                               reinterpret_cast<T *>(h->ws));
 }
 
