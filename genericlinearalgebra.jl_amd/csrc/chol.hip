@@ -1033,16 +1033,6 @@ int launch_solve_batched(hipStream_t s, int nb, const T *L, int64_t ldl, int64_t
 }
 
 template <typename T>
-__global__ void identity_blocks_kernel(int64_t nblk, T *D)
-{
-    const int64_t e = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (e < nblk * kPanelNB * kPanelNB) {
-        const int64_t r = e % kPanelNB, c = (e / kPanelNB) % kPanelNB;
-        D[e] = r == c ? T(1) : T(0);
-    }
-}
-
-template <typename T>
 int launch_tile_inverse(hipStream_t s, int64_t n, const T *L, int64_t ldl, T *LinvG)
 {
     if (n <= 0) return GLA_OK;
@@ -1328,30 +1318,6 @@ int trsm_rlt_batched(hipStream_t s, int64_t m, int n, const T *L, int64_t ldl, i
 }
 size_t tile_inverse_elems(int64_t n) { return linv_elems(n); }
 
-// Inverses of the 128×128 diagonal blocks of a lower n×n L, transposed:
-// block b (rows/columns 128b .. 128b+127, the last one possibly partial)
-// gets Dt_b = L_bb⁻ᵀ, column-major 128×128 at Dt + b·128².  Linv holds the
-// 16×16 diagonal-tile inverses of L (tile_inverses).  Two launches: the
-// identity, then every block's rdiv! I·L_bb⁻ᵀ at once.
-template <typename T>
-int diag_block_inverses(hipStream_t s, int64_t n, const T *L, int64_t ldl, const T *Linv, T *Dt)
-{
-    if (n <= 0) return GLA_OK;
-    const int64_t nblk = cdiv(n, kPanelNB), nfull = n / kPanelNB;
-    const int64_t bs = (int64_t)kPanelNB * kPanelNB;
-    hipLaunchKernelGGL((identity_blocks_kernel<T>), dim3((unsigned)cdiv(nblk * bs, 256)), dim3(256),
-                       0, s, nblk, Dt);
-    GLA_LAUNCH_CHECK();
-    const int64_t dstride = kPanelNB * (1 + ldl), lstride = (kPanelNB / 16) * 256;
-    GLA_TRY(launch_solve_batched<T>(s, kPanelNB, L, ldl, dstride, Linv, lstride, Dt, kPanelNB, bs,
-                                    kPanelNB, nfull));
-    if (nfull < nblk)
-        GLA_TRY(launch_solve_batched<T>(s, (int)(n - nfull * kPanelNB), L + nfull * dstride, ldl, 0,
-                                        Linv + nfull * lstride, 0, Dt + nfull * bs, kPanelNB, 0,
-                                        kPanelNB, 1));
-    return GLA_OK;
-}
-
 #define GLA_INST_BLOCKS(T)                                                                    \
     template int chol_factor_block<T>(hipStream_t, int, T *, int64_t, int *, int64_t, T *);  \
     template int ldlt_factor_block<T>(hipStream_t, int, T *, int64_t, T *);                  \
@@ -1367,8 +1333,7 @@ int diag_block_inverses(hipStream_t s, int64_t n, const T *L, int64_t ldl, const
     template int tile_inverses_batched<T>(hipStream_t, int64_t, const T *, int64_t, int64_t,  \
                                           T *, int64_t, int64_t);                             \
     template int trsm_rlt_batched<T>(hipStream_t, int64_t, int, const T *, int64_t, int64_t,  \
-                                     const T *, int64_t, T *, int64_t, int64_t, int64_t);     \
-    template int diag_block_inverses<T>(hipStream_t, int64_t, const T *, int64_t, const T *, T *);
+                                     const T *, int64_t, T *, int64_t, int64_t, int64_t);
 
 GLA_INST_BLOCKS(double)
 GLA_INST_BLOCKS(float)

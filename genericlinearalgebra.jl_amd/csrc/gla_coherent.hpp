@@ -20,6 +20,31 @@ __device__ __forceinline__ T load_coherent(const T *p)
     return __hip_atomic_load(const_cast<T *>(p), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
+// Arrival marks: a signalling NaN that no arithmetic produces, with which an
+// exchange is filled before its values come.
+template <typename T>
+struct NaNMark;
+template <>
+struct NaNMark<double> {
+    typedef unsigned long long bits;
+    static constexpr bits value = 0xFFF4C0DEC0DEC0DEull;
+};
+template <>
+struct NaNMark<float> {
+    typedef unsigned bits;
+    static constexpr bits value = 0xFFA5C0DEu;
+};
+template <typename T>
+__device__ __forceinline__ bool is_mark(T v)
+{
+    return __builtin_bit_cast(typename NaNMark<T>::bits, v) == NaNMark<T>::value;
+}
+
+// v with a signalling NaN made quiet: an element that happens to have the
+// mark's bits is no mark.
+__device__ __forceinline__ double quiet(double v) { return __builtin_canonicalize(v); }
+__device__ __forceinline__ float quiet(float v) { return __builtin_canonicalizef(v); }
+
 // Eight agent-coherent (sc1) loads in flight at once, then one wait.  The
 // compiler issues relaxed atomic loads one round trip at a time; this block
 // keeps the memory-level parallelism.  Outputs are early-clobber and the

@@ -637,27 +637,40 @@ template <typename T>
 int trsm_rlt(hipStream_t s, int64_t m, int64_t n, const T *L, int64_t ldl, const T *Linv, T *B,
              int64_t ldb);
 size_t tile_inverse_elems(int64_t n);
-// Dt_b = L_bb⁻ᵀ for every 128×128 diagonal block b of L (column-major
-// 128×128 at Dt + b·128²), from the tile inverses Linv.
+// Y = M⁻¹ R for a few right-hand sides in one launch (trsv.hip).  M lower
+// triangular of order n, element (i, j) at M[i·si + j·sj], one stride ±1
+// (a leading stride of 1 is read first); only i ≥ j is read, and with `unit`
+// not the diagonal.  R's element (i, k) at R[i·ri + (k mod 16)·rk +
+// (k div 16)·rp], divided by div[i·ds] if div is given.  Y: tri_solve_elems
+// elements, rows of 16 per pass (element (i, k) at [(k div 16)·npad·16 + 16 i +
+// k mod 16], npad = n rounded up to 128), and a ticket, both set by
+// tri_solve_prepare.  If `out` is given, out[i·oi + k·ok] = mul[i·ms]·y (mul
+// may be null); if X is, X[i·oi + k·ok] += y.
 template <typename T>
-int diag_block_inverses(hipStream_t s, int64_t n, const T *L, int64_t ldl, const T *Linv, T *Dt);
-
-// Multi-right-hand-side lower triangular solve (trsv.hip): Y = L⁻¹ R for up
-// to 16 right-hand sides held row-major (element (i, k) at [16 i + k]),
-// blocked by 128 rows, one launch.  Dt from diag_block_inverses, Mt from
-// diag_sub (npad × 128, npad = n rounded up to 128).  rev:
-// row i of the solve reads R row n−1−i and adds into X row n−1−i (the
-// backward solve Lᵀ z = y run as a lower solve with the reversed matrix
-// J Lᵀ J).  If X is given, X[·, k] += Y[·, k] for k < nrhs (FP64,
-// column-major).  Y is scratch of the same layout; flags: one int per
-// 128-row block, values below `epoch`; err is raised if a wait times out.
+struct TriSolve {
+    int64_t n;
+    const T *M;
+    int64_t si, sj;
+    int unit, nrhs;
+    const T *R;
+    int64_t ri, rk, rp;
+    const T *div;
+    int64_t ds;
+    T *Y, *out;
+    double *X;
+    int64_t oi, ok;
+    const T *mul;
+    int64_t ms;
+    int *ticket, *err;       // *err = 1 if a wait gave up (err may be null)
+    unsigned spin_limit;
+    int npass;               // set by tri_solve
+};
+size_t tri_solve_elems(int64_t n, int64_t nrhs);
+// cnt elements of Y marked, and the tickets of `solves` launches zeroed.
 template <typename T>
-int trsv16(Handle *h, hipStream_t s, int64_t n, const T *L, int64_t ldl, const T *Dt, const T *Mt,
-           const T *R, T *Y, int rev, double *X, int64_t ldx, int nrhs, int *flags, int epoch,
-           int *err);
-// Mt (npad × 128) = L_bb⁻¹ L_{b,b−1} stacked over the 128-row blocks b ≥ 1.
+int tri_solve_prepare(hipStream_t s, int64_t cnt, T *Y, int *ticket, int solves);
 template <typename T>
-int diag_sub(hipStream_t s, int64_t n, const T *L, int64_t ldl, const T *Dt, T *Mt);
+int tri_solve(hipStream_t s, TriSolve<T> p);
 // R (row-major n×16, type T) = B − sym(A) X for the lower-stored FP64 A and
 // nrhs ≤ 16 columns of X, B (column-major); Xt: symv_scratch(n) doubles;
 // nrm[k] += ‖r_k‖², nrm[16 + k] += ‖x_k‖² (nrm zeroed by the caller).

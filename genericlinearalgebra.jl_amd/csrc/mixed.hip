@@ -15,9 +15,8 @@
 //            until the normwise backward error
 //            η = max_k ‖r_k‖ / (‖A‖_F ‖x_k‖ + ‖b_k‖) ≤ tol.
 //
-// The triangular solves are one-launch dataflow solves (trsv16): L y = r
-// directly, and Lᵀ z = y as a lower solve with the reversed matrix
-// L' = P Lᵀ P (P the reversal), z = P (L'⁻¹ (P y)).
+// The triangular solves are one launch each (tri_solve): L y = r, and
+// Lᵀ z = y with rows and columns from the last.
 #include <algorithm>
 #include <cmath>
 #include <type_traits>
@@ -429,13 +428,6 @@ __global__ void cvt_lower_d2s(int64_t n, const double *src, int64_t lds, float *
     GLA_ROW(i);
     GLA_COLS(j, n) if (i < n && i >= j) dst[i + j * ldd] = (float)src[i + j * lds];
 }
-// Lr[i][j] = L[n-1-j][n-1-i] for i >= j: the reversal P Lᵀ P, lower.
-template <typename T>
-__global__ void reverse_transpose_lower(int64_t n, const T *L, int64_t ldl, T *Lr, int64_t ldr)
-{
-    GLA_ROW(i);
-    GLA_COLS(j, n) if (i < n && i >= j) Lr[i + j * ldr] = L[(n - 1 - j) + (n - 1 - i) * ldl];
-}
 __global__ void copy2d_d(int64_t m, int64_t n, const double *S, int64_t lds, double *D, int64_t ldd)
 {
     GLA_ROW(i);
@@ -575,11 +567,6 @@ int chol_mixed_la(Handle *h, hipStream_t s, int64_t n, float *W, int64_t ldw, fl
     return GLA_OK;
 }
 
-__global__ void fill_int(int64_t n, int *p, int v)
-{
-    const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < n) p[i] = v;
-}
 __global__ void fill_dbl(int64_t n, double *p)
 {
     const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
@@ -602,32 +589,30 @@ double backward_error(const double *rr, const double *xx, const double *bb, int6
 // Workspace of one mixed solve (element type T of the factor).
 template <typename T>
 struct MixedWS {
-    T *W, *Lr, *Linv, *Linvr, *Dt, *Dtr, *Mt, *Mtr, *Rt, *Yt, *Zt;
+    T *W, *Linv, *Rt, *Yt;   // Yt: the exchanges of the two solves
     double *Xt, *nrm;
     float *Linv32;
-    int *flags, *err;
+    int *ticket, *err;
     // packed low-precision panels (A' and B' of two alternating steps),
     // pk_bytes each, and their FP16 scale words
     void *pk0a, *pk0b, *pk1a, *pk1b;
     unsigned *maxbits;
-    int64_t nblk, npad, nchunk;
+    int64_t npad, nchunk;
 
     // pk_bytes: one packed panel of the BF16/FP16 factorisation (0 otherwise)
     static size_t bytes(int64_t n, int64_t nrhs, size_t pk_bytes)
     {
-        const int64_t nblk = cdiv(n, 128), npad = nblk * 128, nch = cdiv(nrhs, 16);
+        const int64_t npad = cdiv(n, 128) * 128, nch = cdiv(nrhs, 16);
         const size_t es = sizeof(T), r = 255;
         auto al = [&](size_t b) { return (b + r) / 256 * 256; };
-        return 2 * al(es * (size_t)n * n) + 2 * al(es * tile_inverse_elems(n)) +
-               4 * al(es * (size_t)npad * 128) + al(es * (size_t)npad * 16 * nch) +
-               2 * al(es * (size_t)npad * 16) + al(8 * symv_scratch(n)) +
-               al(8 * (size_t)(32 * nch + n + 64)) +
-               al(4 * 8 * 256) + al(4 * (size_t)(nblk + 64)) + 4 * al(pk_bytes) + 4096;
+        return al(es * (size_t)n * n) + al(es * tile_inverse_elems(n)) +
+               al(es * (size_t)npad * 16 * nch) + al(es * 2 * tri_solve_elems(n, nrhs)) +
+               al(8 * symv_scratch(n)) + al(8 * (size_t)(32 * nch + n + 64)) +
+               al(4 * 8 * 256) + al(4 * 64) + 4 * al(pk_bytes) + 4096;
     }
     void carve(void *base, int64_t n, int64_t nrhs, size_t pk_bytes)
     {
-        nblk = cdiv(n, 128);
-        npad = nblk * 128;
+        npad = cdiv(n, 128) * 128;
         nchunk = cdiv(nrhs, 16);
         char *p = reinterpret_cast<char *>(base);
         auto take = [&](size_t b) {
@@ -637,22 +622,15 @@ struct MixedWS {
         };
         const size_t es = sizeof(T);
         W = reinterpret_cast<T *>(take(es * (size_t)n * n));
-        Lr = reinterpret_cast<T *>(take(es * (size_t)n * n));
         Linv = reinterpret_cast<T *>(take(es * tile_inverse_elems(n)));
-        Linvr = reinterpret_cast<T *>(take(es * tile_inverse_elems(n)));
-        Dt = reinterpret_cast<T *>(take(es * (size_t)npad * 128));
-        Dtr = reinterpret_cast<T *>(take(es * (size_t)npad * 128));
-        Mt = reinterpret_cast<T *>(take(es * (size_t)npad * 128));
-        Mtr = reinterpret_cast<T *>(take(es * (size_t)npad * 128));
         Rt = reinterpret_cast<T *>(take(es * (size_t)npad * 16 * nchunk));
-        Yt = reinterpret_cast<T *>(take(es * (size_t)npad * 16));
-        Zt = reinterpret_cast<T *>(take(es * (size_t)npad * 16));
+        Yt = reinterpret_cast<T *>(take(es * 2 * tri_solve_elems(n, nrhs)));
         Xt = reinterpret_cast<double *>(take(8 * symv_scratch(n)));
         nrm = reinterpret_cast<double *>(take(8 * (size_t)(32 * nchunk + n + 64)));
         Linv32 = reinterpret_cast<float *>(take(4 * 8 * 256));
-        flags = reinterpret_cast<int *>(take(4 * (size_t)(nblk + 64)));
-        err = flags + nblk;
-        maxbits = reinterpret_cast<unsigned *>(flags + nblk + 8);
+        ticket = reinterpret_cast<int *>(take(4 * 64));
+        err = ticket + 2;
+        maxbits = reinterpret_cast<unsigned *>(ticket + 8);
         pk0a = pk_bytes ? take(pk_bytes) : nullptr;
         pk0b = pk_bytes ? take(pk_bytes) : nullptr;
         pk1a = pk_bytes ? take(pk_bytes) : nullptr;
@@ -688,22 +666,6 @@ int chol_mixed_run(Handle *h, hipStream_t s, char prec, int64_t n, float *W, flo
     return chol_mixed_la<TIN>(h, s, n, W, n, Linv32, Linv, h->mixed_block, p0, p1);
 }
 
-// Solve structures of the factor in ws.W: tile inverses, diagonal-block
-// inverses, and the same for the reversed Lr = J Lᵀ J (backward solve).
-template <typename T>
-int prepare_solves(hipStream_t s, int64_t n, MixedWS<T> &ws)
-{
-    GLA_TRY(tile_inverses<T>(s, n, ws.W, n, ws.Linv));
-    GLA_TRY(diag_block_inverses<T>(s, n, ws.W, n, ws.Linv, ws.Dt));
-    GLA_TRY(diag_sub<T>(s, n, ws.W, n, ws.Dt, ws.Mt));
-    hipLaunchKernelGGL((reverse_transpose_lower<T>), g2(n, n), dim3(256), 0, s, n, ws.W, n, ws.Lr,
-                       n);
-    GLA_LAUNCH_CHECK();
-    GLA_TRY(tile_inverses<T>(s, n, ws.Lr, n, ws.Linvr));
-    GLA_TRY(diag_block_inverses<T>(s, n, ws.Lr, n, ws.Linvr, ws.Dtr));
-    return diag_sub<T>(s, n, ws.Lr, n, ws.Dtr, ws.Mtr);
-}
-
 // Refinement outcome.
 enum { kConverged = 0, kMaxIter = 1, kStalled = 2 };
 
@@ -712,7 +674,7 @@ enum { kConverged = 0, kMaxIter = 1, kStalled = 2 };
 template <typename T>
 int refine(Handle *h, hipStream_t s, int64_t n, const double *A, int64_t lda, int64_t nrhs,
            const double *B, int64_t ldb, double *X, int64_t ldx, MixedWS<T> &ws, double anorm,
-           double tol, int max_iter, int &epoch, int *iters, double *berr, int *outcome)
+           double tol, int max_iter, int *iters, double *berr, int *outcome)
 {
     const int64_t nch = ws.nchunk;
     std::vector<double> hn((size_t)32 * nch), bb((size_t)nrhs), rr((size_t)nrhs), xx((size_t)nrhs);
@@ -761,15 +723,37 @@ int refine(Handle *h, hipStream_t s, int64_t n, const double *A, int64_t lda, in
             prev2 = prev1;
             prev1 = eta;
         }
-        // x += (L Lᵀ)⁻¹ r: forward solve, then the backward one as a lower
-        // solve with Lr on reversed rows, adding into X
-        for (int64_t c = 0; c < nch; ++c) {
-            const int nr = (int)std::min<int64_t>(16, nrhs - 16 * c);
-            GLA_TRY(trsv16<T>(h, s, n, ws.W, n, ws.Dt, ws.Mt, ws.Rt + c * ws.npad * 16, ws.Yt, 0,
-                              nullptr, 0, nr, ws.flags, ++epoch, ws.err));
-            GLA_TRY(trsv16<T>(h, s, n, ws.Lr, n, ws.Dtr, ws.Mtr, ws.Yt, ws.Zt, 1, X + 16 * c * ldx,
-                              ldx, nr, ws.flags, ++epoch, ws.err));
-        }
+        // x += (L Lᵀ)⁻¹ r: L y = r, then Lᵀ z = y with rows and columns from
+        // the last, added into X; the chunks of 16 columns side by side
+        const size_t ye = tri_solve_elems(n, nrhs);
+        GLA_TRY(tri_solve_prepare<T>(s, (int64_t)(2 * ye), ws.Yt, ws.ticket, 2));
+        TriSolve<T> p{};
+        p.n = n;
+        p.nrhs = (int)nrhs;
+        p.spin_limit = h->spin_limit;
+        p.err = ws.err;
+        p.M = ws.W;
+        p.si = 1;
+        p.sj = n;
+        p.R = ws.Rt;
+        p.ri = 16;
+        p.rk = 1;
+        p.rp = ws.npad * 16;
+        p.Y = ws.Yt;
+        p.ticket = ws.ticket;
+        GLA_TRY(tri_solve<T>(s, p));
+        const int64_t l = n - 1;
+        p.M = ws.W + l * (n + 1);
+        p.si = -n;
+        p.sj = -1;
+        p.R = ws.Yt + l * 16;
+        p.ri = -16;
+        p.Y = ws.Yt + ye;
+        p.X = X + l;
+        p.oi = -1;
+        p.ok = ldx;
+        p.ticket = ws.ticket + 1;
+        GLA_TRY(tri_solve<T>(s, p));
     }
     *iters = corr;
     *berr = eta;
@@ -793,8 +777,7 @@ int mixed_attempt(Handle *h, hipStream_t s, char prec, int64_t n, const double *
 {
     MixedWS<T> ws;
     ws.carve(h->ws, n, nrhs, pk_bytes_of(prec, n, h->mixed_block));
-    hipLaunchKernelGGL(fill_int, dim3((unsigned)cdiv(ws.nblk + 1, 256)), dim3(256), 0, s,
-                       ws.nblk + 1, ws.flags, 0);
+    hipLaunchKernelGGL(k_set_int, dim3(1), dim3(1), 0, s, ws.err, 0);
     GLA_LAUNCH_CHECK();
     hipLaunchKernelGGL(k_set_int, dim3(1), dim3(1), 0, s, h->dinfo, 0);
     GLA_LAUNCH_CHECK();
@@ -826,10 +809,8 @@ int mixed_attempt(Handle *h, hipStream_t s, char prec, int64_t n, const double *
         *outcome = kStalled;
         return GLA_OK;
     }
-    GLA_TRY(prepare_solves<T>(s, n, ws));
-    int epoch = 0;
-    return refine<T>(h, s, n, A, lda, nrhs, B, ldb, X, ldx, ws, anorm, tol, max_iter, epoch, iters,
-                     berr, outcome);
+    return refine<T>(h, s, n, A, lda, nrhs, B, ldb, X, ldx, ws, anorm, tol, max_iter, iters, berr,
+                     outcome);
 }
 
 int mixed_solve(Handle *h, hipStream_t s, char prec, int64_t n, const double *A, int64_t lda,

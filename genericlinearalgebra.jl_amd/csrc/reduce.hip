@@ -413,29 +413,6 @@ constexpr int kTRRows = 8;           // rows per workgroup
 constexpr int kTRMax = 2048;         // largest order: 256 workgroups of 512 threads
 
 template <typename T>
-struct NaNMark;
-template <>
-struct NaNMark<double> {
-    typedef unsigned long long bits;
-    static constexpr bits value = 0xFFF4C0DEC0DEC0DEull;
-};
-template <>
-struct NaNMark<float> {
-    typedef unsigned bits;
-    static constexpr bits value = 0xFFA5C0DEu;
-};
-template <typename T>
-__device__ __forceinline__ bool is_mark(T v)
-{
-    return __builtin_bit_cast(typename NaNMark<T>::bits, v) == NaNMark<T>::value;
-}
-
-// v with a signalling NaN made quiet: an element that happens to have the
-// mark's bits is no mark.
-__device__ __forceinline__ double quiet(double v) { return __builtin_canonicalize(v); }
-__device__ __forceinline__ float quiet(float v) { return __builtin_canonicalizef(v); }
-
-template <typename T>
 __global__ void mark_kernel(int64_t cnt, T *p)
 {
     const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;

@@ -6,10 +6,11 @@
 // src/qr.jl:86-146); these are the solves a caller applies to their
 // results.
 //
-// Device plan.  The triangular solves run as right-side solves on the
-// transposed right-hand sides (rows of length n, one per right-hand side)
-// with the Cholesky driver's B <- B L⁻ᵀ (16×16 tile inverses, MFMA GEMMs
-// between 128-wide leaves):
+// Device plan.  Up to kFewRhs right-hand sides: one launch per triangle
+// (tri_solve), which reads the factor where it lies.  More: right-side solves
+// on the transposed right-hand sides (rows of length n, one per right-hand
+// side) with the Cholesky driver's B <- B L⁻ᵀ (16×16 tile inverses, MFMA
+// GEMMs between 128-wide leaves):
 //   L y = b           ⇔  yᵀ = bᵀ L⁻ᵀ;
 //   Lᵀ x = y          ⇔  xᵀ = yᵀ L⁻¹ = ((yᵀ J) Lr⁻ᵀ) J,  Lr = J Lᵀ J lower;
 //   R x = y (R upper) ⇔  xᵀ = yᵀ R⁻ᵀ = ((yᵀ J) Kr⁻ᵀ) J,  Kr = J R J lower,
@@ -170,20 +171,79 @@ int reversed_tail(hipStream_t s, int64_t n, int64_t nrhs, const T *M, int64_t ld
 
 }  // namespace
 
-// Scratch elements of the Cholesky solve: Uᵀ (uplo 'U'), Lr, two tile-inverse
-// sets, two nrhs×n row blocks.
+// Up to here one tri_solve launch per triangle, which reads the factor where
+// it lies; beyond, the GEMM form, whose tiles of L serve more columns at a
+// time.  Two solves with a Cholesky factor, GEMM form -> tri_solve, µs: FP64
+// n = 5001 3507 -> 473 (16 right-hand sides) and 4243 -> 1088 (512), 4096
+// 3621 -> 2736 (2000) but 7359 -> 10435 (8192), 1000 541 -> 106 (16),
+// 646 -> 153 (1000) and 1745 -> 1930 (20000); FP32 5001 2768 -> 312 (16),
+// 4096 4645 -> 3945 (8192).
+constexpr int64_t kFewRhs = 2048;
+
+// L Lᵀ X = B or L D Lᵀ X = B, L the lower triangle of F or the transposed
+// upper one (unit: its diagonal is taken as 1 and F's is D).
+template <typename T>
+int few_rhs_solve(const Handle *h, hipStream_t s, char uplo, int unit, int64_t n, int64_t nrhs,
+                  const T *F, int64_t ldf, T *B, int64_t ldb, T *scratch)
+{
+    const size_t ye = tri_solve_elems(n, nrhs);
+    int *ticket = reinterpret_cast<int *>(scratch + 2 * ye);
+    GLA_TRY(tri_solve_prepare<T>(s, (int64_t)(2 * ye), scratch, ticket, 2));
+    TriSolve<T> p{};
+    p.n = n;
+    p.unit = unit;
+    p.nrhs = (int)nrhs;
+    p.spin_limit = h->spin_limit;
+    // L y = b
+    p.M = F;
+    p.si = uplo == 'U' ? ldf : 1;
+    p.sj = uplo == 'U' ? 1 : ldf;
+    p.R = B;
+    p.ri = 1;
+    p.rk = ldb;
+    p.rp = 16 * ldb;
+    p.Y = scratch;
+    p.ticket = ticket;
+    GLA_TRY(tri_solve<T>(s, p));
+    // Lᵀ x = y (D⁻¹ y), rows and columns from the last
+    const int64_t l = n - 1;
+    p.M = F + l * (ldf + 1);
+    const int64_t t = p.si;
+    p.si = -p.sj;
+    p.sj = -t;
+    p.R = scratch + l * 16;
+    p.ri = -16;
+    p.rk = 1;
+    p.rp = (int64_t)(ye / cdiv(nrhs, 16));
+    if (unit) {
+        p.div = F + l * (ldf + 1);
+        p.ds = -(ldf + 1);
+    }
+    p.Y = scratch + ye;
+    p.out = B + l;
+    p.oi = -1;
+    p.ok = ldb;
+    p.ticket = ticket + 1;
+    return tri_solve<T>(s, p);
+}
+
+// Scratch elements of the Cholesky solve: two exchanges and their tickets, or
+// Uᵀ (uplo 'U'), Lr, two tile-inverse sets, two nrhs×n row blocks.
 size_t chol_solve_scratch(int64_t n, int64_t nrhs)
 {
+    if (nrhs <= kFewRhs) return 2 * tri_solve_elems(n, nrhs) + 64;
     return 2 * (size_t)n * n + 2 * tile_inverse_elems(n) + 2 * (size_t)nrhs * n + 256;
 }
 
 // B (n×nrhs) <- A⁻¹ B with A = L Lᵀ (uplo 'L', L lower) or A = Uᵀ U
 // (uplo 'U', U upper); the other triangle of F is not read.
 template <typename T>
-int chol_solve_dev(hipStream_t s, char uplo, int64_t n, int64_t nrhs, const T *F, int64_t ldf,
+int chol_solve_dev(const Handle *h, hipStream_t s, char uplo, int64_t n, int64_t nrhs, const T *F, int64_t ldf,
                    T *B, int64_t ldb, T *scratch)
 {
     if (n <= 0 || nrhs <= 0) return GLA_OK;
+    if (nrhs <= kFewRhs)
+        return few_rhs_solve<T>(h, s, uplo, 0, n, nrhs, F, ldf, B, ldb, scratch);
     const size_t nn = (size_t)n * n, ti = tile_inverse_elems(n);
     T *Lx = scratch, *Lr = Lx + nn, *Li = Lr + nn, *Lri = Li + ti, *Y = Lri + ti,
       *Z = Y + (size_t)nrhs * n;
@@ -212,10 +272,12 @@ int chol_solve_dev(hipStream_t s, char uplo, int64_t n, int64_t nrhs, const T *F
 // strict lower triangle, D on the diagonal; 'U': L = Uᵀ) — ldiv!(F::LDLt, X),
 // src/ldlt.jl:225-228.  Same scratch as the Cholesky solve.
 template <typename T>
-int ldlt_solve_dev(hipStream_t s, char uplo, int64_t n, int64_t nrhs, const T *F, int64_t ldf,
+int ldlt_solve_dev(const Handle *h, hipStream_t s, char uplo, int64_t n, int64_t nrhs, const T *F, int64_t ldf,
                    T *B, int64_t ldb, T *scratch)
 {
     if (n <= 0 || nrhs <= 0) return GLA_OK;
+    if (nrhs <= kFewRhs)
+        return few_rhs_solve<T>(h, s, uplo, 1, n, nrhs, F, ldf, B, ldb, scratch);
     const size_t nn = (size_t)n * n, ti = tile_inverse_elems(n);
     T *Lx = scratch, *Lr = Lx + nn, *Li = Lr + nn, *Lri = Li + ti, *Y = Lri + ti,
       *Z = Y + (size_t)nrhs * n;
@@ -263,7 +325,7 @@ int ldlt_lmul_dev(hipStream_t s, char uplo, int64_t n, int64_t nrhs, const T *F,
 size_t qr_solve_scratch(int64_t m, int64_t n, int64_t nrhs)
 {
     return (size_t)m * n + (size_t)n * n + tile_inverse_elems(n) + 3 * (size_t)nrhs * n +
-           8 * (size_t)nrhs * n + 256;
+           8 * (size_t)nrhs * n + (nrhs <= kFewRhs ? 2 * tri_solve_elems(n, nrhs) : 0) + 256;
 }
 
 // Least squares for m ≥ n: B (m×nrhs) <- Qᵀ B, then B[0:n] <- R⁻¹ B[0:n],
@@ -274,7 +336,7 @@ size_t qr_solve_scratch(int64_t m, int64_t n, int64_t nrhs)
 // unit lower L = I + stril(VᵀV) D: a solve with nrhs rows instead of T's
 // explicit inverse (1501×700: 1.0 ms of 128-wide inverses).
 template <typename T>
-int qr_solve_dev(hipStream_t s, int64_t m, int64_t n, int64_t nrhs, const T *F, int64_t ldf,
+int qr_solve_dev(const Handle *h, hipStream_t s, int64_t m, int64_t n, int64_t nrhs, const T *F, int64_t ldf,
                  const T *tau, T *B, int64_t ldb, int *info, T *scratch)
 {
     if (n <= 0 || nrhs <= 0) return GLA_OK;
@@ -292,6 +354,49 @@ int qr_solve_dev(hipStream_t s, int64_t m, int64_t n, int64_t nrhs, const T *F, 
     GLA_LAUNCH_CHECK();
     // W = VᵀB, Z = (L⁻¹ W)ᵀ, W2 = D Zᵀ, B -= V W2
     GLA_TRY(gemm<T>(s, 'T', 'N', 0, n, nrhs, m, T(1), Vw, m, B, ldb, T(0), W, n, 0, split, 8 * nr));
+    if (nrhs <= kFewRhs) {
+        const size_t ye = tri_solve_elems(n, nrhs);
+        T *Y = split + 8 * nr;
+        int *ticket = reinterpret_cast<int *>(Y + 2 * ye);
+        GLA_TRY(tri_solve_prepare<T>(s, (int64_t)(2 * ye), Y, ticket, 2));
+        TriSolve<T> p{};
+        p.n = n;
+        p.nrhs = (int)nrhs;
+        p.spin_limit = h->spin_limit;
+        p.unit = 1;                       // W2 = D L⁻¹ W
+        p.M = G;
+        p.si = 1;
+        p.sj = n;
+        p.R = W;
+        p.ri = 1;
+        p.rk = n;
+        p.rp = 16 * n;
+        p.Y = Y;
+        p.out = W2;
+        p.oi = 1;
+        p.ok = n;
+        p.mul = tau;
+        p.ms = 1;
+        p.ticket = ticket;
+        GLA_TRY(tri_solve<T>(s, p));
+        GLA_TRY(gemm<T>(s, 'N', 'N', 0, m, nrhs, n, T(-1), Vw, m, W2, n, T(1), B, ldb));
+        const int64_t l = n - 1;          // R x = y, rows and columns from the last
+        p.unit = 0;
+        p.M = F + l * (ldf + 1);
+        p.si = -1;
+        p.sj = -ldf;
+        p.R = B + l;
+        p.ri = -1;
+        p.rk = ldb;
+        p.rp = 16 * ldb;
+        p.Y = Y + ye;
+        p.out = B + l;
+        p.oi = -1;
+        p.ok = ldb;
+        p.mul = nullptr;
+        p.ticket = ticket + 1;
+        return tri_solve<T>(s, p);
+    }
     hipLaunchKernelGGL((to_rows_k<T>), g2(n, nrhs), dim3(256), 0, s, n, nrhs, W, n, Z, 0);
     GLA_LAUNCH_CHECK();
     GLA_TRY(tile_inverses<T>(s, n, G, n, Gi));
@@ -329,7 +434,7 @@ int chol_solve_entry(gla_handle_t hh, char uplo, int64_t n, int64_t nrhs, const 
     if (n == 0 || nrhs == 0) return GLA_OK;
     GLA_HIP_TRY(hipSetDevice(h->device));
     GLA_TRY(gla::ensure_workspace(h, gla::chol_solve_scratch(n, nrhs) * sizeof(T)));
-    return gla::chol_solve_dev<T>(reinterpret_cast<hipStream_t>(stream), uplo, n, nrhs, F, ldf, B,
+    return gla::chol_solve_dev<T>(h, reinterpret_cast<hipStream_t>(stream), uplo, n, nrhs, F, ldf, B,
                                   ldb, reinterpret_cast<T *>(h->ws));
 }
 
@@ -352,7 +457,7 @@ int ldlt_apply_entry(gla_handle_t hh, int mode, char uplo, int64_t n, int64_t nr
                                   : (size_t)n * n + (size_t)n * nrhs + 64;
     GLA_TRY(gla::ensure_workspace(h, need * sizeof(T)));
     T *ws = reinterpret_cast<T *>(h->ws);
-    if (mode == 0) return gla::ldlt_solve_dev<T>(s, uplo, n, nrhs, F, ldf, B, ldb, ws);
+    if (mode == 0) return gla::ldlt_solve_dev<T>(h, s, uplo, n, nrhs, F, ldf, B, ldb, ws);
     return gla::ldlt_lmul_dev<T>(s, uplo, n, nrhs, F, ldf, B, ldb, ws);
 }
 
@@ -373,7 +478,7 @@ int qr_solve_entry(gla_handle_t hh, int64_t m, int64_t n, int64_t nrhs, const T 
     GLA_HIP_TRY(hipSetDevice(h->device));
     hipStream_t s = reinterpret_cast<hipStream_t>(stream);
     GLA_TRY(gla::ensure_workspace(h, gla::qr_solve_scratch(m, n, nrhs) * sizeof(T)));
-    GLA_TRY(gla::qr_solve_dev<T>(s, m, n, nrhs, F, ldf, tau, B, ldb, h->dinfo + 8,
+    GLA_TRY(gla::qr_solve_dev<T>(h, s, m, n, nrhs, F, ldf, tau, B, ldb, h->dinfo + 8,
                                  reinterpret_cast<T *>(h->ws)));
     if (info) {
         int hv = 0;
