@@ -220,12 +220,12 @@ __device__ __forceinline__ void store_tile(int nb, TS *__restrict__ A, int64_t l
 // per tile) and every barrier waited for the stores of the tile inverse.
 // TS: storage type of A (T, or FP32 for the mixed-precision driver, which
 // factors its FP32 diagonal tiles in FP64); Linv32: optional FP32 copy of
-// the tile inverses.
+// the tile inverses.  L is stored in D, which may be A.
 constexpr int kFactorX = 2 * (kPanelNB / 16) * 256;   // LDS elements: Xb,
 constexpr int kFactorLi = 2 * 16 * kXLD;              // Lib (Db: one tile, 256)
 template <typename T, int W, typename TS = T>
-__device__ __forceinline__ void factor_body(int nb, TS *__restrict__ A, int64_t lda, int *info,
-                                             int64_t info_base, T *__restrict__ LinvG, T *Xb,
+__device__ __forceinline__ void factor_body(int nb, const TS *A, int64_t lda, TS *D, int64_t ldd,
+                                             int *info, int64_t info_base, T *__restrict__ LinvG, T *Xb,
                                              T *Db, T *Lib, float *__restrict__ Linv32 = nullptr)
 {
     typedef PanelMfma<T> M;
@@ -255,7 +255,7 @@ __device__ __forceinline__ void factor_body(int nb, TS *__restrict__ A, int64_t 
                 if (LinvG) LinvG[kb * 256 + lc * 16 + lg + 4 * t] = w[t];
                 if (Linv32) Linv32[kb * 256 + lc * 16 + lg + 4 * t] = float(w[t]);
             }
-            store_tile<T, TS>(nb, A, lda, kb, kb, d);
+            store_tile<T, TS>(nb, D, ldd, kb, kb, d);
             lds_barrier();                                            // end of (A)
         }
     } else {
@@ -320,7 +320,7 @@ __device__ __forceinline__ void factor_body(int nb, TS *__restrict__ A, int64_t 
 #pragma unroll
                     for (int kq = 0; kq < 4; ++kq) dg[d] = M::mma(-acc[q][kq], acc[q][kq], dg[d]);
                 }
-                store_tile<T, TS>(nb, A, lda, bi, kb, acc[q]);
+                store_tile<T, TS>(nb, D, ldd, bi, kb, acc[q]);
             }
             lds_barrier();                                            // end of (B)
         }
@@ -341,10 +341,10 @@ __global__ __launch_bounds__(kPanelThreads) void chol_factor_kernel(int nb, T *_
     __shared__ T Db[256];
     __shared__ T Lib[kFactorLi];
     switch (threadIdx.x >> 6) {
-    case 0: factor_body<T, 0>(nb, A, lda, info, info_base, LinvG, Xb, Db, Lib); break;
-    case 1: factor_body<T, 1>(nb, A, lda, info, info_base, LinvG, Xb, Db, Lib); break;
-    case 2: factor_body<T, 2>(nb, A, lda, info, info_base, LinvG, Xb, Db, Lib); break;
-    default: factor_body<T, 3>(nb, A, lda, info, info_base, LinvG, Xb, Db, Lib); break;
+    case 0: factor_body<T, 0>(nb, A, lda, A, lda, info, info_base, LinvG, Xb, Db, Lib); break;
+    case 1: factor_body<T, 1>(nb, A, lda, A, lda, info, info_base, LinvG, Xb, Db, Lib); break;
+    case 2: factor_body<T, 2>(nb, A, lda, A, lda, info, info_base, LinvG, Xb, Db, Lib); break;
+    default: factor_body<T, 3>(nb, A, lda, A, lda, info, info_base, LinvG, Xb, Db, Lib); break;
     }
 }
 
@@ -623,10 +623,10 @@ __global__ __launch_bounds__(kPanelThreads) void chol_factor_near_identity_kerne
         return;
     }
     switch (threadIdx.x >> 6) {
-    case 0: factor_body<T, 0>(nb, A, lda, info, info_base, LinvG, Xb, Db, Lib); break;
-    case 1: factor_body<T, 1>(nb, A, lda, info, info_base, LinvG, Xb, Db, Lib); break;
-    case 2: factor_body<T, 2>(nb, A, lda, info, info_base, LinvG, Xb, Db, Lib); break;
-    default: factor_body<T, 3>(nb, A, lda, info, info_base, LinvG, Xb, Db, Lib); break;
+    case 0: factor_body<T, 0>(nb, A, lda, A, lda, info, info_base, LinvG, Xb, Db, Lib); break;
+    case 1: factor_body<T, 1>(nb, A, lda, A, lda, info, info_base, LinvG, Xb, Db, Lib); break;
+    case 2: factor_body<T, 2>(nb, A, lda, A, lda, info, info_base, LinvG, Xb, Db, Lib); break;
+    default: factor_body<T, 3>(nb, A, lda, A, lda, info, info_base, LinvG, Xb, Db, Lib); break;
     }
 }
 
@@ -643,35 +643,32 @@ __global__ __launch_bounds__(kPanelThreads) void chol_factor_f32io_kernel(int nb
     __shared__ double Db[256];
     __shared__ double Lib[kFactorLi];
     switch (threadIdx.x >> 6) {
-    case 0: factor_body<double, 0, float>(nb, A, lda, info, info_base, nullptr, Xb, Db, Lib, Linv32); break;
-    case 1: factor_body<double, 1, float>(nb, A, lda, info, info_base, nullptr, Xb, Db, Lib, Linv32); break;
-    case 2: factor_body<double, 2, float>(nb, A, lda, info, info_base, nullptr, Xb, Db, Lib, Linv32); break;
-    default: factor_body<double, 3, float>(nb, A, lda, info, info_base, nullptr, Xb, Db, Lib, Linv32); break;
+    case 0: factor_body<double, 0, float>(nb, A, lda, A, lda, info, info_base, nullptr, Xb, Db, Lib, Linv32); break;
+    case 1: factor_body<double, 1, float>(nb, A, lda, A, lda, info, info_base, nullptr, Xb, Db, Lib, Linv32); break;
+    case 2: factor_body<double, 2, float>(nb, A, lda, A, lda, info, info_base, nullptr, Xb, Db, Lib, Linv32); break;
+    default: factor_body<double, 3, float>(nb, A, lda, A, lda, info, info_base, nullptr, Xb, Db, Lib, Linv32); break;
     }
 }
 
 // A strided batch of diagonal-block factorisations (nb ≤ 128 each), one
-// workgroup per matrix: matrix b at A + b·sA, tile inverses at LinvG + b·sLinv,
+// workgroup per matrix: matrix b at A + b·sA, its factor at D + b·sD,
 // its first failing pivot in info[b] (info zeroed by the caller).
 template <typename T>
-__global__ __launch_bounds__(kPanelThreads) void chol_factor_batched_kernel(int nb, T *A,
-                                                                            int64_t lda,
-                                                                            int64_t sA, int *info,
-                                                                            T *LinvG,
-                                                                            int64_t sLinv)
+__global__ __launch_bounds__(kPanelThreads) void chol_factor_batched_kernel(
+    int nb, const T *A, int64_t lda, int64_t sA, T *D, int64_t ldd, int64_t sD, int *info)
 {
     __shared__ T Xb[kFactorX];
     __shared__ T Db[256];
     __shared__ T Lib[kFactorLi];
     const int64_t b = blockIdx.x;
-    T *Ab = A + b * sA;
-    T *Lg = LinvG + b * sLinv;
+    const T *Ab = A + b * sA;
+    T *Lb = D + b * sD;
     int *ib = info + b;
     switch (threadIdx.x >> 6) {
-    case 0: factor_body<T, 0>(nb, Ab, lda, ib, 0, Lg, Xb, Db, Lib); break;
-    case 1: factor_body<T, 1>(nb, Ab, lda, ib, 0, Lg, Xb, Db, Lib); break;
-    case 2: factor_body<T, 2>(nb, Ab, lda, ib, 0, Lg, Xb, Db, Lib); break;
-    default: factor_body<T, 3>(nb, Ab, lda, ib, 0, Lg, Xb, Db, Lib); break;
+    case 0: factor_body<T, 0>(nb, Ab, lda, Lb, ldd, ib, 0, nullptr, Xb, Db, Lib); break;
+    case 1: factor_body<T, 1>(nb, Ab, lda, Lb, ldd, ib, 0, nullptr, Xb, Db, Lib); break;
+    case 2: factor_body<T, 2>(nb, Ab, lda, Lb, ldd, ib, 0, nullptr, Xb, Db, Lib); break;
+    default: factor_body<T, 3>(nb, Ab, lda, Lb, ldd, ib, 0, nullptr, Xb, Db, Lib); break;
     }
 }
 
@@ -679,11 +676,8 @@ __global__ __launch_bounds__(kPanelThreads) void chol_factor_batched_kernel(int 
 // padded with the identity); one wave per tile.
 template <typename T>
 __global__ __launch_bounds__(256) void tile_inverse_kernel(int64_t n, const T *__restrict__ L,
-                                                           int64_t ldl, T *__restrict__ LinvG,
-                                                           int64_t sL = 0, int64_t sLinv = 0)
+                                                           int64_t ldl, T *__restrict__ LinvG)
 {
-    L += blockIdx.y * sL;          // strided batch along grid y
-    LinvG += blockIdx.y * sLinv;
     const int64_t tile = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
     if (tile * 16 >= n) return;
     const int lane = threadIdx.x & 63;
@@ -817,13 +811,8 @@ __global__ __launch_bounds__(kPanelThreads) void chol_solve_kernel(int nb, const
                                                                    int64_t ldl,
                                                                    const T *__restrict__ LinvG,
                                                                    T *__restrict__ B, int64_t ldb,
-                                                                   int64_t nrows, int64_t sL,
-                                                                   int64_t sLinv, int64_t sB)
+                                                                   int64_t nrows)
 {
-    // batched form: blockIdx.y selects (L, LinvG, B) at the given strides
-    L += blockIdx.y * sL;
-    LinvG += blockIdx.y * sLinv;
-    B += blockIdx.y * sB;
     typedef PanelMfma<T> M;
     typedef typename M::acc_t acc_t;
     constexpr int NBLK = kPanelNB / 16;             // 8
@@ -1003,7 +992,7 @@ int launch_solve(hipStream_t s, int nb, const T *L, int64_t ldl, const T *LinvG,
 {
     if (nrows <= 0 || nb <= 0) return GLA_OK;
     hipLaunchKernelGGL((chol_solve_kernel<T>), dim3((unsigned)cdiv(nrows, kPanelRB)),
-                       dim3(kPanelThreads), 0, s, nb, L, ldl, LinvG, B, ldb, nrows, 0, 0, 0);
+                       dim3(kPanelThreads), 0, s, nb, L, ldl, LinvG, B, ldb, nrows);
     GLA_LAUNCH_CHECK();
     return GLA_OK;
 }
@@ -1015,19 +1004,6 @@ int launch_psolve(hipStream_t s, int nb, const T *L, int64_t ldl, const T *LinvG
     if (nrows <= 0) return GLA_OK;
     hipLaunchKernelGGL((chol_psolve_kernel<T>), dim3((unsigned)cdiv(nrows, kPanelRB)),
                        dim3(kPanelThreads), 0, s, nb, L, ldl, LinvG, B, ldb, nrows);
-    GLA_LAUNCH_CHECK();
-    return GLA_OK;
-}
-
-// `batch` independent solves at strides sL, sLinv, sB (one grid row each).
-template <typename T>
-int launch_solve_batched(hipStream_t s, int nb, const T *L, int64_t ldl, int64_t sL,
-                         const T *LinvG, int64_t sLinv, T *B, int64_t ldb, int64_t sB,
-                         int64_t nrows, int64_t batch)
-{
-    if (nrows <= 0 || batch <= 0 || nb <= 0) return GLA_OK;
-    hipLaunchKernelGGL((chol_solve_kernel<T>), dim3((unsigned)cdiv(nrows, kPanelRB), (unsigned)batch),
-                       dim3(kPanelThreads), 0, s, nb, L, ldl, LinvG, B, ldb, nrows, sL, sLinv, sB);
     GLA_LAUNCH_CHECK();
     return GLA_OK;
 }
@@ -1287,34 +1263,14 @@ int trsm_rlt(hipStream_t s, int64_t m, int64_t n, const T *L, int64_t ldl, const
     return trsm_rlt_dev<T>(s, m, n, L, ldl, Linv, B, ldb);
 }
 template <typename T>
-int chol_factor_batched(hipStream_t s, int nb, T *A, int64_t lda, int64_t sA, int *info, T *LinvG,
-                        int64_t sLinv, int64_t batch)
+int chol_factor_batched(hipStream_t s, int nb, const T *A, int64_t lda, int64_t sA, T *L,
+                        int64_t ldl, int64_t sL, int *info, int64_t batch)
 {
     if (batch <= 0 || nb <= 0) return GLA_OK;
     hipLaunchKernelGGL((chol_factor_batched_kernel<T>), dim3((unsigned)batch), dim3(kPanelThreads),
-                       0, s, nb, A, lda, sA, info, LinvG, sLinv);
+                       0, s, nb, A, lda, sA, L, ldl, sL, info);
     GLA_LAUNCH_CHECK();
     return GLA_OK;
-}
-template <typename T>
-int tile_inverses_batched(hipStream_t s, int64_t n, const T *L, int64_t ldl, int64_t sL, T *LinvG,
-                          int64_t sLinv, int64_t batch)
-{
-    if (n <= 0 || batch <= 0) return GLA_OK;
-    hipLaunchKernelGGL((tile_inverse_kernel<T>), dim3((unsigned)cdiv(cdiv(n, 16), 4), (unsigned)batch),
-                       dim3(256), 0, s, n, L, ldl, LinvG, sL, sLinv);
-    GLA_LAUNCH_CHECK();
-    return GLA_OK;
-}
-template <typename T>
-int trsm_rlt_batched(hipStream_t s, int64_t m, int n, const T *L, int64_t ldl, int64_t sL,
-                     const T *Linv, int64_t sLinv, T *B, int64_t ldb, int64_t sB, int64_t batch)
-{
-    if (n > kPanelNB) {
-        set_error("trsm_rlt_batched: n = %d exceeds %d", n, kPanelNB);
-        return GLA_ERR_UNSUPPORTED;
-    }
-    return launch_solve_batched<T>(s, n, L, ldl, sL, Linv, sLinv, B, ldb, sB, m, batch);
 }
 size_t tile_inverse_elems(int64_t n) { return linv_elems(n); }
 
@@ -1328,12 +1284,8 @@ size_t tile_inverse_elems(int64_t n) { return linv_elems(n); }
     template int tile_inverses<T>(hipStream_t, int64_t, const T *, int64_t, T *);            \
     template int trsm_rlt<T>(hipStream_t, int64_t, int64_t, const T *, int64_t, const T *,   \
                              T *, int64_t); \
-    template int chol_factor_batched<T>(hipStream_t, int, T *, int64_t, int64_t, int *, T *,  \
-                                        int64_t, int64_t);                                    \
-    template int tile_inverses_batched<T>(hipStream_t, int64_t, const T *, int64_t, int64_t,  \
-                                          T *, int64_t, int64_t);                             \
-    template int trsm_rlt_batched<T>(hipStream_t, int64_t, int, const T *, int64_t, int64_t,  \
-                                     const T *, int64_t, T *, int64_t, int64_t, int64_t);
+    template int chol_factor_batched<T>(hipStream_t, int, const T *, int64_t, int64_t, T *,   \
+                                        int64_t, int64_t, int *, int64_t);
 
 GLA_INST_BLOCKS(double)
 GLA_INST_BLOCKS(float)
