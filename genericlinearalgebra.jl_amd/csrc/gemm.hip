@@ -213,6 +213,53 @@ __device__ __forceinline__ bool tile_of(const P &p, int &tm, int &tn)
     return false;
 }
 
+// C's elements of a wave's MI×NJ grid of 16×16 blocks from (r0, c0).  The
+// products are formed transposed (operands swapped), so a block holds 16
+// consecutive rows of a column across its lanes — row lane % 16, column
+// lane / 16 + 4 r (FP64) or 4 (lane / 16) + r (FP32) for register r — and every
+// access is of whole lines.  A row of blocks of C is read at once, ahead of
+// its stores: an element at a time, each load waited for the store before it
+// (7168×2944 += 7168×128·128×2944 FP64: 204 -> 164 µs, FP32 124 -> 78).
+template <typename T, int MI, int NJ, int MODE>
+__device__ __forceinline__ void store_blocks(const typename Mfma<T>::acc_t (&acc)[MI][NJ], T *C,
+                                             int64_t ldc, int64_t M, int64_t N, int64_t diag_off,
+                                             int64_t r0, int64_t c0, T alpha, T beta)
+{
+    const int lane = threadIdx.x & 63;
+    const bool beta0 = beta == T(0);
+    const int64_t cl = c0 + (sizeof(T) == 8 ? lane >> 4 : 4 * (lane >> 4));
+    constexpr int CS = sizeof(T) == 8 ? 4 : 1;
+#pragma unroll
+    for (int i = 0; i < MI; ++i) {
+        const int64_t row = r0 + i * 16 + (lane & 15);
+        T *const cr = C + (row < M ? row : M - 1);
+        T old[NJ][4];
+        if (!beta0) {
+#pragma unroll
+            for (int j = 0; j < NJ; ++j)
+#pragma unroll
+                for (int r = 0; r < 4; ++r) {
+                    const int64_t col = cl + j * 16 + CS * r;
+                    old[j][r] = cr[(col < N ? col : N - 1) * ldc];
+                }
+        }
+#pragma unroll
+        for (int j = 0; j < NJ; ++j)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                const int64_t col = cl + j * 16 + CS * r;
+                bool ok = row < M && col < N;
+                if (MODE == 1) ok = ok && row + diag_off >= col;
+                if (MODE == 2) ok = ok && row + diag_off <= col;
+                if (ok) {
+                    T v = alpha * acc[i][j][r];
+                    if (!beta0) v += beta * old[j][r];
+                    cr[col * ldc] = v;
+                }
+            }
+    }
+}
+
 // NBUF = 1: one LDS buffer (half the LDS: kernels of the caller's stream
 // then fit beside two workgroups of this one on a CU) at the cost of a
 // second barrier per K-slab.
@@ -244,11 +291,6 @@ __global__ __launch_bounds__(kThreads, 2) void gemm_kernel(GemmP<T> p)
     const T *Ap = p.A + (TA ? koff : koff * p.lda);
     const T *Bp = p.B + (TB ? koff * p.ldb : koff);
 
-    // Accumulator element r of block (i,j) is C(row, col) with col = lane%16
-    // inside the 16×16 block and row = 4*(lane/16) + r for the f32
-    // instruction, row = lane/16 + 4*r for the f64 one (measured on gfx950:
-    // the f64 16x16x4 result interleaves its four row groups).
-    constexpr bool kF64Rows = sizeof(T) == 8;
     const bool split = p.ws != nullptr;
     // Accumulators start at zero; C is read in the epilogue.  (Starting them
     // at ±C instead stalls the first MFMA on the C loads: measured 15%
@@ -298,7 +340,7 @@ __global__ __launch_bounds__(kThreads, 2) void gemm_kernel(GemmP<T> p)
 #pragma unroll
             for (int i = 0; i < MI; ++i)
 #pragma unroll
-                for (int j = 0; j < NJ; ++j) acc[i][j] = Mfma<T>::mma(a[i], b[j], acc[i][j]);
+                for (int j = 0; j < NJ; ++j) acc[i][j] = Mfma<T>::mma(b[j], a[i], acc[i][j]);
         }
         if (more) {
             if (NBUF == 1) __syncthreads();   // every wave is done with the buffer
@@ -310,30 +352,9 @@ __global__ __launch_bounds__(kThreads, 2) void gemm_kernel(GemmP<T> p)
 
     // Epilogue.
     const T alpha = split ? T(1) : p.alpha, beta = split ? T(0) : p.beta;
-    const bool beta0 = beta == T(0);
-    T *const Cp = split ? p.ws + (int64_t)blockIdx.y * p.M * p.N : p.C;
-    const int64_t ldc = split ? p.M : p.ldc;
-#pragma unroll
-    for (int i = 0; i < MI; ++i)
-#pragma unroll
-        for (int j = 0; j < NJ; ++j) {
-            const int64_t row = m0 + wm * WM + i * 16 + (kF64Rows ? (lane >> 4) : 4 * (lane >> 4));
-            const int64_t col = n0 + wn * WN + j * 16 + (lane & 15);
-            if (col >= p.N) continue;
-#pragma unroll
-            for (int r = 0; r < 4; ++r) {
-                const int64_t gr = row + (kF64Rows ? 4 * r : r);
-                T *c = Cp + gr + col * ldc;
-                bool ok = gr < p.M;
-                if (MODE == 1) ok = ok && (gr + p.diag_off >= col);
-                if (MODE == 2) ok = ok && (gr + p.diag_off <= col);
-                if (ok) {
-                    T v = alpha * acc[i][j][r];
-                    if (!beta0) v += beta * *c;
-                    *c = v;
-                }
-            }
-        }
+    store_blocks<T, MI, NJ, MODE>(acc, split ? p.ws + (int64_t)blockIdx.y * p.M * p.N : p.C,
+                                  split ? p.M : p.ldc, p.M, p.N, p.diag_off, m0 + wm * WM,
+                                  n0 + wn * WN, alpha, beta);
 }
 
 // Direct-to-LDS variant for FP64 with MN-contiguous operands (op(A) = A
@@ -343,7 +364,10 @@ __global__ __launch_bounds__(kThreads, 2) void gemm_kernel(GemmP<T> p)
 // registers; the waves wait only for the slab they are about to use
 // (vmcnt), so NS − 1 slabs stay in flight behind the MFMAs.  Rows past M or
 // N load clamped (valid) addresses whose results are never written; K must
-// be a multiple of BKD.
+// be a multiple of BKD.  C an element at a time, rows in the registers: with
+// store_blocks this kernel by itself is 2% faster, but takes 24…48 registers
+// more and the Cholesky whose block columns it runs beside 7% longer
+// (n = 16384 27.5 -> 29.4 ms).
 template <int BKD, int NS, int MODE>
 __global__ __launch_bounds__(kThreads, (2 * NS * BKD * 132 * 8 <= 81920 ? 2 : 1)) void
 gemm_dl_kernel(GemmP<double> p)
@@ -542,14 +566,21 @@ int pick_tile(hipStream_t s, const GemmP<T> &p, size_t ws_elems)
     // 128×128 tiles when the problem yields enough of them to fill the
     // chip; 64×64 otherwise, split along K when even those are too few and
     // K is long (tall-skinny products such as Vᵀ A in the WY update).
+    // Updates with a short K (A − V W) also take 64×64: reading and writing C
+    // is then much of the work, and more and smaller tiles overlap it better
+    // (7168×2944, K = 128: FP64 164 -> 149 µs, FP32 78 -> 68; K = 256: 267 ->
+    // 254, 127 -> 115; at K = 4096 64×64 is 4–14% slower).
     int64_t big = cdiv(p.M, 128) * cdiv(p.N, 128);
     if (MODE != 0) big /= 2;
-    if (big >= 384) return launch<T, 128, 128, TA, TB, MODE, VEC>(s, p, 1);
+    const bool update = MODE == 0 && !TA && !TB && p.K <= 256;
+    if (big >= 384 && !update) return launch<T, 128, 128, TA, TB, MODE, VEC>(s, p, 1);
     int64_t small = cdiv(p.M, 64) * cdiv(p.N, 64);
     if (MODE != 0) small = (small + 1) / 2;
     int splits = 1;
     if (p.ws && small < 256 && p.K >= 1024) {
-        splits = (int)std::min<int64_t>(cdiv(p.K, 512), cdiv(512, small));
+        // four workgroups a CU: the loads of one slab take longer than its
+        // products (QR 8192×4096 12.55 -> 12.17 ms against two a CU; eight 12.17)
+        splits = (int)std::min<int64_t>(cdiv(p.K, 256), cdiv(1024, small));
         const int64_t mn = p.M * p.N;
         if (mn > 0) splits = (int)std::min<int64_t>(splits, (int64_t)(ws_elems / (size_t)mn));
     }
