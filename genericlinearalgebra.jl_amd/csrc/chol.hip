@@ -337,6 +337,7 @@ __global__ __launch_bounds__(kPanelThreads) void chol_factor_kernel(int nb, T *_
                                                                     int64_t info_base,
                                                                     T *__restrict__ LinvG)
 {
+    __builtin_amdgcn_s_setprio(3);
     __shared__ T Xb[kFactorX];
     __shared__ T Db[256];
     __shared__ T Lib[kFactorLi];
@@ -602,6 +603,7 @@ __global__ __launch_bounds__(kPanelThreads) void chol_factor_near_identity_kerne
     int nb, T *__restrict__ A, int64_t lda, int *info, int64_t info_base, T *__restrict__ LinvG,
     const int *flags)
 {
+    __builtin_amdgcn_s_setprio(3);
     __shared__ T Xb[kFactorX];
     __shared__ T Db[256];
     __shared__ T Lib[kFactorLi];
@@ -745,18 +747,21 @@ __device__ __forceinline__ void stage_l_tiles(int nb, const T *__restrict__ L, i
         const int kb = lt_kb(q), bj = lt_bj(q);
         const int gi = bj * 16 + ri, gj = kb * 16 + rj;
         const int gic = gi < nb ? gi : nb - 1, gjc = gj < nb ? gj : nb - 1;
-        const T v = L[gic + (int64_t)gjc * ldl];
-        lv[q] = (gi < nb && gj < nb) ? v : T(0);
+        lv[q] = L[gic + (int64_t)gjc * ldl];
     }
 #pragma unroll
-    for (int q = 0; q < NBLK; ++q) {
-        const T v = LinvG[(q < nkb ? q : nkb - 1) * 256 + threadIdx.x];
-        iv[q] = q < nkb ? v : T(0);
+    for (int q = 0; q < NBLK; ++q) iv[q] = LinvG[(q < nkb ? q : nkb - 1) * 256 + threadIdx.x];
+#pragma unroll
+    for (int q = 0; q < NLT; ++q) hold(lv[q]);
+#pragma unroll
+    for (int q = 0; q < NBLK; ++q) hold(iv[q]);
+#pragma unroll
+    for (int q = 0; q < NLT; ++q) {
+        const bool in = lt_bj(q) * 16 + ri < nb && lt_kb(q) * 16 + rj < nb;
+        Lt[q * TS + ri * kXLD + rj] = in ? lv[q] : T(0);
     }
 #pragma unroll
-    for (int q = 0; q < NLT; ++q) Lt[q * TS + ri * kXLD + rj] = lv[q];
-#pragma unroll
-    for (int q = 0; q < NBLK; ++q) Li[q * TS + i * kXLD + j] = iv[q];
+    for (int q = 0; q < NBLK; ++q) Li[q * TS + i * kXLD + j] = q < nkb ? iv[q] : T(0);
 }
 
 // acc (this wave's 16 rows × 128 columns as eight 16×16 tiles, each held
@@ -768,9 +773,9 @@ __device__ __forceinline__ void stage_l_tiles(int nb, const T *__restrict__ L, i
 // registers and only L read from LDS: no LDS round trip and no barrier
 // (every wave touches only its own rows).  The column-block loop is
 // unrolled, so every tile index is static.
-template <typename T>
-__device__ __forceinline__ void solve_tiles(int nkb, typename PanelMfma<T>::acc_t acc[8],
-                                            const T *Lt, const T *Li)
+template <typename T, bool FULL>
+__device__ __forceinline__ void solve_tiles_of(int nkb, typename PanelMfma<T>::acc_t acc[8],
+                                               const T *Lt, const T *Li)
 {
     typedef PanelMfma<T> M;
     typedef typename M::acc_t acc_t;
@@ -780,7 +785,7 @@ __device__ __forceinline__ void solve_tiles(int nkb, typename PanelMfma<T>::acc_
     const int lc = lane & 15;
 #pragma unroll
     for (int kb = 0; kb < NBLK; ++kb) {
-        if (kb >= nkb) break;
+        if (!FULL && kb >= nkb) break;
         const T *Lik = Li + kb * TS;
         acc_t x = {T(0), T(0), T(0), T(0)};
 #pragma unroll
@@ -792,7 +797,7 @@ __device__ __forceinline__ void solve_tiles(int nkb, typename PanelMfma<T>::acc_
         for (int kq = 0; kq < 4; ++kq) nx[kq] = -x[kq];
 #pragma unroll
         for (int bj = kb + 1; bj < NBLK; ++bj) {
-            if (bj >= nkb) break;
+            if (!FULL && bj >= nkb) break;
             const T *Lt_jk = Lt + lt_index(bj, kb) * TS;
 #pragma unroll
             for (int kq = 0; kq < 4; ++kq)
@@ -800,12 +805,25 @@ __device__ __forceinline__ void solve_tiles(int nkb, typename PanelMfma<T>::acc_
         }
     }
 }
+// (a full block without branches, so that L's reads run ahead of their use)
+template <typename T>
+__device__ __forceinline__ void solve_tiles(int nkb, typename PanelMfma<T>::acc_t acc[8],
+                                            const T *Lt, const T *Li)
+{
+    if (nkb == kPanelNB / 16)
+        solve_tiles_of<T, true>(nkb, acc, Lt, Li);
+    else
+        solve_tiles_of<T, false>(nkb, acc, Lt, Li);
+}
 
 // B (nrows×nb) <- B L⁻ᵀ for the lower nb×nb L (nb ≤ 128) whose 16×16
 // diagonal-tile inverses are in LinvG — rdiv!(A21, LowerTriangular(A11)'),
 // src/cholesky.jl:28,48.  Each workgroup takes 64 rows; wave w holds tile
 // row w of them (8 tiles).  L's 28 strictly-lower tiles and the 8 inverses
-// are read into LDS once, then solve_tiles runs the column sweep.
+// are read into LDS once, then solve_tiles runs the column sweep.  Bound by
+// the sweep, 36 tile products a wave (FP64 4 µs), between two memory round
+// trips: 1501×128 FP64 12 µs (22 with the loads under branches, one round trip
+// after another, and a branch per tile in the sweep).
 template <typename T>
 __global__ __launch_bounds__(kPanelThreads) void chol_solve_kernel(int nb, const T *__restrict__ L,
                                                                    int64_t ldl,
@@ -813,6 +831,7 @@ __global__ __launch_bounds__(kPanelThreads) void chol_solve_kernel(int nb, const
                                                                    T *__restrict__ B, int64_t ldb,
                                                                    int64_t nrows)
 {
+    __builtin_amdgcn_s_setprio(3);
     typedef PanelMfma<T> M;
     typedef typename M::acc_t acc_t;
     constexpr int NBLK = kPanelNB / 16;             // 8
@@ -837,10 +856,17 @@ __global__ __launch_bounds__(kPanelThreads) void chol_solve_kernel(int nb, const
         for (int r = 0; r < 4; ++r) {
             const int gj = bj * 16 + M::row(lane, r);
             const int gjc = gj < nb ? gj : nb - 1;
-            const T v = B[grc + (int64_t)gjc * ldb];
-            acc[bj][r] = (gr < nrows && gj < nb) ? v : T(0);
+            acc[bj][r] = B[grc + (int64_t)gjc * ldb];
         }
     stage_l_tiles<T>(nb, L, ldl, LinvG, Lt, Li);
+#pragma unroll
+    for (int bj = 0; bj < NBLK; ++bj)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            T v = acc[bj][r];
+            hold(v);
+            acc[bj][r] = (gr < nrows && bj * 16 + M::row(lane, r) < nb) ? v : T(0);
+        }
     __syncthreads();
     solve_tiles<T>(nkb, acc, Lt, Li);
 #pragma unroll

@@ -470,6 +470,15 @@ __device__ __forceinline__ void tile_factor(typename PanelMfma<T>::acc_t &a, T w
     for (int q = 0; q < 4; ++q) w[q] *= ysel;
 }
 
+// Holds a loaded value where it is.  A load from a clamped address whose value
+// a select then drops is otherwise turned into a load under a branch, and a
+// row of them into round trips one after another: load all, hold all, select.
+template <typename T>
+__device__ __forceinline__ void hold(T &v)
+{
+    asm volatile("" : "+v"(v));
+}
+
 // Barrier over the workgroup that orders LDS only: outstanding global
 // stores stay in flight (__syncthreads waits for them, about a memory round
 // trip per barrier).

@@ -30,6 +30,7 @@
 // split-K), W = Tᵀ W, A2 -= Vw W — the same three contractions the
 // reference makes, with V1 folded into Vw.
 #include <algorithm>
+#include <type_traits>
 
 #include "gla_coherent.hpp"
 #include "gla_internal.hpp"
@@ -866,6 +867,7 @@ __global__ __launch_bounds__(256) void hr_gram_kernel(int64_t m, int k, const T 
                                                       T *part, T *copy_to, int64_t ldc,
                                                       int *flag)
 {
+    __builtin_amdgcn_s_setprio(3);
     typedef PanelMfma<T> Mf;
     typedef typename Mf::acc_t acc_t;
     __shared__ T Xs[kGrRB * kGrLD];
@@ -932,6 +934,7 @@ template <typename T>
 __global__ __launch_bounds__(1024) void hr_gram_reduce_kernel(int k, int P, const T *part, T *G,
                                                               int *flag, int check)
 {
+    __builtin_amdgcn_s_setprio(3);
     __shared__ T red[4][256];
     __shared__ double wsum[4];
     const int t = threadIdx.x, e = t & 255, g = t >> 8;
@@ -972,6 +975,7 @@ __global__ __launch_bounds__(1024) void hr_gram_reduce_kernel(int k, int P, cons
 template <typename T>
 __global__ __launch_bounds__(256) void hr_r_kernel(int k, const T *L1, const T *L2, T *R)
 {
+    __builtin_amdgcn_s_setprio(3);
     const int bi = blockIdx.x, bj = blockIdx.y;
     if (bi > bj) return;
     __shared__ T A[128 * 17], B[128 * 17];   // A[l][ii] = L₂(l, i), B[l][jj] = L₁(j, l)
@@ -1005,7 +1009,7 @@ __device__ __forceinline__ T wave_bcast(T v, int src)
 }
 
 constexpr int kHrLD = 129;   // LDS leading dimension of the top block
-constexpr int kHrThreads = 256;
+constexpr int kHrThreads = 512;
 constexpr int kHrTL = 17;    // leading dimension of the 16×16 inverses in LDS
 
 __device__ __forceinline__ void hr_wave_order() { __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront"); }
@@ -1046,28 +1050,24 @@ struct HrLuRow<C, 16, T> {
 };
 template <int C, typename T>
 struct HrLuCols {
-    static __device__ __forceinline__ void run(T d[16], T dv[16], T uv[16], int r, int nbk)
+    static __device__ __forceinline__ void run(T d[16], int r)
     {
-        if (C < nbk) {
-            const T mjj = row_bcast<C>(d[C]);   // −q̂_CC
-            const T dj = dcopysign<T>(T(1), mjj);
-            const T uj = mjj + dj;              // |u_C| = 1 + |q̂_CC|
-            const T ru = recip1(uj);
-            // rows at or above the pivot take l = 0, which leaves them as
-            // they are (fma(−0, u, d) = d)
-            const bool below = r > C;
-            const T l = d[C] * ru;
-            HrLuRow<C, C + 1, T>::run(d, below ? l : T(0));
-            d[C] = below ? l : (r == C ? uj : d[C]);
-            dv[C] = dj;
-            uv[C] = uj;
-        }
-        HrLuCols<C + 1, T>::run(d, dv, uv, r, nbk);
+        const T mjj = row_bcast<C>(d[C]);   // −q̂_CC
+        const T dj = dcopysign<T>(T(1), mjj);
+        const T uj = mjj + dj;              // |u_C| = 1 + |q̂_CC|
+        const T ru = recip1(uj);
+        // rows at or above the pivot take l = 0, which leaves them as
+        // they are (fma(−0, u, d) = d)
+        const bool below = r > C;
+        const T l = d[C] * ru;
+        HrLuRow<C, C + 1, T>::run(d, below ? l : T(0));
+        d[C] = below ? l : (r == C ? uj : d[C]);
+        HrLuCols<C + 1, T>::run(d, r);
     }
 };
 template <typename T>
 struct HrLuCols<16, T> {
-    static __device__ __forceinline__ void run(T *, T *, T *, int, int) {}
+    static __device__ __forceinline__ void run(T *, int) {}
 };
 
 // Multipliers of the backward elimination for Z = U⁻¹ (rows of U in
@@ -1087,7 +1087,7 @@ struct HrUpMul<16, T> {
     static __device__ __forceinline__ void run(const T *, T, int, T *) {}
 };
 
-// Steps (2)-(3) on the top block: one workgroup of 4 waves, k ≤ 128, the
+// Steps (2)-(3) on the top block: one workgroup of 8 waves, k ≤ 128, the
 // block in LDS (M, column-major), blocked by 16 columns as a right-looking
 // LU without pivoting.  Per block J = jb..jb+15:
 //   wave 0 eliminates the 16×16 diagonal block column by column (lane r
@@ -1097,19 +1097,24 @@ struct HrUpMul<16, T> {
 //   from the rows still in its registers; then, on MFMA over 16×16 tiles:
 //   U_J,right = W_J M_J,right,
 //   L_below,J = M_below,J Z, and M_below,right −= L_below,J U_J,right.
-// Then T = Û V₁⁻ᵀ (Û = U S) in place over U, by column blocks:
-//   T[:, J] = Acc[:, J] W_Jᵀ, Acc[:, right] −= T[:, J] V₁[right, J]ᵀ
-// (T upper and V₁ strictly lower share M).  Writes V₁ (explicit: unit
+// Then T = Û V₁⁻ᵀ, Û = U S.  Writes V₁ (explicit: unit
 // diagonal, zero above) over Q's top block, Un = −Uᵀ (lower, ld k) and the
 // inverses of its 16×16 diagonal tiles (UnInv) for the solve of the rows
 // below, T (zero below the diagonal), S (Sv) and τ.
+// Bound by the serial chain of eight eliminations (2.9 µs each: 0.75 the
+// columns, the rest the two inverses and the hand-over) and four products.
+// 128×128 FP64 44 µs; 67 with four waves, the loads under branches (one round
+// trip after another, 5 µs), a branch per column, and T swept in LDS with two
+// barriers per 16 columns.
 template <typename T>
 __global__ __launch_bounds__(kHrThreads) void hr_lu_kernel(int k, T *Q, int64_t ldq,
                                                            const int *flag, T *Un, T *UnInv,
                                                            T *Tw, int64_t ldt, T *Sv, T *tau)
 {
+    __builtin_amdgcn_s_setprio(3);
     typedef PanelMfma<T> Mf;
     typedef typename Mf::acc_t acc_t;
+    constexpr int NW = kHrThreads / 64;
     __shared__ T M[128 * kHrLD];
     __shared__ T Ws[8][16 * kHrTL];
     __shared__ T Zs[16 * kHrTL];
@@ -1119,28 +1124,31 @@ __global__ __launch_bounds__(kHrThreads) void hr_lu_kernel(int k, T *Q, int64_t 
     const int w = __builtin_amdgcn_readfirstlane(t >> 6);
     const int li = lane & 15, lk = lane >> 4;
     {
-#pragma unroll 1
-      for (int q0 = 0; q0 < 32; q0 += 16) {
         // unconditional loads from clamped indices (the top k×k block always
         // exists), so that all 32 stay in flight; out-of-range values are
         // replaced afterwards
-        T v[16][2];
+        T v[128 / NW][2];
 #pragma unroll
-        for (int qq = 0; qq < 16; ++qq)
+        for (int q = 0; q < 128 / NW; ++q)
 #pragma unroll
             for (int s = 0; s < 2; ++s) {
-                const int i = lane + 64 * s, l = w + 4 * (q0 + qq);
+                const int i = lane + 64 * s, l = w + NW * q;
                 const int ic = i < k ? i : k - 1, lcl = l < k ? l : k - 1;
-                const T q = Q[ic + (int64_t)lcl * ldq];
-                v[qq][s] = (i < k && l < k) ? -q : T(0);
+                v[q][s] = Q[ic + (int64_t)lcl * ldq];
             }
 #pragma unroll
-        for (int qq = 0; qq < 16; ++qq)
+        for (int q = 0; q < 128 / NW; ++q)
 #pragma unroll
-            for (int s = 0; s < 2; ++s) M[lane + 64 * s + (w + 4 * (q0 + qq)) * kHrLD] = v[qq][s];
-      }
+            for (int s = 0; s < 2; ++s) hold(v[q][s]);
+#pragma unroll
+        for (int q = 0; q < 128 / NW; ++q)
+#pragma unroll
+            for (int s = 0; s < 2; ++s) {
+                const int i = lane + 64 * s, l = w + NW * q;
+                M[i + l * kHrLD] = (i < k && l < k) ? -v[q][s] : T(0);
+            }
     }
-    __syncthreads();
+    lds_barrier();
 
     // one 16×16 tile product on MFMA: acc += A B, A(i, kk) = a(i, kk),
     // B(kk, j) = b(kk, j); element r of lane l of the result sits at
@@ -1158,18 +1166,17 @@ __global__ __launch_bounds__(kHrThreads) void hr_lu_kernel(int k, T *Q, int64_t 
         // scheduling fences between the chained stages of this wave's
         // work keep their loads from being hoisted into the elimination
         __builtin_amdgcn_sched_barrier(0);
-        T dv[16], uv[16];
-        HrLuCols<0, T>::run(d, dv, uv, r, nbk);
+        HrLuCols<0, T>::run(d, r);
         __builtin_amdgcn_sched_barrier(0);
-        if (lane == 0) {
+        // u_r, and S_r, whose sign it has
+        T udiag = d[0];
 #pragma unroll
-            for (int c = 0; c < 16; ++c)
-                if (c < nbk) {
-                    Dv[jb + c] = dv[c];
-                    Uv[jb + c] = uv[c];
-                }
+        for (int c = 1; c < 16; ++c) udiag = r == c ? d[c] : udiag;
+        if (lane < 16) {
+            Dv[jb + r] = dcopysign<T>(T(1), udiag);
+            Uv[jb + r] = udiag;
         }
-        if (lane < 16 && jb + r < 128) {
+        if (lane < 16) {
 #pragma unroll
             for (int c = 0; c < 16; ++c) M[jb + r + (jb + c) * kHrLD] = d[c];
         }
@@ -1183,9 +1190,6 @@ __global__ __launch_bounds__(kHrThreads) void hr_lu_kernel(int k, T *Q, int64_t 
 #pragma unroll
         for (int t = 0; t < 4; ++t) wv[t] = zv[t] = (r == g + 4 * t) ? T(1) : T(0);
         TileInvSteps<0, T>::run(m, wv);
-        T udiag = d[0];
-#pragma unroll
-        for (int c = 1; c < 16; ++c) udiag = r == c ? d[c] : udiag;
         const T myr = r < nbk ? recip1(udiag) : T(1);
         // unscaled rows Y[i] = U_ii Z[i]: Y[i] −= (U[i][k]/U[k][k]) Y[k]
         HrUpMul<0, T>::run(d, myr, r, m);
@@ -1218,14 +1222,14 @@ __global__ __launch_bounds__(kHrThreads) void hr_lu_kernel(int k, T *Q, int64_t 
         for (int q = 0; q < 4; ++q) M[io + Mf::row(lane, q) + (jo + li) * kHrLD] = acc[q];
     };
     if (w == 0) elim(0);
-    __syncthreads();
+    lds_barrier();
     for (int jb = 0; jb < k; jb += 16) {
         const int nbk = min(16, k - jb), c0 = jb + nbk;
         T *Wb = Ws[jb >> 4];
         if (c0 >= k) break;
         const int nct = (k - c0 + 15) / 16;
         // ---- U_J,right = W M_J,right and L_below,J = M_below,J Z
-        for (int it = w; it < 2 * nct; it += kHrThreads / 64) {
+        for (int it = w; it < 2 * nct; it += NW) {
             const int o = c0 + 16 * (it >> 1);
             acc_t acc = {T(0), T(0), T(0), T(0)};
             if ((it & 1) == 0) {
@@ -1246,7 +1250,7 @@ __global__ __launch_bounds__(kHrThreads) void hr_lu_kernel(int k, T *Q, int64_t 
                 for (int q = 0; q < 4; ++q) M[o + Mf::row(lane, q) + (jb + li) * kHrLD] = acc[q];
             }
         }
-        __syncthreads();
+        lds_barrier();
         // ---- M_below,right −= L_below,J U_J,right: wave 0 updates the next
         //      diagonal tile and eliminates it while waves 1–3 update the rest
         if (w == 0) {
@@ -1254,113 +1258,87 @@ __global__ __launch_bounds__(kHrThreads) void hr_lu_kernel(int k, T *Q, int64_t 
             __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
             elim(c0);
         } else {
-            for (int it = w; it < nct * nct; it += kHrThreads / 64 - 1) trail_tile(jb, c0, nct, it);
+            for (int it = w; it < nct * nct; it += NW - 1) trail_tile(jb, c0, nct, it);
         }
-        __syncthreads();
+        lds_barrier();
     }
 
-    // ---- outputs of the LU: V₁ over Q's top block, Û = U S in place
+    // From here on M is only read.  V₁ over Q's top block, and Un(l, i) =
+    // −U(i, l), written down the columns of both
     {
-#pragma unroll 1
-      for (int q0 = 0; q0 < 32; q0 += 8) {
-        T v[8][2];
+        T v[128 / NW][2];
 #pragma unroll
-        for (int qq = 0; qq < 8; ++qq)
-#pragma unroll
-            for (int s = 0; s < 2; ++s) v[qq][s] = M[lane + 64 * s + (w + 4 * (q0 + qq)) * kHrLD];
-#pragma unroll
-        for (int qq = 0; qq < 8; ++qq)
+        for (int q = 0; q < 128 / NW; ++q)
 #pragma unroll
             for (int s = 0; s < 2; ++s) {
-                const int i = lane + 64 * s, l = w + 4 * (q0 + qq);
-                if (i < k && l < k) {
-                    Q[i + (int64_t)l * ldq] = i > l ? v[qq][s] : (i == l ? T(1) : T(0));
-                    if (i <= l) M[i + l * kHrLD] = v[qq][s] * Dv[l];
-                }
+                const int i = lane + 64 * s, l = w + NW * q;
+                v[q][s] = M[i >= l ? i + l * kHrLD : l];
             }
-      }
+#pragma unroll
+        for (int q = 0; q < 128 / NW; ++q)
+#pragma unroll
+            for (int s = 0; s < 2; ++s) {
+                const int i = lane + 64 * s, l = w + NW * q;
+                if (i < k && l < k)
+                    Q[i + (int64_t)l * ldq] = i > l ? v[q][s] : (i == l ? T(1) : T(0));
+            }
+#pragma unroll
+        for (int q = 0; q < 128 / NW; ++q)
+#pragma unroll
+            for (int s = 0; s < 2; ++s) {
+                const int i = w + NW * q, l = lane + 64 * s;
+                if (i <= l && l < k) Un[l + (int64_t)i * k] = -M[i + l * kHrLD];
+            }
     }
     if (t < k) {
         Sv[t] = Dv[t];
         tau[t] = Dv[t] * Uv[t];
     }
-    __syncthreads();
-    // Un(l, i) = −U(i, l) = −Û(i, l) S_l, written down the columns of Un
-    {
-#pragma unroll 1
-      for (int q0 = 0; q0 < 32; q0 += 8) {
-        T v[8][2];
-#pragma unroll
-        for (int qq = 0; qq < 8; ++qq)
-#pragma unroll
-            for (int s = 0; s < 2; ++s) v[qq][s] = M[w + 4 * (q0 + qq) + (lane + 64 * s) * kHrLD];
-#pragma unroll
-        for (int qq = 0; qq < 8; ++qq)
-#pragma unroll
-            for (int s = 0; s < 2; ++s) {
-                const int i = w + 4 * (q0 + qq), l = lane + 64 * s;
-                if (i <= l && l < k) Un[l + (int64_t)i * k] = -v[qq][s] * Dv[l];
-            }
-      }
-    }
-    __syncthreads();   // the T sweep below rewrites M
 
-    // ---- T = Û V₁⁻ᵀ
-    for (int jb = 0; jb < k; jb += 16) {
-        const int c0 = min(k, jb + 16);
-        const T *Wb = Ws[jb >> 4];
-        // T[0:c0, J] = Acc[0:c0, J] W_Jᵀ (Acc(i, c) for i > c is V₁: zero)
-        for (int it = w; it <= (jb >> 4); it += kHrThreads / 64) {
-            const int io = 16 * it;
-            acc_t acc = {T(0), T(0), T(0), T(0)};
+    // ---- T = Û V₁⁻ᵀ, Û = U S: rows of T are independent, so a wave takes 16
+    // of them through all columns in registers, transposed (a tile in the
+    // accumulator's layout is the B operand of the products of the sweep)
+    {
+        const int c = w < 4 ? w : 11 - w;     // waves of one SIMD: c and 7 − c
+        acc_t x[8];
 #pragma unroll
-            for (int kq = 0; kq < 4; ++kq) {
-                const int kk = 4 * kq + lk;
-                const T a = (io + li <= jb + kk) ? M[io + li + (jb + kk) * kHrLD] : T(0);
-                acc = Mf::mma(a, Wb[li + kk * kHrTL], acc);
-            }
+        for (int J = 0; J < 8; ++J)
 #pragma unroll
             for (int q = 0; q < 4; ++q) {
-                const int i = io + Mf::row(lane, q), c = jb + li;
-                if (i <= c) M[i + c * kHrLD] = acc[q];
+                const int i = 16 * c + li, l = 16 * J + Mf::row(lane, q);
+                const T v = M[i <= l ? i + l * kHrLD : l] * Dv[l];
+                x[J][q] = i <= l && l < k ? v : T(0);
             }
-        }
-        __syncthreads();
-        if (c0 >= k) break;
-        const int nct = (k - c0 + 15) / 16, nrt = (jb >> 4) + 1;
-        // Acc[0:c0, right] −= T[0:c0, J] V₁[right, J]ᵀ
-        for (int it = w; it < nrt * nct; it += kHrThreads / 64) {
-            const int io = 16 * (it % nrt), jo = c0 + 16 * (it / nrt);
-            acc_t acc;
+        auto sweep = [&](auto full) {   // a full block without branches on k
 #pragma unroll
-            for (int q = 0; q < 4; ++q) acc[q] = M[io + Mf::row(lane, q) + (jo + li) * kHrLD];
+            for (int J = 0; J < 8; ++J) {
+                if (J < c || (!decltype(full)::value && 16 * J >= k)) continue;
+                acc_t y = {T(0), T(0), T(0), T(0)};
 #pragma unroll
-            for (int kq = 0; kq < 4; ++kq) {
-                const int kk = 4 * kq + lk;
-                const T a = (io + li <= jb + kk) ? -M[io + li + (jb + kk) * kHrLD] : T(0);
-                acc = Mf::mma(a, M[jo + li + (jb + kk) * kHrLD], acc);
+                for (int kq = 0; kq < 4; ++kq)
+                    y = Mf::mma(Ws[J][li + Mf::row(lane, kq) * kHrTL], x[J][kq], y);
+                x[J] = y;
+#pragma unroll
+                for (int j = J + 1; j < 8; ++j) {
+                    if (!decltype(full)::value && 16 * j >= k) continue;
+#pragma unroll
+                    for (int kq = 0; kq < 4; ++kq)
+                        x[j] = Mf::mma(M[16 * j + li + (16 * J + Mf::row(lane, kq)) * kHrLD], -y[kq],
+                                       x[j]);
+                }
             }
+        };
+        if (k == 128)
+            sweep(std::true_type{});
+        else
+            sweep(std::false_type{});
 #pragma unroll
-            for (int q = 0; q < 4; ++q) M[io + Mf::row(lane, q) + (jo + li) * kHrLD] = acc[q];
-        }
-        __syncthreads();
-    }
-    {
-#pragma unroll 1
-      for (int q0 = 0; q0 < 32; q0 += 8) {
-        T v[8][2];
+        for (int J = 0; J < 8; ++J)
 #pragma unroll
-        for (int qq = 0; qq < 8; ++qq)
-#pragma unroll
-            for (int s = 0; s < 2; ++s) v[qq][s] = M[lane + 64 * s + (w + 4 * (q0 + qq)) * kHrLD];
-#pragma unroll
-        for (int qq = 0; qq < 8; ++qq)
-#pragma unroll
-            for (int s = 0; s < 2; ++s) {
-                const int i = lane + 64 * s, l = w + 4 * (q0 + qq);
-                if (i < k && l < k) Tw[i + (int64_t)l * ldt] = i <= l ? v[qq][s] : T(0);
+            for (int q = 0; q < 4; ++q) {
+                const int i = 16 * c + li, l = 16 * J + Mf::row(lane, q);
+                if (i < k && l < k) Tw[i + (int64_t)l * ldt] = i <= l ? x[J][q] : T(0);
             }
-      }
     }
 }
 
@@ -1371,6 +1349,7 @@ template <typename T>
 __global__ void hr_finish_kernel(int64_t m, int k, const T *Vw, int64_t ldv, const T *R,
                                  const T *Sv, T *A, int64_t lda, const int *flag)
 {
+    __builtin_amdgcn_s_setprio(3);
     if (*flag != 0) return;
     const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
     const int j = blockIdx.y;
