@@ -72,55 +72,47 @@ __global__ __launch_bounds__(256) void zgemm_kernel(int64_t M, int64_t N, int64_
             acci[i][j] = acc_t{0, 0, 0, 0};
         }
     // slab at k0 of op(A) (x, k): N — A[x + k·lda]; C — conj(A[k + x·lda]);
-    // and of op(B) (k, y): N — B[k + y·ldb]; C — conj(B[y + k·ldb])
-    T ar[4], ai[4], br[4], bi[4];
+    // and of op(B) (k, y): N — B[k + y·ldb]; C — conj(B[y + k·ldb]).  Loads
+    // from clamped places, out-of-range values dropped when they are staged
+    typedef T z2 __attribute__((ext_vector_type(2), aligned(sizeof(T))));
+    z2 av[4], bv[4];
+    auto ax = [&](int l) { return TA ? (t >> 4) + 16 * l : t & 63; };
+    auto ak = [&](int l) { return TA ? t & 15 : (t >> 6) + 4 * l; };
+    auto by = [&](int l) { return TB ? t & 63 : (t >> 4) + 16 * l; };
+    auto bk = [&](int l) { return TB ? (t >> 6) + 4 * l : t & 15; };
     auto fetch = [&](int64_t k0) {
 #pragma unroll
         for (int l = 0; l < 4; ++l) {
-            int x, k;
-            if (!TA) { x = t & 63; k = (t >> 6) + 4 * l; }
-            else { k = t & 15; x = (t >> 4) + 16 * l; }
-            const int64_t gx = m0 + x, gk = k0 + k;
-            ar[l] = T(0);
-            ai[l] = T(0);
-            if (gx < M && gk < k_end) {
-                const T *p = A + 2 * (TA ? gk + gx * lda : gx + gk * lda);
-                ar[l] = p[0];
-                ai[l] = TA ? -p[1] : p[1];
-            }
+            const int64_t x = m0 + ax(l), k = k0 + ak(l);
+            const int64_t gx = x < M ? x : M - 1, gk = k < k_end ? k : k_end - 1;
+            av[l] = *reinterpret_cast<const z2 *>(A + 2 * (TA ? gk + gx * lda : gx + gk * lda));
         }
 #pragma unroll
         for (int l = 0; l < 4; ++l) {
-            int y, k;
-            if (TB) { y = t & 63; k = (t >> 6) + 4 * l; }
-            else { k = t & 15; y = (t >> 4) + 16 * l; }
-            const int64_t gy = n0 + y, gk = k0 + k;
-            br[l] = T(0);
-            bi[l] = T(0);
-            if (gy < N && gk < k_end) {
-                const T *p = B + 2 * (TB ? gy + gk * ldb : gk + gy * ldb);
-                br[l] = p[0];
-                bi[l] = TB ? -p[1] : p[1];
-            }
+            const int64_t y = n0 + by(l), k = k0 + bk(l);
+            const int64_t gy = y < N ? y : N - 1, gk = k < k_end ? k : k_end - 1;
+            bv[l] = *reinterpret_cast<const z2 *>(B + 2 * (TB ? gy + gk * ldb : gk + gy * ldb));
         }
     };
-    // one slab ahead: VᴴA 64×64, K = 4096 in splits of 128: 48 µs (100 in
-    // splits of 256 with every load waited for)
-    fetch(k_begin);
+    // one slab ahead: VᴴA 64×64, K = 3700 in splits of 64 or 128: 21 and 35 µs
+    // (48 in splits of 128 with each load under a branch of its own, so that
+    // one waited for the other; 100 in splits of 256 with no slab ahead)
+    if (k_begin < k_end) fetch(k_begin);
     for (int64_t k0 = k_begin; k0 < k_end; k0 += kZK) {
         __syncthreads();   // the previous slab is consumed
 #pragma unroll
         for (int l = 0; l < 4; ++l) {
-            int x, k;
-            if (!TA) { x = t & 63; k = (t >> 6) + 4 * l; }
-            else { k = t & 15; x = (t >> 4) + 16 * l; }
-            Ar[k * LD + x] = ar[l];
-            Ai[k * LD + x] = ai[l];
-            int y, kb;
-            if (TB) { y = t & 63; kb = (t >> 6) + 4 * l; }
-            else { kb = t & 15; y = (t >> 4) + 16 * l; }
-            Br[kb * LD + y] = br[l];
-            Bi[kb * LD + y] = bi[l];
+            hold(av[l]);
+            hold(bv[l]);
+        }
+#pragma unroll
+        for (int l = 0; l < 4; ++l) {
+            const bool ina = m0 + ax(l) < M && k0 + ak(l) < k_end;
+            const bool inb = n0 + by(l) < N && k0 + bk(l) < k_end;
+            Ar[ak(l) * LD + ax(l)] = ina ? av[l].x : T(0);
+            Ai[ak(l) * LD + ax(l)] = ina ? (TA ? -av[l].y : av[l].y) : T(0);
+            Br[bk(l) * LD + by(l)] = inb ? bv[l].x : T(0);
+            Bi[bk(l) * LD + by(l)] = inb ? (TB ? -bv[l].y : bv[l].y) : T(0);
         }
         __syncthreads();
         if (k0 + kZK < k_end) fetch(k0 + kZK);   // in flight behind this slab's products
@@ -142,41 +134,50 @@ __global__ __launch_bounds__(256) void zgemm_kernel(int64_t M, int64_t N, int64_
             for (int i = 0; i < 2; ++i)
 #pragma unroll
                 for (int j = 0; j < 2; ++j) {
-                    accr[i][j] = Mf::mma(a_r[i], b_r[j], accr[i][j]);
-                    accr[i][j] = Mf::mma(-a_i[i], b_i[j], accr[i][j]);
-                    acci[i][j] = Mf::mma(a_r[i], b_i[j], acci[i][j]);
-                    acci[i][j] = Mf::mma(a_i[i], b_r[j], acci[i][j]);
+                    accr[i][j] = Mf::mma(b_r[j], a_r[i], accr[i][j]);
+                    accr[i][j] = Mf::mma(b_i[j], -a_i[i], accr[i][j]);
+                    acci[i][j] = Mf::mma(b_i[j], a_r[i], acci[i][j]);
+                    acci[i][j] = Mf::mma(b_r[j], a_i[i], acci[i][j]);
                 }
         }
     }
-    const bool beta0 = beta == T(0);
+    // the products are formed transposed, so that a block's lanes hold 16
+    // consecutive rows of its columns; C is read a row of blocks at a time
+    const bool beta0 = beta == T(0) || part;
 #pragma unroll
-    for (int i = 0; i < 2; ++i)
+    for (int i = 0; i < 2; ++i) {
+        const int64_t gr = m0 + wm * 32 + i * 16 + (lane & 15), grc = gr < M ? gr : M - 1;
+        z2 old[2][4];
+        if (!beta0) {
+#pragma unroll
+            for (int j = 0; j < 2; ++j)
+#pragma unroll
+                for (int r = 0; r < 4; ++r) {
+                    const int64_t gc = n0 + wn * 32 + j * 16 + Mf::row(lane, r);
+                    old[j][r] = *reinterpret_cast<const z2 *>(C + 2 * (grc + (gc < N ? gc : N - 1) * ldc));
+                }
+        }
 #pragma unroll
         for (int j = 0; j < 2; ++j)
 #pragma unroll
             for (int r = 0; r < 4; ++r) {
-                const int64_t gr = m0 + wm * 32 + i * 16 + Mf::row(lane, r);
-                const int64_t gc = n0 + wn * 32 + j * 16 + (lane & 15);
+                const int64_t gc = n0 + wn * 32 + j * 16 + Mf::row(lane, r);
                 if (gr >= M || gc >= N) continue;
+                z2 v = {alpha * accr[i][j][r], alpha * acci[i][j][r]};
                 if (part) {
-                    T *q = part + 2 * ((int64_t)blockIdx.z * M * N + gr + gc * M);
-                    q[0] = alpha * accr[i][j][r];
-                    q[1] = alpha * acci[i][j][r];
+                    *reinterpret_cast<z2 *>(part + 2 * ((int64_t)blockIdx.z * M * N + gr + gc * M)) = v;
                     continue;
                 }
                 if (MODE == 1 && gr + diag_off < gc) continue;
                 if (MODE == 2 && gr + diag_off > gc) continue;
-                T *c = C + 2 * (gr + gc * ldc);
-                T re = alpha * accr[i][j][r], im = alpha * acci[i][j][r];
                 if (!beta0) {
-                    re += beta * c[0];
-                    im += beta * c[1];
+                    v.x += beta * old[j][r].x;
+                    v.y += beta * old[j][r].y;
                 }
-                if (HERM && gr + diag_off == gc) im = T(0);
-                c[0] = re;
-                c[1] = im;
+                if (HERM && gr + diag_off == gc) v.y = T(0);
+                *reinterpret_cast<z2 *>(C + 2 * (gr + gc * ldc)) = v;
             }
+    }
 }
 
 // C = β C + Σ_z part[z] (M×N complex, ld M), the partials in a fixed order.
@@ -215,7 +216,7 @@ int zgemm_launch(hipStream_t s, int64_t M, int64_t N, int64_t K, T alpha, const 
     const int64_t tiles = cdiv(M, kZB) * cdiv(N, kZB);
     int64_t S = 1;
     if (MODE == 0 && !HERM && ws && tiles < 128 && K >= 1024) {
-        S = std::min<int64_t>(std::min<int64_t>(cdiv(K, 128), std::max<int64_t>(1, 512 / tiles)),
+        S = std::min<int64_t>(std::min<int64_t>(cdiv(K, 64), std::max<int64_t>(1, 512 / tiles)),
                               64);
         while (S > 1 && 2 * S * M * N > ws_elems) --S;
     }
@@ -1326,7 +1327,7 @@ struct ZqrWS {
 // whatever the block size (the factors do not depend on it): the panel and
 // its T by one launch, then Hᴴ on the next block column, on which the next
 // panel starts while the side stream applies Hᴴ to the rest (depth-1
-// look-ahead, as qr_blocked_dev).  4096×2048 ComplexF64: 13.8 ms (45.8 with
+// look-ahead, as qr_blocked_dev).  4096×2048 ComplexF64: 12.8 ms (45.5 with
 // 32-wide block columns, two launches per column and no look-ahead); the
 // chain of panels and next-block updates is what it takes.
 template <typename T>
