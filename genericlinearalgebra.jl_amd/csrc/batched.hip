@@ -65,45 +65,32 @@ __device__ __forceinline__ void border() { __builtin_amdgcn_fence(__ATOMIC_SEQ_C
 //       which is what keeps the wave busy: the columns of L come back from
 //       HBM, not from a cache); the first group also carries the diagonal
 //       tile C_dd, whose two operands are the same panel block;
-//   (2) after the first group's K loop, C_dd is factored in row layout by
-//       the Cholesky's tile factor (cholUnblocked!'s column steps,
-//       src/cholesky.jl:3-15), L_dd is written back, y_p = L_dd⁻¹ b_p is
-//       solved by 16 broadcast steps and W = L_dd⁻¹ formed in registers;
+//   (2) after the first group's K loop, C_dd is factored and inverted by the
+//       Cholesky's tile factor (cholUnblocked!'s column steps,
+//       src/cholesky.jl:3-15), L_dd is written back and y_p = W b_p, W =
+//       L_dd⁻¹;
 //   (3) each group: X = C L_dd⁻ᵀ as Xᵀ = W Cᵀ on MFMA, written back, and
 //       b_rows −= X y_p.
 // Then Lᵀ x = y from the last panel: z = y_p − L_belowᵀ x_below (16-lane row
 // sums), and a 16-step back substitution on the columns of L_dd.
+// Bound: the chain of each wave (memory round trips, diagonal tiles), eight
+// waves a CU.  10000 FP64 matrices of 8…256: 1.25 ms; 1.63 with the tiles'
+// loads under branches (one round trip after another) and the diagonal tiles
+// factored, inverted and solved in row layout.
 
-// A[r][c] for r, c < n, else 0; the load itself is unconditional (clamped
-// indices), so that a run of them stays in flight.
 // Global-memory view of a pointer read from device memory (the compiler
 // cannot infer it, and flat accesses cost more than global ones).
 template <typename T>
 using gmem = __attribute__((address_space(1))) T;
 
+// A[r][c] from clamped indices: a run of them stays in flight until the
+// callers hold their values and drop those out of range.
 template <typename T>
-__device__ __forceinline__ T ldz(const gmem<T> *__restrict__ A, int lda, int n, int r, int c)
+__device__ __forceinline__ T ldc(const gmem<T> *__restrict__ A, int lda, int n, int r, int c)
 {
     const int rc = r < n ? r : n - 1, cc = c < n ? c : n - 1;
-    const T v = A[rc + (int64_t)cc * lda];
-    return (r < n && c < n) ? v : T(0);
+    return A[rc + (int64_t)cc * lda];
 }
-
-// Forward substitution on the diagonal tile (row layout, a[c] = L[i][c],
-// zero above the diagonal; rd[c] = 1/L[c][c] in every lane): z_i ← y_i.
-template <int C, typename T>
-struct DiagFwd {
-    static __device__ __forceinline__ void run(const T a[16], const T rd[16], int i, T &z)
-    {
-        const T y = row_bcast<C>(z) * rd[C];
-        z = i == C ? y : fma_t(-a[C], y, z);
-        DiagFwd<C + 1, T>::run(a, rd, i, z);
-    }
-};
-template <typename T>
-struct DiagFwd<16, T> {
-    static __device__ __forceinline__ void run(const T *, const T *, int, T &) {}
-};
 
 // Back substitution on the diagonal tile's transpose (column layout,
 // lc[k] = L[k][i], zero above the diagonal; rdi = 1/L[i][i]): z_i ← x_i.
@@ -166,6 +153,10 @@ __device__ void wave_chol_solve(int n, T *Ap, int lda, T *bp, int *info, T *S)
     typedef PanelMfma<T> Mf;
     typedef typename Mf::acc_t acc_t;
     const int lane = threadIdx.x & 63, li = lane & 15, g = lane >> 4;
+    if (n <= 0) {   // nothing to read: the clamped indices below need a row
+        if (lane == 0 && info) *info = 0;
+        return;
+    }
     T *ring = S;                        // NS slabs
     T *Ts = S + NS * WL::kSlab;         // 16 × kMTL staging tile
     T *bv = Ts + 16 * kMTL;             // b, then y, then x
@@ -227,46 +218,6 @@ __device__ void wave_chol_solve(int n, T *Ap, int lda, T *bp, int *info, T *S)
     for (int e = lane; e < n; e += 64) bv[e] = b[e];
     border();
     int bad = 0;
-    auto nothing = [] {};
-    // factor + invert + forward-solve one 16×16 diagonal tile given in the
-    // accumulator layout: L written back at (row0, row0) for the first nv
-    // rows, y = L⁻¹ z at bv[row0..], W = L⁻¹ to w (w[q] = W[i][c_q])
-    auto diag_tile = [&](const acc_t &t, int row0, int nv, T zin, T w[4]) {
-#pragma unroll
-        for (int q = 0; q < 4; ++q) Ts[li * kMTL + cq[q]] = t[q];
-        border();
-        T a[16], rd[16];
-#pragma unroll
-        for (int j = 0; j < 16; ++j)
-            a[j] = li >= nv ? (j == li ? T(1) : T(0)) : (j <= li ? Ts[li * kMTL + j] : T(0));
-        border();
-        int fneg = 16;
-        TileFactorCols<0, T>::run(a, rd, li, fneg);
-        if (fneg < nv && !bad) bad = row0 + fneg + 1;
-#pragma unroll
-        for (int j = 0; j < 16; ++j) a[j] = j <= li ? a[j] : T(0);
-        if (g == 0 && li < nv) {
-#pragma unroll
-            for (int j = 0; j < 16; ++j)
-                if (j <= li) A[(row0 + li) + (int64_t)(row0 + j) * lda] = a[j];
-        }
-        T z = li < nv ? zin : T(0);
-        DiagFwd<0, T>::run(a, rd, li, z);
-        if (g == 0 && li < nv) bv[row0 + li] = z;
-        // W = L⁻¹: a[k] becomes the multiplier L[i][k]/L[k][k] (i > k)
-        T ri = rd[0];
-#pragma unroll
-        for (int k = 0; k < 16; ++k) {
-            ri = li == k ? rd[k] : ri;
-            a[k] = li > k ? a[k] * rd[k] : T(0);
-        }
-#pragma unroll
-        for (int q = 0; q < 4; ++q) w[q] = li == cq[q] ? T(1) : T(0);
-        TileInvSteps<0, T>::run(a, w);
-#pragma unroll
-        for (int q = 0; q < 4; ++q) w[q] *= ri;
-        border();
-    };
     // Σ over the tile's 4 columns of this lane (values v, weights y) and
     // the four lane groups: the same sum in every lane of row i
     auto row_dot = [&](const T v[4], const T y[4]) {
@@ -279,6 +230,39 @@ __device__ void wave_chol_solve(int n, T *Ap, int lda, T *bp, int *info, T *S)
         border();
         return sum;
     };
+    // factor, invert and forward-solve one 16×16 diagonal tile given in the
+    // accumulator layout, symmetric: L written back at (row0, row0) for the
+    // first nv rows, W = L⁻¹ to w (w[q] = W[i][c_q]), y = W z at bv[row0..]
+    auto diag_tile = [&](acc_t t, int row0, int nv, T zin, T w[4]) {
+#pragma unroll
+        for (int q = 0; q < 4; ++q)   // past nv the identity
+            if (li >= nv || cq[q] >= nv) t[q] = li == cq[q] ? T(1) : T(0);
+        const unsigned neg = tile_factor<T>(t, w, nv);
+        if constexpr (sizeof(T) == 4) {   // from columns g + 4q to 4g + q
+            T v[4];
+#pragma unroll
+            for (int q = 0; q < 4; ++q)
+#pragma unroll
+                for (int r = 0; r < 4; ++r) {
+                    const T x = __shfl(w[r], li + 16 * q);
+                    v[q] = r == 0 ? x : (g == r ? x : v[q]);
+                }
+#pragma unroll
+            for (int q = 0; q < 4; ++q) w[q] = v[q];
+        }
+        if (neg != 0 && !bad) bad = row0 + __builtin_ctz(neg) + 1;
+#pragma unroll
+        for (int q = 0; q < 4; ++q)
+            if (li < nv && cq[q] <= li) A[(row0 + li) + (int64_t)(row0 + cq[q]) * lda] = t[q];
+        if (g == 0) Ts[li] = li < nv ? zin : T(0);
+        border();
+        T zq[4];
+#pragma unroll
+        for (int q = 0; q < 4; ++q) zq[q] = Ts[cq[q]];
+        const T y = row_dot(w, zq);
+        if (g == 0 && li < nv) bv[row0 + li] = y;
+        border();
+    };
     for (int p0 = 0; p0 < n; p0 += kPW2) {
         // panel of 32 columns as tiles 0 (p0..p0+15) and 1 (p0+16..p0+31)
         const int pw = min(kPW2, n - p0), pw0 = min(16, pw), pw1 = pw - pw0;
@@ -288,14 +272,31 @@ __device__ void wave_chol_solve(int n, T *Ap, int lda, T *bp, int *info, T *S)
         {
             // the 32×32 diagonal block: T00, T10, T11
             acc_t t00, t10, t11;
+            T u00[4], u10[4], u11[4];
 #pragma unroll
             for (int q = 0; q < 4; ++q) {
-                t00[q] = ldz(A, lda, n, p0 + li, p0 + cq[q]);
-                t10[q] = ldz(A, lda, n, p0 + 16 + li, p0 + cq[q]);
-                t11[q] = ldz(A, lda, n, p0 + 16 + li, p0 + 16 + cq[q]);
+                // (the diagonal tiles symmetric, from their lower triangles)
+                const int hi = max(li, cq[q]), lo = min(li, cq[q]);
+                u00[q] = ldc(A, lda, n, p0 + hi, p0 + lo);
+                u10[q] = ldc(A, lda, n, p0 + 16 + li, p0 + cq[q]);
+                u11[q] = ldc(A, lda, n, p0 + 16 + hi, p0 + 16 + lo);
             }
+            auto settle = [&] {
+#pragma unroll
+                for (int q = 0; q < 4; ++q) {
+                    hold(u00[q]);
+                    hold(u10[q]);
+                    hold(u11[q]);
+                }
+#pragma unroll
+                for (int q = 0; q < 4; ++q) {
+                    t00[q] = u00[q];
+                    t10[q] = p0 + 16 + li < n && p0 + cq[q] < n ? u10[q] : T(0);
+                    t11[q] = u11[q];
+                }
+            };
             const int rb[2] = {p0, p0 + 16};
-            stream(std::integral_constant<int, 2>{}, rb, nslab, nothing, [&](const T *st, int) {
+            stream(std::integral_constant<int, 2>{}, rb, nslab, settle, [&](const T *st, int) {
 #pragma unroll
                 for (int h = 0; h < KB / 4; ++h) {
                     const int o = (4 * h + g) * 16 + li;
@@ -329,17 +330,33 @@ __device__ void wave_chol_solve(int n, T *Ap, int lda, T *bp, int *info, T *S)
         for (int r0 = p0 + kPW2; r0 < n; r0 += 32) {
             const int nt = min(2, (n - r0 + 15) >> 4);
             acc_t c[2][2];
+            T u[2][2][4];
 #pragma unroll
             for (int t = 0; t < 2; ++t)
 #pragma unroll
                 for (int j = 0; j < 2; ++j)
 #pragma unroll
                     for (int q = 0; q < 4; ++q)
-                        c[t][j][q] = t < nt ? ldz(A, lda, n, r0 + 16 * t + li, p0 + 16 * j + cq[q]) : T(0);
+                        u[t][j][q] = ldc(A, lda, n, r0 + 16 * t + li, p0 + 16 * j + cq[q]);
+            auto settle = [&] {
+#pragma unroll
+                for (int t = 0; t < 2; ++t)
+#pragma unroll
+                    for (int j = 0; j < 2; ++j)
+#pragma unroll
+                        for (int q = 0; q < 4; ++q) hold(u[t][j][q]);
+#pragma unroll
+                for (int t = 0; t < 2; ++t)
+#pragma unroll
+                    for (int j = 0; j < 2; ++j)
+#pragma unroll
+                        for (int q = 0; q < 4; ++q)
+                            c[t][j][q] = r0 + 16 * t + li < n ? u[t][j][q] : T(0);
+            };
             const int rb[4] = {p0, p0 + 16, r0, r0 + 16};
             auto group = [&](auto nbc) {
                 constexpr int NB = decltype(nbc)::value;
-                stream(nbc, rb, nslab, nothing, [&](const T *st, int) {
+                stream(nbc, rb, nslab, settle, [&](const T *st, int) {
 #pragma unroll
                     for (int h = 0; h < KB / 4; ++h) {
                         const int o = (4 * h + g) * 16 + li;
@@ -411,12 +428,24 @@ __device__ void wave_chol_solve(int n, T *Ap, int lda, T *bp, int *info, T *S)
         T lt00[4], lt10[4], lt11[4];
 #pragma unroll
         for (int q = 0; q < 4; ++q) {
-            lt00[q] = ldz(A, lda, n, p0 + li, p0 + cq[q]);
-            lt10[q] = ldz(A, lda, n, p0 + 16 + li, p0 + cq[q]);
-            lt11[q] = ldz(A, lda, n, p0 + 16 + li, p0 + 16 + cq[q]);
+            lt00[q] = ldc(A, lda, n, p0 + li, p0 + cq[q]);
+            lt10[q] = ldc(A, lda, n, p0 + 16 + li, p0 + cq[q]);
+            lt11[q] = ldc(A, lda, n, p0 + 16 + li, p0 + 16 + cq[q]);
         }
         T xr0 = T(0), xr1 = T(0);
         auto solve = [&] {
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+                hold(lt00[q]);
+                hold(lt10[q]);
+                hold(lt11[q]);
+            }
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+                lt00[q] = p0 + li < n && p0 + cq[q] < n ? lt00[q] : T(0);
+                lt10[q] = p0 + 16 + li < n && p0 + cq[q] < n ? lt10[q] : T(0);
+                lt11[q] = p0 + 16 + li < n && p0 + 16 + cq[q] < n ? lt11[q] : T(0);
+            }
             xr1 = diag_bwd(lt11, p0 + 16, pw1, bv[p0 + 16 + li]);
             // S[j] = Σ_i L10[i][j] x1[i] for the columns c_q of this lane group
             T s[4];

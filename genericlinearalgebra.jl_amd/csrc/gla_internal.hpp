@@ -182,62 +182,6 @@ __device__ __forceinline__ void sqrt_and_rsqrt(float a, float &s, float &r)
     r = zero ? __builtin_inff() : y;
 }
 
-// Row layout of a 16×16 tile: lane (i = l % 16, g = l / 16) holds all of row
-// i in a[0..15], the same in each of the four 16-lane groups, so that every
-// value a column step needs moves by a DPP broadcast within the lane's own
-// 16-lane row (a few cycles) rather than through the LDS crossbar.
-
-// Column C's rank-1 update of the entries a[J..15]: a[j] -= l_i l_j, with
-// l_j = L[j][C] broadcast from lane j.  Entries right of the diagonal (j > i)
-// take meaningless values and are cleared by the caller.
-template <int C, int J, typename T>
-struct TileColUpdate {
-    static __device__ __forceinline__ void run(T a[16], T l)
-    {
-        const T lj = row_bcast<J>(l);
-        if constexpr (sizeof(T) == 8)
-            a[J] = __builtin_fma(-l, lj, a[J]);
-        else
-            a[J] = __builtin_fmaf(-l, lj, a[J]);
-        TileColUpdate<C, J + 1, T>::run(a, l);
-    }
-};
-template <int C, typename T>
-struct TileColUpdate<C, 16, T> {
-    static __device__ __forceinline__ void run(T *, T) {}
-};
-
-// Factors the symmetric tile held in row layout in place, right-looking,
-// column by column as cholUnblocked! does (src/cholesky.jl:3-15): sqrt of
-// the pivot, scale by its reciprocal, rank-1 update (the update products are
-// (a_ic r)(a_jc r), each factor rounded once, as in the scaled column).
-// rd[c] receives 1/L[c][c].  The first pivot whose square root is taken of
-// a negative number, among the first `nvalid`, is recorded in *info as
-// gbase + c + 1.  Entries right of the diagonal are left meaningless.
-// The 16 column steps are one branch-free block (the first negative pivot
-// is only noted in `fneg`, its column or 16 if none, and reported after the
-// tile), so that the compiler can overlap the trailing updates of column c
-// with the square root of c + 1.
-template <int C, typename T>
-struct TileFactorCols {
-    static __device__ __forceinline__ void run(T a[16], T rd[16], int i, int &fneg)
-    {
-        const T d = row_bcast<C>(a[C]);
-        fneg = (d < T(0) && fneg == 16) ? C : fneg;
-        T s, r;
-        sqrt_and_rsqrt(d, s, r);
-        rd[C] = r;
-        const T l = a[C] * r;
-        a[C] = i == C ? s : l;
-        TileColUpdate<C, C + 1, T>::run(a, l);
-        TileFactorCols<C + 1, T>::run(a, rd, i, fneg);
-    }
-};
-template <typename T>
-struct TileFactorCols<16, T> {
-    static __device__ __forceinline__ void run(T *, T *, int, int &) {}
-};
-
 // 16×16×4 MFMA with one A and one B element per lane; accumulator element r
 // of lane l sits at (row(l, r), l % 16) of the 16×16 tile.
 template <typename T>
@@ -441,11 +385,10 @@ __device__ __forceinline__ void tile_four_columns(typename PanelMfma<T>::acc_t &
 // cholUnblocked! does (src/cholesky.jl:3-15; the products are (a_ic r)(a_jc
 // r), each factor rounded once), then one rank-4 MFMA for the rest of the
 // tile.  The inverse's elimination steps fill the pivot chain's latency.
-// The first pivot among the first `nvalid` whose square root is taken of a
-// negative number is recorded in *info as gbase + index + 1.
+// Returns the mask of the pivots among the first `nvalid` whose square root is
+// taken of a negative number.
 template <typename T>
-__device__ __forceinline__ void tile_factor(typename PanelMfma<T>::acc_t &a, T w[4], int nvalid,
-                                            int *info, int64_t gbase)
+__device__ __forceinline__ unsigned tile_factor(typename PanelMfma<T>::acc_t &a, T w[4], int nvalid)
 {
     typedef PanelMfma<T> M;
     const int lane = threadIdx.x & 63;
@@ -459,7 +402,6 @@ __device__ __forceinline__ void tile_factor(typename PanelMfma<T>::acc_t &a, T w
     tile_four_columns<2, T>(a, lt, w, dsel, ysel, i, g);
     tile_four_columns<3, T>(a, lt, w, dsel, ysel, i, g);
     const unsigned neg = (unsigned)__ballot(dsel < T(0) && i < nvalid) & 0xffffu;
-    if (neg != 0 && lane == 0 && info) atomicCAS(info, 0, (int)(gbase + __builtin_ctz(neg) + 1));
     // the diagonal: √d = d·y corrected once
     T s = dsel * ysel;
     s = fma_t(fma_t(-s, s, dsel), T(0.5) * ysel, s);
@@ -468,6 +410,16 @@ __device__ __forceinline__ void tile_factor(typename PanelMfma<T>::acc_t &a, T w
     for (int r = 0; r < 4; ++r) a[r] = M::row(lane, r) == i ? s : lt[r];
 #pragma unroll
     for (int q = 0; q < 4; ++q) w[q] *= ysel;
+    return neg;
+}
+// The same; the first such pivot is recorded in *info as gbase + index + 1.
+template <typename T>
+__device__ __forceinline__ void tile_factor(typename PanelMfma<T>::acc_t &a, T w[4], int nvalid,
+                                            int *info, int64_t gbase)
+{
+    const unsigned neg = tile_factor<T>(a, w, nvalid);
+    if (neg != 0 && (threadIdx.x & 63) == 0 && info)
+        atomicCAS(info, 0, (int)(gbase + __builtin_ctz(neg) + 1));
 }
 
 // Holds a loaded value where it is.  A load from a clamped address whose value
