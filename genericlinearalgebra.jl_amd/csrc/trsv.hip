@@ -365,7 +365,11 @@ __global__ void tri_solve_prepare_kernel(int64_t cnt, T *Y, int *ticket, int sol
 
 // ---------------------------------------------------- symmetric residual --
 constexpr int kVB = 64;    // rows of a block
-constexpr int kRB = 8;     // blocks per rectangle side (512 rows)
+// Blocks per rectangle side: the smaller, the more workgroups and the more
+// partials a row (2 n/128 of 128 bytes against n/2 of A's elements).  Solve with
+// two corrections, 2 -> 4 -> 8 per side: n = 1000 559 -> 672 -> 1146 µs, 8192 4.30 ->
+// 4.36 -> 4.78 ms; n = 16384 18.9 ms with 2 and 4, and 4 takes half the workspace.
+inline int symv_rb(int64_t n) { return n <= 8192 ? 2 : 4; }
 
 // Symmetric product Y = A X over the lower triangle of A, each element of A
 // read once.  Workgroup (I, J), J ≤ I, takes the rectangle of 64×64 blocks
@@ -377,6 +381,7 @@ constexpr int kRB = 8;     // blocks per rectangle side (512 rows)
 // each written by exactly one workgroup; symv_finish_kernel adds them in a
 // fixed order, so the result does not depend on scheduling.  The next block
 // is loaded into registers while the current one is multiplied.
+template <int kRB>
 __global__ __launch_bounds__(kST, 2) void symv_rect_kernel(int64_t n, const double *__restrict__ A,
                                                            int64_t lda,
                                                            const double *__restrict__ Xt,
@@ -399,35 +404,43 @@ __global__ __launch_bounds__(kST, 2) void symv_rect_kernel(int64_t n, const doub
     const int64_t nb = (n + kVB - 1) / kVB;
     const int64_t i0 = (int64_t)I * kRB, j0 = (int64_t)J * kRB;
 
-    // thread t holds rows lane, columns w + 4u (u < 16) of a block
-    auto gload = [&](int64_t i, int64_t j, double (&r)[16]) {
-        const int64_t row = i * kVB + lane;
+    // thread t holds rows lane, columns w + 4u (u < 16) of a block and four
+    // elements of its x_i; loads from clamped places, what is out of range
+    // dropped when they are staged
+    double ra[16], rx[4];
+    auto gload = [&](int64_t i, int64_t j) {
+        const int64_t row = i * kVB + lane, rc = row < n ? row : n - 1;
 #pragma unroll
         for (int u = 0; u < 16; ++u) {
             const int64_t col = j * kVB + w + 4 * u;
-            r[u] = (row < n && col < n) ? A[row + col * lda] : 0.0;
+            ra[u] = A[rc + (col < n ? col : n - 1) * lda];
         }
+#pragma unroll
+        for (int u = 0; u < 4; ++u) rx[u] = Xt[i * kVB * kSR + t + kST * u];
     };
     d4 yr[kRB];
 #pragma unroll
     for (int b = 0; b < kRB; ++b) yr[b] = d4{0.0, 0.0, 0.0, 0.0};
-    double ra[16];
-    gload(i0, j0, ra);
+    gload(i0, j0);
     for (int bj = 0; bj < kRB; ++bj) {
         const int64_t j = j0 + bj;
         if (j >= nb) break;
+#pragma unroll
+        for (int u = 0; u < 4; ++u) xj[t + kST * u] = Xt[j * kVB * kSR + t + kST * u];
         d4 yc = d4{0.0, 0.0, 0.0, 0.0};
 #pragma unroll
         for (int bi = 0; bi < kRB; ++bi) {
             const int64_t i = i0 + bi;
             if (i >= nb || i < j) continue;
 #pragma unroll
-            for (int u = 0; u < 16; ++u) Ts[(w + 4 * u) * LDT + lane] = ra[u];
+            for (int u = 0; u < 16; ++u) hold(ra[u]);
 #pragma unroll
-            for (int e = t; e < kVB * kSR; e += kST) {
-                xi[e] = Xt[i * kVB * kSR + e];
-                xj[e] = Xt[j * kVB * kSR + e];
+            for (int u = 0; u < 16; ++u) {
+                const bool in = i * kVB + lane < n && j * kVB + w + 4 * u < n;
+                Ts[(w + 4 * u) * LDT + lane] = in ? ra[u] : 0.0;
             }
+#pragma unroll
+            for (int u = 0; u < 4; ++u) xi[t + kST * u] = rx[u];
             __syncthreads();
             if (i == j) {
                 // upper half of a diagonal block from its lower half
@@ -444,7 +457,7 @@ __global__ __launch_bounds__(kST, 2) void symv_rect_kernel(int64_t n, const doub
                     nj = j + 1;
                     ni = nj > i0 ? nj : i0;
                 }
-                if (nj < j0 + kRB && nj < nb && ni < nb && ni < i0 + kRB) gload(ni, nj, ra);
+                if (nj < j0 + kRB && nj < nb && ni < nb && ni < i0 + kRB) gload(ni, nj);
             }
 #pragma unroll
             for (int kq = 0; kq < kVB / 4; ++kq)
@@ -478,7 +491,7 @@ __global__ __launch_bounds__(kST, 2) void symv_rect_kernel(int64_t n, const doub
 template <typename T>
 __global__ __launch_bounds__(kST) void symv_finish_kernel(int64_t n, const double *__restrict__ Prow,
                                                           const double *__restrict__ Pcol,
-                                                          int64_t npad, int NR,
+                                                          int64_t npad, int NR, int rb,
                                                           const double *__restrict__ Xt,
                                                           const double *__restrict__ B,
                                                           int64_t ldb, int nrhs, T *__restrict__ R,
@@ -486,7 +499,7 @@ __global__ __launch_bounds__(kST) void symv_finish_kernel(int64_t n, const doubl
 {
     __shared__ double sr[2 * kST];
     const int64_t r0 = (int64_t)blockIdx.x * kVB;
-    const int Rr = (int)(blockIdx.x / kRB);
+    const int Rr = (int)(blockIdx.x / rb);
     // every element this thread visits has k = threadIdx.x % 16 (256 is a
     // multiple of 16): accumulate locally, reduce over the 16 threads of each
     // k, one atomic per k and workgroup
@@ -498,8 +511,19 @@ __global__ __launch_bounds__(kST) void symv_finish_kernel(int64_t n, const doubl
         double v = 0.0;
         if (k < nrhs) {
             double ax = 0.0;
-            for (int q = 0; q <= Rr; ++q) ax += Prow[((int64_t)q * npad + row) * kSR + k];
-            for (int q = Rr; q < NR; ++q) ax += Pcol[((int64_t)q * npad + row) * kSR + k];
+            const double *pr = Prow + row * kSR + k, *pc = Pcol + row * kSR + k;
+            int q = 0;
+            for (; q + 8 <= NR + 1; q += 8) {   // eight in flight
+                double p[8];
+#pragma unroll
+                for (int u = 0; u < 8; ++u)
+                    p[u] = q + u <= Rr ? pr[(int64_t)(q + u) * npad * kSR]
+                                       : pc[(int64_t)(q + u - 1) * npad * kSR];
+#pragma unroll
+                for (int u = 0; u < 8; ++u) ax += p[u];
+            }
+            for (; q < NR + 1; ++q)
+                ax += q <= Rr ? pr[(int64_t)q * npad * kSR] : pc[(int64_t)(q - 1) * npad * kSR];
             v = B[row + k * ldb] - ax;
             const double x = Xt[row * kSR + k];
             xs += x * x;
@@ -572,24 +596,29 @@ int symv_residual(hipStream_t s, int64_t n, const double *A, int64_t lda, const 
 {
     if (n <= 0) return GLA_OK;
     const int64_t nb = cdiv(n, kVB), npad = nb * kVB;
-    const int NR = (int)cdiv(nb, kRB);
+    const int rb = symv_rb(n), NR = (int)cdiv(nb, rb);
     double *Prow = Xt + npad * kSR;
     double *Pcol = Prow + (int64_t)NR * npad * kSR;
     hipLaunchKernelGGL(rowmajor16_kernel, dim3((unsigned)cdiv(npad * kSR, 256)), dim3(256), 0, s,
                        n, npad, nrhs, X, ldx, Xt);
     GLA_LAUNCH_CHECK();
-    hipLaunchKernelGGL(symv_rect_kernel, dim3((unsigned)(NR * (NR + 1) / 2)), dim3(kST), 0, s, n,
-                       A, lda, Xt, Prow, Pcol, npad, NR);
+    const dim3 grid((unsigned)(NR * (NR + 1) / 2));
+    if (rb == 2)
+        hipLaunchKernelGGL(symv_rect_kernel<2>, grid, dim3(kST), 0, s, n, A, lda, Xt, Prow, Pcol,
+                           npad, NR);
+    else
+        hipLaunchKernelGGL(symv_rect_kernel<4>, grid, dim3(kST), 0, s, n, A, lda, Xt, Prow, Pcol,
+                           npad, NR);
     GLA_LAUNCH_CHECK();
     hipLaunchKernelGGL((symv_finish_kernel<T>), dim3((unsigned)nb), dim3(kST), 0, s, n, Prow, Pcol,
-                       npad, NR, Xt, B, ldb, nrhs, R, nrm);
+                       npad, NR, rb, Xt, B, ldb, nrhs, R, nrm);
     GLA_LAUNCH_CHECK();
     return GLA_OK;
 }
 
 size_t symv_scratch(int64_t n)
 {
-    const int64_t nb = cdiv(n, kVB), NR = cdiv(nb, kRB);
+    const int64_t nb = cdiv(n, kVB), NR = cdiv(nb, symv_rb(n));
     return (size_t)(nb * kVB) * kSR * (1 + 2 * NR);
 }
 
