@@ -1514,12 +1514,15 @@ inline int panel_rows(const Handle *h, int w)
 }
 
 // Whether block column mm×w is factored by the reconstructed-Householder
-// path: at least as tall as wide, qr_hr rows or taller (auto: any height
-// for w ≥ 64, where it was faster from 128×128 up; 2048 rows for narrower
-// block columns), and within the fallback panel's capacity.
+// path: at least as tall as wide, qr_hr rows or taller, and within the
+// fallback panel's capacity.  Auto: any height for w ≥ 32, 512 rows for
+// w ≥ 24, none for narrower ones — the path takes 125…225 µs whatever the width, the
+// column-by-column panel 4…6 µs a column.  FP64 path / panel, µs: 64×32 136 / 164,
+// 861×63 160 / 333, 2000×63 224 / 403, 300×24 135 / 134, 861×24 137 / 164,
+// 861×16 129 / 126, 6000×8 162 / 90; FP32 64×32 125 / 131, 861×24 131 / 156.
 inline bool use_hr(const Handle *h, int64_t mm, int w)
 {
-    const int64_t minrows = h->qr_hr >= 0 ? h->qr_hr : (w >= 64 ? 1 : 2048);
+    const int64_t minrows = h->qr_hr >= 0 ? h->qr_hr : (w >= 32 ? 1 : (w >= 24 ? 512 : INT64_MAX));
     if (h->qr_hr == 0 || mm < w || mm < minrows || w > kQrNB) return false;
     return cdiv(mm, panel_rows(h, w)) <= h->num_cus;
 }
