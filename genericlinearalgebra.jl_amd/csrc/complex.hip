@@ -777,16 +777,19 @@ int zqr_panel(hipStream_t s, int64_t m, int w, T *A, int64_t lda, T *tau, T *ws)
 // 128 rows each in registers: wave v columns 8v…8v+7, lane l rows l + 64q.
 // Per column j: its owner puts it in LDS; every lane forms its rows' share of
 // xᴴ a_c (rows > j) for its wave's columns, summed over the wave; the
-// workgroup publishes the sums and workgroup 0 also row j, tagged; every
+// workgroup publishes the sums and workgroup 0 also row j; every
 // workgroup gathers all of them in a fixed order (so all hold the same
 // totals), forms reflector!'s scalars and applies them to its registers.
 // One more workgroup holds no rows: it follows the exchange and builds T from
 // the totals of the finished columns (v_iᴴ v_j = conj(a_ji) + conj(d_i)/ξ).
-// Every column has an exchange slot of its own, so nobody waits for it.
-// Bound: latency.  4096×64 FP64: 315 µs, 4.9 µs a column, of which the round
-// trip through the device-coherent level takes about 2 (3700 cycles for one
-// batch of loads) and the chain of sums, square root and update the rest; the
-// two launches per column it replaced took 14.6 µs.
+// The slots are filled with arrival marks beforehand, so a value announces
+// itself; every column has one of its own, and there are two sets: a panel marks
+// the other set's slots again for the next one.
+// Bound: latency.  4096×64 FP64: 296 µs, 4.6 µs a column, of which the round
+// trip through the device-coherent level takes about 2 and the chain of sums,
+// square root and update the rest; with each half of a value beside a tag, twice
+// the bytes, 317 µs; the two launches per column it replaced took 14.6 µs a
+// column.
 constexpr int kZP = 64;                 // panel width
 constexpr int kZPThreads = 512;
 constexpr int kZPRPL = 2;               // rows per lane
@@ -801,8 +804,8 @@ struct ZPanelP {
     int64_t lda;
     T *tau, *V, *Tm;
     int64_t ldv;
-    uint4 *xch;          // [kZP columns][P + 1][kZP] tagged complex values
-    unsigned tag0;       // tags tag0 + 1 … tag0 + kmax
+    T *xch, *xch_next;   // [kZP columns][entries][kZP] complex: this panel's, the next one's
+    int entries;         // workgroups' sums, the last entry row j
     unsigned spin_limit;
 };
 
@@ -831,7 +834,8 @@ template <typename T>
 __global__ __launch_bounds__(kZPThreads) void zqr_panel_kernel(ZPanelP<T> p)
 {
     constexpr int RPL = kZPRPL, NB = kZP, H = kZPThreads / NB;   // H = waves = 8
-    constexpr int EW = sizeof(T) / 4;                            // uint4 per complex value
+    typedef typename NaNMark<T>::bits B;
+    typedef T z2 __attribute__((ext_vector_type(2)));
     __shared__ T xs[2][kZPRows][2];
     __shared__ T red[H][NB][2];
     __shared__ T tot[NB][2], rowj[NB][2], rows[NB][2], scal[5];
@@ -852,15 +856,14 @@ __global__ __launch_bounds__(kZPThreads) void zqr_panel_kernel(ZPanelP<T> p)
             const bool ok = !tw && r < p.m && c0 + c < p.w;
             const T *src = p.A + 2 * ((ok ? r : 0) + (int64_t)(ok ? c0 + c : 0) * p.lda);
             const T re = src[0], im = src[1];
-            ar[c][q] = ok ? re : T(0);
-            ai[c][q] = ok ? im : T(0);
+            ar[c][q] = ok ? quiet(re) : T(0);
+            ai[c][q] = ok ? quiet(im) : T(0);
         }
     if (tw)
         for (int e = t; e < 2 * NB * NB; e += kZPThreads) Ts[e] = T(0);
 
     for (int j = 0; j < p.kmax; ++j) {
-        const unsigned tag = p.tag0 + (unsigned)j + 1;
-        uint4 *xb = p.xch + (size_t)j * (P + 1) * NB * EW;
+        T *xb = p.xch + 2 * (size_t)j * p.entries * NB;
         T xr[RPL], xi[RPL];
         if (!tw) {
             // (1) column j to LDS
@@ -908,9 +911,8 @@ __global__ __launch_bounds__(kZPThreads) void zqr_panel_kernel(ZPanelP<T> p)
             T z0, z1;
             wave_reduce16<T>(d, z0, z1);
             auto put = [&](int pp, int c, int cp, T v) {
-                uint4 *e = xb + ((size_t)pp * NB + c) * EW;
-                if constexpr (sizeof(T) == 8) tagged_store(e + cp, v, tag);
-                else tagged_store(reinterpret_cast<uint2 *>(e) + cp, v, tag);
+                store_coherent(reinterpret_cast<B *>(xb + 2 * ((size_t)pp * NB + c) + cp),
+                               __builtin_bit_cast(B, v));
             };
             if ((lane & 7) < 2)
                 put(wg, c0 + 4 * ((lane >> 4) & 1) + 2 * ((lane >> 3) & 1) + (lane & 1), lane >> 5,
@@ -924,7 +926,8 @@ __global__ __launch_bounds__(kZPThreads) void zqr_panel_kernel(ZPanelP<T> p)
                     }
                 }
                 __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
-                if (lane < 16) put(P, c0 + lane / 2, lane & 1, rows[c0 + lane / 2][lane & 1]);
+                if (lane < 16)
+                    put(p.entries - 1, c0 + lane / 2, lane & 1, rows[c0 + lane / 2][lane & 1]);
             }
         }
         // (3) wave h sums column `lane` over the workgroups ≡ h (mod 8); row j
@@ -933,57 +936,42 @@ __global__ __launch_bounds__(kZPThreads) void zqr_panel_kernel(ZPanelP<T> p)
             const int h = wv;
             const int cnt = h < P ? (P - h + H - 1) / H : 0;
             T sr = T(0), si = T(0);
-            constexpr int EB = 8 / EW;            // entries per batch of eight loads
             bool lost = false;
-            for (int i0 = 0; i0 == 0 || i0 < cnt; i0 += EB) {
-                const tagged4 *ptr[10];
-                tagged4 v[10];
+            for (int i0 = 0; i0 == 0 || i0 < cnt;) {
+                const z2 *ptr[5];
+                z2 v[5];
                 const bool row = h == H - 1 && i0 == 0;
+                const int eb = row ? 4 : 5;           // entries of this batch of five
                 auto entry = [&](int pp) {
-                    return reinterpret_cast<const tagged4 *>(xb + ((size_t)pp * NB + lane) * EW);
+                    return reinterpret_cast<const z2 *>(xb + 2 * ((size_t)pp * NB + lane));
                 };
-                // past the last: row j, whose words arrive as well
+                // past the last: row j, which arrives as well
 #pragma unroll
-                for (int u = 0; u < 8; ++u)
-                    ptr[u] = entry(i0 + u / EW < cnt ? h + (i0 + u / EW) * H : P) + u % EW;
-                ptr[8] = row ? entry(P) : ptr[0];
-                ptr[9] = row ? entry(P) + (EW - 1) : ptr[0];
+                for (int u = 0; u < 5; ++u)
+                    ptr[u] = entry(u < eb && i0 + u < cnt ? h + (i0 + u) * H : p.entries - 1);
                 unsigned spins = 0;
                 for (;;) {
-                    tagged_load10(ptr, v);
+                    load5_coherent(ptr, v);
                     bool ok = true;
 #pragma unroll
-                    for (int u = 0; u < 10; ++u) ok = ok && v[u][1] == tag && v[u][3] == tag;
+                    for (int u = 0; u < 5; ++u) ok = ok && !is_mark((T)v[u].x) && !is_mark((T)v[u].y);
                     if (__all(ok)) break;
                     if (++spins > p.spin_limit) {
                         lost = true;
                         break;
                     }
                 }
-                auto value = [&](int e, T &re, T &im) {
-                    if constexpr (sizeof(T) == 8) {
-                        re = tagged_value(v[e]);
-                        im = tagged_value(v[e + 1]);
-                    } else {
-                        re = __builtin_bit_cast(float, (unsigned)v[e][0]);
-                        im = __builtin_bit_cast(float, (unsigned)v[e][2]);
-                    }
-                };
 #pragma unroll
-                for (int e = 0; e < EB; ++e) {
-                    T re, im;
-                    value(e * EW, re, im);
-                    if (i0 + e < cnt) {
-                        sr += re;
-                        si += im;
+                for (int u = 0; u < 5; ++u)
+                    if (u < eb && i0 + u < cnt) {
+                        sr += v[u].x;
+                        si += v[u].y;
                     }
-                }
                 if (row) {
-                    T re, im;
-                    value(8, re, im);
-                    rowj[lane][0] = re;
-                    rowj[lane][1] = im;
+                    rowj[lane][0] = v[4].x;
+                    rowj[lane][1] = v[4].y;
                 }
+                i0 += eb;
             }
             // a wait that gave up makes the results NaN
             if (lost) sr = si = T(__builtin_nan(""));
@@ -1033,6 +1021,21 @@ __global__ __launch_bounds__(kZPThreads) void zqr_panel_kernel(ZPanelP<T> p)
             }
         }
         lds_barrier();
+        // the next panel's slot of this column, for that panel: nobody
+        // reads it before then
+        if (wv == 5) {
+            B *mk = reinterpret_cast<B *>(p.xch_next + 2 * ((size_t)j * p.entries + wg) * NB);
+            if (!tw) {
+                store_coherent(mk + 2 * lane, NaNMark<T>::value);
+                store_coherent(mk + 2 * lane + 1, NaNMark<T>::value);
+            }
+            if (wg == 0) {
+                B *mr = reinterpret_cast<B *>(
+                    p.xch_next + 2 * ((size_t)j * p.entries + p.entries - 1) * NB);
+                store_coherent(mr + 2 * lane, NaNMark<T>::value);
+                store_coherent(mr + 2 * lane + 1, NaNMark<T>::value);
+            }
+        }
         const T fr = scal[0], fi = scal[1], taur = scal[2], taui = scal[3], nu = scal[4];
         const bool live = nu != T(0);
         if (tw) {
@@ -1127,11 +1130,12 @@ __global__ __launch_bounds__(kZPThreads) void zqr_panel_kernel(ZPanelP<T> p)
     }
 }
 
-// Clears the tagged words of the exchange.
-__global__ void zqr_clear_kernel(uint4 *x, int64_t n)
+// Fills the exchange with marks.
+template <typename T>
+__global__ void zqr_clear_kernel(T *x, int64_t n)
 {
     const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < n) x[i] = uint4{0u, 0u, 0u, 0u};
+    if (i < n) reinterpret_cast<typename NaNMark<T>::bits *>(x)[i] = NaNMark<T>::value;
 }
 
 // V (m×k, ld ldv): the unit lower reflectors of F explicitly (ones on the
@@ -1292,13 +1296,13 @@ inline int64_t zqr_part_elems(int64_t n) { return 2 * 16 * (int64_t)kZQ * std::m
 
 // Workspace of zqr_blocked_dev in elements of T, every part on 32 elements:
 // two (V, T) panel sets and two (W1, W2, split-K) update sets, since the side
-// stream updates with one while the next panel fills the other; the tagged
+// stream updates with one while the next panel fills the other; the panels'
 // exchange.
 template <typename T>
 struct ZqrWS {
     T *V[2], *Tm[2], *W1[2], *W2[2], *part[2];
-    uint4 *xch;
-    int64_t part_elems, xch_words;
+    T *xch;               // two sets of slots, for alternate panels
+    int64_t part_elems, xch_elems;
     size_t elems;
     ZqrWS(T *base, int64_t m, int64_t n)
     {
@@ -1317,8 +1321,8 @@ struct ZqrWS {
             W2[q] = take(2 * (size_t)kZP * n);
             part[q] = take((size_t)part_elems);
         }
-        xch_words = kZP * (P + 1) * kZP * (int64_t)(sizeof(T) / 4);
-        xch = reinterpret_cast<uint4 *>(take((size_t)xch_words * (16 / sizeof(T))));
+        xch_elems = 2 * kZP * (P + 1) * kZP;
+        xch = take(2 * (size_t)xch_elems);
         elems = off;
     }
 };
@@ -1327,7 +1331,7 @@ struct ZqrWS {
 // whatever the block size (the factors do not depend on it): the panel and
 // its T by one launch, then Hᴴ on the next block column, on which the next
 // panel starts while the side stream applies Hᴴ to the rest (depth-1
-// look-ahead, as qr_blocked_dev).  4096×2048 ComplexF64: 12.8 ms (45.5 with
+// look-ahead, as qr_blocked_dev).  4096×2048 ComplexF64: 12.0 ms (45.5 with
 // 32-wide block columns, two launches per column and no look-ahead); the
 // chain of panels and next-block updates is what it takes.
 template <typename T>
@@ -1339,8 +1343,8 @@ int zqr_blocked_dev(Handle *h, hipStream_t s0, int64_t m, int64_t n, T *A, int64
     const bool la = h->qr_lookahead && cdiv(k, (int64_t)kZP) > 2;
     const bool masked = la && h->masked != nullptr;
     hipStream_t s = masked ? h->chain : s0, side = masked ? h->masked : h->side;
-    hipLaunchKernelGGL(zqr_clear_kernel, dim3((unsigned)cdiv(ws.xch_words, 256)), dim3(256), 0, s0,
-                       ws.xch, ws.xch_words);
+    hipLaunchKernelGGL((zqr_clear_kernel<T>), dim3((unsigned)cdiv(2 * ws.xch_elems, 256)), dim3(256),
+                       0, s0, ws.xch, 2 * ws.xch_elems);
     GLA_LAUNCH_CHECK();
     if (la) {
         GLA_HIP_TRY(hipEventRecord(h->ev_fork, s0));
@@ -1361,8 +1365,9 @@ int zqr_blocked_dev(Handle *h, hipStream_t s0, int64_t m, int64_t n, T *A, int64
         p.V = ws.V[q];
         p.ldv = mm;
         p.Tm = ws.Tm[q];
-        p.xch = ws.xch;
-        p.tag0 = (unsigned)off;
+        p.xch = ws.xch + q * ws.xch_elems;
+        p.xch_next = ws.xch + (1 - q) * ws.xch_elems;
+        p.entries = (int)cdiv(m, kZPRows) + 1;
         p.spin_limit = h->spin_limit;
         hipLaunchKernelGGL((zqr_panel_kernel<T>), dim3((unsigned)cdiv(mm, kZPRows) + 1),
                            dim3(kZPThreads), 0, s, p);

@@ -169,54 +169,34 @@ __device__ __forceinline__ void load9_coherent(const float *const p[8], float v[
 // included, have completed (s_waitcnt vmcnt(0)).
 __device__ __forceinline__ void stores_done() { __builtin_amdgcn_s_waitcnt(0x0F70); }
 
-// Values published together with a tag, so that one round trip brings the
-// value and the proof that it has arrived: each 32-bit part of the value
-// shares an 8-byte word (written and read whole) with the tag.  A double
-// takes 16 bytes, a float 8; a reader polls until every word carries the
-// tag it expects.  Buffers are cleared before the first use and a tag is
-// used once, so no word of an earlier exchange can pass.
-__device__ __forceinline__ void tagged_store(uint4 *p, double v, unsigned tag)
-{
-    const uint2 u = __builtin_bit_cast(uint2, v);
-    typedef unsigned u4 __attribute__((ext_vector_type(4)));
-    const u4 w = {u.x, tag, u.y, tag};
-    // the s_nop keeps the data registers unwritten for the cycle a store of
-    // over 8 bytes needs them
-    asm volatile("global_store_dwordx4 %0, %1, off sc1\n\ts_nop 1" ::"v"(p), "v"(w) : "memory");
-}
-__device__ __forceinline__ void tagged_store(uint2 *p, float v, unsigned tag)
-{
-    const unsigned long long w =
-        ((unsigned long long)tag << 32) | __builtin_bit_cast(unsigned, v);
-    store_coherent(reinterpret_cast<unsigned long long *>(p), w);
-}
-typedef unsigned tagged4 __attribute__((ext_vector_type(4)));   // two tagged words
-
-// Ten 16-byte tagged words in flight at once, then one wait: a batch of
-// eight and two of a row that travels with it.
-__device__ __forceinline__ void tagged_load10(const tagged4 *const p[10], tagged4 v[10])
+// Five complex values (16 or 8 bytes each) in flight at once, then one wait.
+typedef double zd2 __attribute__((ext_vector_type(2)));
+typedef float zf2 __attribute__((ext_vector_type(2)));
+__device__ __forceinline__ void load5_coherent(const zd2 *const p[5], zd2 v[5])
 {
     asm volatile(
-        "global_load_dwordx4 %0, %10, off sc1\n\t"
-        "global_load_dwordx4 %1, %11, off sc1\n\t"
-        "global_load_dwordx4 %2, %12, off sc1\n\t"
-        "global_load_dwordx4 %3, %13, off sc1\n\t"
-        "global_load_dwordx4 %4, %14, off sc1\n\t"
-        "global_load_dwordx4 %5, %15, off sc1\n\t"
-        "global_load_dwordx4 %6, %16, off sc1\n\t"
-        "global_load_dwordx4 %7, %17, off sc1\n\t"
-        "global_load_dwordx4 %8, %18, off sc1\n\t"
-        "global_load_dwordx4 %9, %19, off sc1\n\t"
+        "global_load_dwordx4 %0, %5, off sc1\n\t"
+        "global_load_dwordx4 %1, %6, off sc1\n\t"
+        "global_load_dwordx4 %2, %7, off sc1\n\t"
+        "global_load_dwordx4 %3, %8, off sc1\n\t"
+        "global_load_dwordx4 %4, %9, off sc1\n\t"
         "s_waitcnt vmcnt(0)"
-        : "=&v"(v[0]), "=&v"(v[1]), "=&v"(v[2]), "=&v"(v[3]), "=&v"(v[4]), "=&v"(v[5]),
-          "=&v"(v[6]), "=&v"(v[7]), "=&v"(v[8]), "=&v"(v[9])
-        : "v"(p[0]), "v"(p[1]), "v"(p[2]), "v"(p[3]), "v"(p[4]), "v"(p[5]), "v"(p[6]), "v"(p[7]),
-          "v"(p[8]), "v"(p[9])
+        : "=&v"(v[0]), "=&v"(v[1]), "=&v"(v[2]), "=&v"(v[3]), "=&v"(v[4])
+        : "v"(p[0]), "v"(p[1]), "v"(p[2]), "v"(p[3]), "v"(p[4])
         : "memory");
 }
-__device__ __forceinline__ double tagged_value(const tagged4 &w)
+__device__ __forceinline__ void load5_coherent(const zf2 *const p[5], zf2 v[5])
 {
-    return __builtin_bit_cast(double, uint2{w[0], w[2]});
+    asm volatile(
+        "global_load_dwordx2 %0, %5, off sc1\n\t"
+        "global_load_dwordx2 %1, %6, off sc1\n\t"
+        "global_load_dwordx2 %2, %7, off sc1\n\t"
+        "global_load_dwordx2 %3, %8, off sc1\n\t"
+        "global_load_dwordx2 %4, %9, off sc1\n\t"
+        "s_waitcnt vmcnt(0)"
+        : "=&v"(v[0]), "=&v"(v[1]), "=&v"(v[2]), "=&v"(v[3]), "=&v"(v[4])
+        : "v"(p[0]), "v"(p[1]), "v"(p[2]), "v"(p[3]), "v"(p[4])
+        : "memory");
 }
 
 }  // namespace gla
