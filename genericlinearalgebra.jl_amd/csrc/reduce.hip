@@ -1307,12 +1307,6 @@ __global__ __launch_bounds__(512, 4) void bd_resident_kernel(BdResP<T> q)
         const T nu = copysign(nrm, xi_), xi = xi_ + nu;
         const T tau = live ? xi / nu : T(0), rxi = live ? T(1) / xi : T(1);
         if (t < kBRLoc) {
-            // the grid column's peers are done with the previous step's sums
-            if (i > 0) {
-                T *old = q.e1 + ((i + 2) % 3) * slot + ((int64_t)gc * PR + gr) * kBRBlk;
-                mark(old + t);
-                if (t == 0) mark(old + kBRLoc);
-            }
             const int c = gc + PC * t;
             const T d = (gsum[0][t] + gsum[1][t]) + (gsum[2][t] + gsum[3][t]);
             const bool in = c > i && c < n;
@@ -1326,6 +1320,13 @@ __global__ __launch_bounds__(512, 4) void bd_resident_kernel(BdResP<T> q)
         } else if (t < 2 * kBRLoc) {
             const int r = gr + PR * tl;
             V[tl] = r > i ? X[tl] * rxi : (r == i ? T(1) : T(0));
+        }
+        // the grid column's peers are done with the previous step's sums (by
+        // waves with nothing else to do here)
+        if (i > 0 && t >= 2 * kBRLoc && t < 3 * kBRLoc) {
+            T *old = q.e1 + ((i + 2) % 3) * slot + ((int64_t)gc * PR + gr) * kBRBlk;
+            mark(old + tl);
+            if (tl == 0) mark(old + kBRLoc);
         }
         if (blockIdx.x == 0 && t == 0) q.taul[i] = tau;
         const T beta_l = live ? -nu : xi_;
@@ -1393,11 +1394,6 @@ __global__ __launch_bounds__(512, 4) void bd_resident_kernel(BdResP<T> q)
             const T nur = copysign(nrmr, zi), xir = zi + nur;
             const T taur = liver ? xir / nur : T(0), rxir = liver ? T(1) / xir : T(1);
             if (t < kBRLoc) {
-                if (i > 0) {
-                    T *old = q.e2 + ((i + 2) % 3) * slot + ((int64_t)gr * PC + gc) * kBRBlk;
-                    mark(old + t);
-                    if (t == 0) mark(old + kBRLoc);
-                }
                 const int r = gr + PR * t;
                 const T e = (gsum[0][t] + gsum[1][t]) + (gsum[2][t] + gsum[3][t]);
                 const bool in = r > i && r < m;
@@ -1411,6 +1407,11 @@ __global__ __launch_bounds__(512, 4) void bd_resident_kernel(BdResP<T> q)
             } else if (t < 2 * kBRLoc) {
                 const int c = gc + PC * tl;
                 Uv[tl] = c > i + 1 ? Z[tl] * rxir : (c == i + 1 ? T(1) : T(0));
+            }
+            if (i > 0 && t >= 2 * kBRLoc && t < 3 * kBRLoc) {
+                T *old = q.e2 + ((i + 2) % 3) * slot + ((int64_t)gr * PC + gc) * kBRBlk;
+                mark(old + tl);
+                if (tl == 0) mark(old + kBRLoc);
             }
             if (blockIdx.x == 0 && t == 0) q.taur[i] = taur;
             lds_barrier();
