@@ -1418,7 +1418,7 @@ int chol_device(Handle *h, hipStream_t s, int64_t n, T *A, int64_t lda, int algo
     bool df = false;
     if (h->chol_block < 0 && h->chol_df > 0 && n > kPanelNB) {
         const int64_t w = n <= h->chol_df ? n : auto_chol_block(n, true);
-        df = ensure_df(h, chol_df_bytes(n, w, sizeof(T)));
+        df = ensure_df(h, s, chol_df_bytes(n, w, sizeof(T)));
         if (df && w == n) return chol_df<T>(h, s, n, n, A, lda, 0, nullptr);
     }
     const int64_t NB = h->chol_block < 0 ? auto_chol_block(n, df) : h->chol_block;

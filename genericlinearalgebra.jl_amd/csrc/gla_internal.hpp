@@ -8,6 +8,7 @@
 #include <cstdint>
 #include <cstdio>
 #include <string>
+#include <vector>
 
 #include "gla_hip.h"
 
@@ -453,6 +454,8 @@ struct Handle {
     size_t ws_bytes = 0;
     void *df = nullptr;               // packed tiles of the dataflow Cholesky
     size_t df_bytes = 0;
+    bool df_captured = false;         // a graph holds df
+    std::vector<void *> df_kept;      // former ones that a graph holds
     int num_cus = 256;
     // Tuning: block width of the look-ahead driver behind cholRecursive!
     // (0: the recursive-halving driver; −1: chosen from n).  Set with
@@ -501,9 +504,10 @@ struct Handle {
 // Ensure the workspace holds at least `bytes` (grows with hipMalloc, which
 // synchronises the device; the first call of a given size pays for it).
 int ensure_workspace(Handle *h, size_t bytes);
-// The same for the dataflow Cholesky's buffer; false if it cannot be had
+// The same for the dataflow Cholesky's buffer; false if it cannot be had, or
+// would have to grow while stream s is being captured
 // (the caller then takes a path without it).
-bool ensure_df(Handle *h, size_t bytes);
+bool ensure_df(Handle *h, hipStream_t s, size_t bytes);
 
 // Launches whose workgroups wait for each other and take most of the chip
 // must not share it with another such launch: each could hold places the

@@ -38,11 +38,29 @@ int ensure_workspace(Handle *h, size_t bytes)
     return GLA_OK;
 }
 
-bool ensure_df(Handle *h, size_t bytes)
+bool ensure_df(Handle *h, hipStream_t s, size_t bytes)
 {
-    if (bytes <= h->df_bytes) return true;
+    // Neither the wait nor the allocation may fall into a capture, and a
+    // buffer that a graph holds stays until the handle goes: then the next is
+    // twice as large, so that those kept are together smaller than it.
+    hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+    const bool eager = hipStreamIsCapturing(s, &cap) == hipSuccess &&
+                       cap == hipStreamCaptureStatusNone;
+    if (!eager) (void)hipGetLastError();
+    if (bytes <= h->df_bytes) {
+        h->df_captured |= !eager;
+        return true;
+    }
+    if (!eager) return false;
     const size_t gran = size_t(16) << 20;
-    const size_t want = (bytes + gran - 1) / gran * gran;
+    size_t want = (bytes + gran - 1) / gran * gran;
+    if (h->df && h->df_captured) {
+        want = std::max(want, 2 * h->df_bytes);
+        h->df_kept.push_back(h->df);
+        h->df = nullptr;
+        h->df_bytes = 0;
+        h->df_captured = false;
+    }
     if (h->df) {
         // the old buffer may still be read by queued work
         if (hipDeviceSynchronize() != hipSuccess || hipFree(h->df) != hipSuccess) {
@@ -324,6 +342,7 @@ int gla_handle_destroy(gla_handle_t hh)
     GLA_HIP_TRY(hipDeviceSynchronize());
     if (h->ws) (void)hipFree(h->ws);
     if (h->df) (void)hipFree(h->df);
+    for (void *p : h->df_kept) (void)hipFree(p);
     if (h->dinfo) (void)hipFree(h->dinfo);
     if (h->dbar) (void)hipFree(h->dbar);
     (void)hipEventDestroy(h->ev_fork);
