@@ -796,6 +796,19 @@ constexpr int kZPRPL = 2;               // rows per lane
 constexpr int kZPRows = 64 * kZPRPL;    // rows per workgroup
 constexpr int kZPMaxP = 127;            // workgroups with rows: beyond, the launches per column
 
+// ‖x‖² for which |ξ|², at most four times as much, and its reciprocal are normal
+// numbers (the hardware estimates are not good for others).
+template <typename T>
+struct ZRange;
+template <>
+struct ZRange<double> {
+    static constexpr double lo = 0x1p-1000, hi = 0x1p1000;
+};
+template <>
+struct ZRange<float> {
+    static constexpr float lo = 0x1p-100f, hi = 0x1p100f;
+};
+
 template <typename T>
 struct ZPanelP {
     int64_t m;
@@ -981,9 +994,9 @@ __global__ __launch_bounds__(kZPThreads) void zqr_panel_kernel(ZPanelP<T> p)
         }
         // (4) wave 0, lane c: the total of column c and the reflector from
         // column j's: ν = copysign(‖x‖, Re x_j), ξ = x_j + ν, τ = ξ/ν, the
-        // divisions by ξ and ν as products with their reciprocals; then the
-        // column's coefficient τ̄ (a_jc + d_c/ξ̄), or for a finished column
-        // g_c = v_cᴴ v_j
+        // divisions by ξ and ν as products with their reciprocals where all
+        // are normal numbers; then the column's coefficient
+        // τ̄ (a_jc + d_c/ξ̄), or for a finished column g_c = v_cᴴ v_j
         if (wv == 0) {
             T dr = T(0), di = T(0);
 #pragma unroll
@@ -993,14 +1006,32 @@ __global__ __launch_bounds__(kZPThreads) void zqr_panel_kernel(ZPanelP<T> p)
             }
             const T br = rowj[lane][0], bi = rowj[lane][1];
             const T xjr = lane_value(br, j), xji = lane_value(bi, j), s = lane_value(dr, j);
-            T nrm, rn;
-            sqrt_and_rsqrt(xjr * xjr + xji * xji + s, nrm, rn);
-            const bool alive = nrm != T(0);
-            const T nv = copysign(nrm, xjr), rnu = copysign(rn, xjr);
-            const T er = xjr + nv, ei = xji;
-            const T den = recip_step(er * er + ei * ei);                // 1/ξ = ξ̄/|ξ|²
-            const T f_r = alive ? er * den : T(0), f_i = alive ? -ei * den : T(0);
-            const T tr = alive ? er * rnu : T(0), ti = alive ? ei * rnu : T(0);
+            const T nrm2 = xjr * xjr + xji * xji + s;
+            const bool alive = nrm2 != T(0);
+            T nv, f_r, f_i, tr, ti;
+            if (nrm2 >= ZRange<T>::lo && nrm2 <= ZRange<T>::hi) {
+                T nrm, rn;
+                sqrt_and_rsqrt(nrm2, nrm, rn);
+                nv = copysign(nrm, xjr);
+                const T rnu = copysign(rn, xjr), er = xjr + nv, ei = xji;
+                const T den = recip_step(er * er + ei * ei);            // 1/ξ = ξ̄/|ξ|²
+                f_r = er * den;
+                f_i = -ei * den;
+                tr = er * rnu;
+                ti = ei * rnu;
+            } else {
+                // |ξ|² or its reciprocal may leave the range: ξ by a power of
+                // two to 1…4 first, and square root and division as they are
+                const T nrm = sqrt(nrm2);
+                nv = copysign(nrm, xjr);
+                const T er = xjr + nv, ei = xji;
+                const int e = alive ? -ilogb(nrm) : 0;
+                const T zr = ldexp(er, e), zi = ldexp(ei, e), den = zr * zr + zi * zi;
+                f_r = alive ? ldexp(zr / den, e) : T(0);
+                f_i = alive ? ldexp(-zi / den, e) : T(0);
+                tr = alive ? er / nv : T(0);
+                ti = alive ? ei / nv : T(0);
+            }
             T kr, ki;
             if (lane < j) {
                 kr = br + (dr * f_r + di * f_i);        // conj(a_jc) + conj(d_c)/ξ
