@@ -1415,11 +1415,14 @@ int chol_device(Handle *h, hipStream_t s, int64_t n, T *A, int64_t lda, int algo
     // cholRecursive!: the reference recurses to 1×1 (cutoff does not reach
     // the A11 branch, :46); on the device the recursion stops at a leaf of
     // at least 2048 (or `cutoff` if larger) that the blocked driver factors.
+    // (an order above a lowered chol_df that one block column would hold takes
+    // the drivers without the buffer)
     bool df = false;
     if (h->chol_block < 0 && h->chol_df > 0 && n > kPanelNB) {
-        const int64_t w = n <= h->chol_df ? n : auto_chol_block(n, true);
-        df = ensure_df(h, s, chol_df_bytes(n, w, sizeof(T)));
-        if (df && w == n) return chol_df<T>(h, s, n, n, A, lda, 0, nullptr);
+        const bool whole = n <= h->chol_df;
+        const int64_t w = whole ? n : auto_chol_block(n, true);
+        df = (whole || w < n) && ensure_df(h, s, chol_df_bytes(n, w, sizeof(T)));
+        if (df && whole) return chol_df<T>(h, s, n, n, A, lda, 0, nullptr);
     }
     const int64_t NB = h->chol_block < 0 ? auto_chol_block(n, df) : h->chol_block;
     if (NB > kPanelNB) return chol_la_dev<T>(h, s, n, A, lda, (int)NB, 0, Linv, df);

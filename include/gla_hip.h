@@ -71,8 +71,8 @@ const char *gla_version(void);
  * 3072, then 256, 512 from 10240, 1024 from 14336).  All compute the same
  * factor up to rounding.  "chol_df": largest order (default 8192, at most
  * 8192) that cholRecursive! factors in one dataflow launch; larger ones take
- * 3072- or 2048-wide block columns of one such launch each; 0 turns both
- * off.  The handle keeps the launch's tile buffer (266 MB at n = 8192 in
+ * 3072- or 2048-wide block columns of one such launch each (those up to 3072
+ * the drivers without its buffer); 0 turns both off.  The handle keeps the launch's tile buffer (266 MB at n = 8192 in
  * FP64), which only grows; if it cannot be allocated the other drivers run.  "chol_psolve": 1 (default) solves each
  * look-ahead panel up to 768 wide in one launch (every 64 rows sweep the
  * 128-wide column blocks), 0 by the recursive rdiv!.  "chol_syrk_late": 1 (default) starts the look-ahead
