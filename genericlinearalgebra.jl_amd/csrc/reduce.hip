@@ -1186,7 +1186,7 @@ __global__ __launch_bounds__(512, 4) void bd_resident_kernel(BdResP<T> q)
             }
         if (t < kBRLoc) {
             const int r = gr + PR * t;
-            const T v = q.A[r < m ? r : 0];
+            const T v = quiet(q.A[r < m ? r : 0]);      // x_0 is published as it is
             const T x = r < m && r > 0 ? v : T(0);
             X[t] = x;
             if (r == 0) xpiv = v;
