@@ -820,6 +820,7 @@ struct ZPanelP {
     T *xch, *xch_next;   // [kZP columns][entries][kZP] complex: this panel's, the next one's
     int entries;         // workgroups' sums, the last entry row j
     unsigned spin_limit;
+    int never;           // (a test) no arrival counts
 };
 
 // Sums of v[0…15] over the wave: lane l returns, for its group of eight
@@ -875,6 +876,7 @@ __global__ __launch_bounds__(kZPThreads) void zqr_panel_kernel(ZPanelP<T> p)
     if (tw)
         for (int e = t; e < 2 * NB * NB; e += kZPThreads) Ts[e] = T(0);
 
+    bool lost = false;
     for (int j = 0; j < p.kmax; ++j) {
         T *xb = p.xch + 2 * (size_t)j * p.entries * NB;
         T xr[RPL], xi[RPL];
@@ -949,7 +951,6 @@ __global__ __launch_bounds__(kZPThreads) void zqr_panel_kernel(ZPanelP<T> p)
             const int h = wv;
             const int cnt = h < P ? (P - h + H - 1) / H : 0;
             T sr = T(0), si = T(0);
-            bool lost = false;
             for (int i0 = 0; i0 == 0 || i0 < cnt;) {
                 const z2 *ptr[5];
                 z2 v[5];
@@ -968,11 +969,8 @@ __global__ __launch_bounds__(kZPThreads) void zqr_panel_kernel(ZPanelP<T> p)
                     bool ok = true;
 #pragma unroll
                     for (int u = 0; u < 5; ++u) ok = ok && !is_mark((T)v[u].x) && !is_mark((T)v[u].y);
-                    if (__all(ok)) break;
-                    if (++spins > p.spin_limit) {
-                        lost = true;
-                        break;
-                    }
+                    if (lost || (__all(ok) && !p.never)) break;
+                    lost = ++spins > p.spin_limit;
                 }
 #pragma unroll
                 for (int u = 0; u < 5; ++u)
@@ -986,7 +984,7 @@ __global__ __launch_bounds__(kZPThreads) void zqr_panel_kernel(ZPanelP<T> p)
                 }
                 i0 += eb;
             }
-            // a wait that gave up makes the results NaN
+            // a wait that gave up makes the results NaN, and there are no more
             if (lost) sr = si = T(__builtin_nan(""));
             red[h][lane][0] = sr;
             red[h][lane][1] = si;
@@ -1400,6 +1398,7 @@ int zqr_blocked_dev(Handle *h, hipStream_t s0, int64_t m, int64_t n, T *A, int64
         p.xch_next = ws.xch + (1 - q) * ws.xch_elems;
         p.entries = (int)cdiv(m, kZPRows) + 1;
         p.spin_limit = h->spin_limit;
+        p.never = h->qr_wait_test;
         hipLaunchKernelGGL((zqr_panel_kernel<T>), dim3((unsigned)cdiv(mm, kZPRows) + 1),
                            dim3(kZPThreads), 0, s, p);
         GLA_LAUNCH_CHECK();

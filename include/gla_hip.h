@@ -108,9 +108,10 @@ const char *gla_version(void);
  * FP64 128×128 tiles through one LDS buffer, 0 through two.  Same results
  * bit for bit in every setting.  "spin_limit": polls (default 2^25, about a
  * second) before a wait of the dataflow Cholesky or a grid-wide wait of the QR panel gives up and the call
- * returns GLA_ERR_TIMEOUT.  "qr_wait_test": 1 makes every such wait target
- * an arrival count that never comes (a test of the timeout report; the
- * kernels still finish, after spin_limit polls per wait). */
+ * returns GLA_ERR_TIMEOUT.  "qr_wait_test": 1 makes every wait of a QR
+ * panel, real or complex, one for an arrival that never comes (a test of
+ * waits that give up; the kernels still finish, after spin_limit polls per
+ * wait, the complex panel's after those of one). */
 int gla_set_tuning(gla_handle_t h, const char *key, int64_t value);
 /* Reads a tuning knob's current value, by the same keys.  No counterpart
  * in the reference. */
