@@ -1360,15 +1360,18 @@ struct ZqrWS {
 // whatever the block size (the factors do not depend on it): the panel and
 // its T by one launch, then Hᴴ on the next block column, on which the next
 // panel starts while the side stream applies Hᴴ to the rest (depth-1
-// look-ahead, as qr_blocked_dev).  4096×2048 ComplexF64: 12.0 ms (45.5 with
+// look-ahead, as qr_blocked_dev).  4096×2048 ComplexF64: 11.7 ms (45.5 with
 // 32-wide block columns, two launches per column and no look-ahead); the
 // chain of panels and next-block updates is what it takes.
+// A panel takes a CU per workgroup (150 registers, FP64), half the chip: two
+// fit beside each other, three or one beside another resident launch need not.
+// The whole call is one link of the device's chain (resident_begin): a link per
+// panel would let other calls' products in between, at two events a panel.
 template <typename T>
 int zqr_blocked_dev(Handle *h, hipStream_t s0, int64_t m, int64_t n, T *A, int64_t lda, T *tau)
 {
     const int64_t k = std::min(m, n);
-    GLA_TRY(ensure_workspace(h, ZqrWS<T>(nullptr, m, n).elems * sizeof(T)));
-    const ZqrWS<T> ws(reinterpret_cast<T *>(h->ws), m, n);
+    const ZqrWS<T> ws(reinterpret_cast<T *>(h->ws), m, n);   // zqr_entry has made it large enough
     const bool la = h->qr_lookahead && cdiv(k, (int64_t)kZP) > 2;
     const bool masked = la && h->masked != nullptr;
     hipStream_t s = masked ? h->chain : s0, side = masked ? h->masked : h->side;
@@ -1433,8 +1436,9 @@ int zqr_blocked_dev(Handle *h, hipStream_t s0, int64_t m, int64_t n, T *A, int64
     return GLA_OK;
 }
 
-// The same for matrices too tall for the panel's registers: block columns of
-// min(blocksize, 32), two launches per column (zqr_panel).
+// The same for matrices too tall for the panel's registers, and for a stream
+// under capture, whose replays nothing orders after other resident launches:
+// block columns of min(blocksize, 32), two launches per column (zqr_panel).
 template <typename T>
 int zqr_tall_dev(hipStream_t s, int64_t m, int64_t n, T *A, int64_t lda, int64_t bs, T *tau,
                     T *ws)
@@ -1495,11 +1499,16 @@ int zqr_entry(gla_handle_t hh, int64_t m, int64_t n, void *Av, int64_t lda, int6
     GLA_HIP_TRY(hipSetDevice(h->device));
     // the panel's workgroups must all be resident, and every one gathers from
     // all; up to 127 of them (16256 rows) hold rows
-    if (cdiv(m, kZPRows) <= std::min(kZPMaxP, h->num_cus / 2))
-        return zqr_blocked_dev<T>(h, reinterpret_cast<hipStream_t>(stream), m, n, A, lda, tau);
-    GLA_TRY(ensure_workspace(h, zqr_scratch(m, n) * sizeof(T)));
-    return zqr_tall_dev<T>(reinterpret_cast<hipStream_t>(stream), m, n, A, lda, bs, tau,
-                           reinterpret_cast<T *>(h->ws));
+    const bool fits = cdiv(m, kZPRows) <= std::min(kZPMaxP, h->num_cus / 2);
+    const hipStream_t s = reinterpret_cast<hipStream_t>(stream);
+    GLA_TRY(ensure_workspace(h, std::max(fits ? ZqrWS<T>(nullptr, m, n).elems : 0, zqr_scratch(m, n)) *
+                                    sizeof(T)));
+    if (fits && resident_begin(h, s)) {
+        const int rc = zqr_blocked_dev<T>(h, s, m, n, A, lda, tau);
+        const int end = resident_end(h, s);
+        return rc != GLA_OK ? rc : end;
+    }
+    return zqr_tall_dev<T>(s, m, n, A, lda, bs, tau, reinterpret_cast<T *>(h->ws));
 }
 
 template <typename T>
