@@ -512,13 +512,27 @@ bool ensure_df(Handle *h, hipStream_t s, size_t bytes);
 // Launches whose workgroups wait for each other and take most of the chip
 // must not share it with another such launch: each could hold places the
 // other waits for.  resident_begin makes stream s wait for the last of them on
-// the handle's device, from any stream and thread of the process;
-// resident_end marks the new one.  Between the two the caller queues its
-// launch; a lock is held meanwhile, so every begin is followed by its end.
+// the handle's device, from any stream and thread of the process, and for the
+// PanelCalls in flight; resident_end marks the new one.  Between the two the
+// caller queues its launch; a lock is held meanwhile, so every begin is followed by its end.
 // False (nothing held): the stream is being captured, where another stream's
 // launch cannot be waited for, or an event failed.
 bool resident_begin(Handle *h, hipStream_t s);
 int resident_end(Handle *h, hipStream_t s);
+// A call that queues panels with grid-wide waits and then waits for its stream:
+// they run beside one another, as many as fit (a panel of the QR takes up to
+// all CUs), but not beside a resident launch.  Made before the first launch;
+// queued() after the last; destroyed when the stream has been waited for.
+struct PanelCall {
+    PanelCall(Handle *h, hipStream_t s);
+    void queued();
+    ~PanelCall();
+    PanelCall(const PanelCall &) = delete;
+    hipStream_t s;
+    int device = -1;
+    bool is_queued = false;
+    PanelCall *link = nullptr;
+};
 
 // ------------------------------------------------------------------ GEMM --
 // C = alpha*op(A)*op(B) + beta*C  with op(A) M×K, op(B) K×N.

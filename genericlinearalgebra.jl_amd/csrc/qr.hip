@@ -1835,7 +1835,9 @@ int qr_entry(gla_handle_t hh, int64_t m, int64_t n, T *A, int64_t lda, int64_t b
     hipStream_t s = reinterpret_cast<hipStream_t>(stream);
     GLA_HIP_TRY(hipSetDevice(h->device));
     if (m == 0 || n == 0) return GLA_OK;
+    PanelCall panels(h, s);
     GLA_TRY(qr_blocked_dev<T>(h, s, m, n, A, lda, nb, tau, work, ldwork));
+    panels.queued();
     // a panel whose grid wait gave up has produced meaningless factors
     int timed_out = 0;
     GLA_HIP_TRY(hipMemcpyAsync(&timed_out, h->dinfo + 1, sizeof(int), hipMemcpyDeviceToHost, s));

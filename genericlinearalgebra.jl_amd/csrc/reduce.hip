@@ -399,9 +399,9 @@ __global__ __launch_bounds__(256) void tri_w_kernel(int64_t n, int64_t c, int j,
 // Each column has an exchange region of its own, filled beforehand with a
 // signalling-NaN pattern no arithmetic produces: a value is its own arrival
 // mark.  All workgroups must be resident: such launches follow one another on
-// a device (resident_begin) and take no more than half of a CU's registers,
-// so that the panel kernels, which wait within a launch too, keep their place
-// beside them.  A wait that gives up makes the result NaN.
+// a device, and run beside no QR panel, which waits within a launch too
+// (resident_begin).  Two workgroups fit on a CU.  A wait that gives up makes
+// the result NaN.
 // Bound: latency.  n = 2048 FP64: 10.4 ms, 5.1 µs a column (3.2 at n = 512),
 // about half of it the exchange; the three launches per column of the
 // deferred form took 38 ms.  With p and the row in index order (eight

@@ -1,4 +1,5 @@
 // Handle, workspace and error reporting of libgla_hip.so.
+#include <condition_variable>
 #include <cstdarg>
 #include <cstring>
 #include <mutex>
@@ -83,33 +84,50 @@ namespace {
 constexpr int kMaxDevices = 64;
 struct ResidentChain {
     std::mutex lock;
-    hipEvent_t last = nullptr;   // the last resident launch, once recorded
+    std::condition_variable turn;
+    hipEvent_t last = nullptr;             // the last resident launch, once recorded
+    hipEvent_t panels = nullptr;           // (reused for every stream waited for)
+    unsigned long next = 0, serving = 0;   // callers take turns in the order they come
+    int queueing = 0;                      // PanelCalls not yet queued
+    PanelCall *queued = nullptr;           // the queued ones, linked by `link`
 };
 ResidentChain g_resident[kMaxDevices];
+
+bool capturing(hipStream_t s)
+{
+    hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(s, &cap) == hipSuccess && cap == hipStreamCaptureStatusNone) return false;
+    (void)hipGetLastError();
+    return true;
+}
 }  // namespace
 
 bool resident_begin(Handle *h, hipStream_t s)
 {
-    if (h->device < 0 || h->device >= kMaxDevices) return false;
-    hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
-    if (hipStreamIsCapturing(s, &cap) != hipSuccess || cap != hipStreamCaptureStatusNone) {
-        (void)hipGetLastError();
-        return false;
-    }
+    if (h->device < 0 || h->device >= kMaxDevices || capturing(s)) return false;
     ResidentChain &c = g_resident[h->device];
-    c.lock.lock();
+    std::unique_lock<std::mutex> lk(c.lock);
+    const unsigned long mine = c.next++;
+    c.turn.wait(lk, [&] { return c.serving == mine && c.queueing == 0; });
     hipError_t e = hipSuccess;
-    if (!c.last) {
-        e = hipEventCreateWithFlags(&c.last, hipEventDisableTiming);
-        if (e != hipSuccess) c.last = nullptr;
-    } else {
-        e = hipStreamWaitEvent(s, c.last, 0);
+    for (hipEvent_t *ev : {&c.last, &c.panels})
+        if (!*ev && e == hipSuccess) {
+            e = hipEventCreateWithFlags(ev, hipEventDisableTiming);
+            if (e != hipSuccess) *ev = nullptr;
+        }
+    if (e == hipSuccess) e = hipStreamWaitEvent(s, c.last, 0);
+    for (const PanelCall *q = c.queued; q; q = q->link) {
+        if (e == hipSuccess) e = hipEventRecord(c.panels, q->s);
+        if (e == hipSuccess) e = hipStreamWaitEvent(s, c.panels, 0);
     }
     if (e != hipSuccess) {
         (void)hipGetLastError();
-        c.lock.unlock();
+        ++c.serving;
+        lk.unlock();
+        c.turn.notify_all();
         return false;
     }
+    lk.release();
     return true;
 }
 
@@ -117,9 +135,57 @@ int resident_end(Handle *h, hipStream_t s)
 {
     ResidentChain &c = g_resident[h->device];
     const hipError_t e = hipEventRecord(c.last, s);
+    ++c.serving;
     c.lock.unlock();
+    c.turn.notify_all();
     GLA_HIP_TRY(e);
     return GLA_OK;
+}
+
+PanelCall::PanelCall(Handle *h, hipStream_t stream) : s(stream)
+{
+    if (h->device < 0 || h->device >= kMaxDevices || capturing(s)) return;
+    device = h->device;
+    ResidentChain &c = g_resident[device];
+    std::unique_lock<std::mutex> lk(c.lock);
+    const unsigned long mine = c.next++;
+    c.turn.wait(lk, [&] { return c.serving == mine; });
+    ++c.serving;
+    ++c.queueing;
+    if (c.last && hipStreamWaitEvent(s, c.last, 0) != hipSuccess) (void)hipGetLastError();
+    lk.unlock();
+    c.turn.notify_all();
+}
+
+void PanelCall::queued()
+{
+    if (device < 0) return;
+    ResidentChain &c = g_resident[device];
+    {
+        std::lock_guard<std::mutex> lk(c.lock);
+        link = c.queued;
+        c.queued = this;
+        --c.queueing;
+    }
+    is_queued = true;
+    c.turn.notify_all();
+}
+
+PanelCall::~PanelCall()
+{
+    if (device < 0) return;
+    ResidentChain &c = g_resident[device];
+    {
+        std::lock_guard<std::mutex> lk(c.lock);
+        if (is_queued) {
+            PanelCall **at = &c.queued;
+            while (*at != this) at = &(*at)->link;
+            *at = link;
+        } else {
+            --c.queueing;
+        }
+    }
+    c.turn.notify_all();
 }
 
 namespace {
