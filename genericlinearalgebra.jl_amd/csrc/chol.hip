@@ -1375,7 +1375,7 @@ GLA_INST_BLOCKS(float)
 // Driver of cholRecursive! for chol_block −1 (the default), from sweeps on
 // MI355X (ms, copy of A included; FP64 | FP32):
 //                                       n = 1000   5001       8192       12288      16384
-//   whole matrix in one dataflow launch  0.21|0.18  1.50|1.01  4.65|2.59
+//   whole matrix in one dataflow launch  0.21|0.18  1.52|0.99  4.72|2.48
 //   look-ahead, 3072-wide dataflow                             4.81|2.87  12.9|7.33  28.4|15.9
 //   look-ahead, 2048-wide dataflow                             4.89|2.99  13.3|7.55  27.6|15.5
 //   a launch per 128-wide step           0.53|0.49  3.37|3.05  7.38|5.65  16.9|11.7  33.2|21.9

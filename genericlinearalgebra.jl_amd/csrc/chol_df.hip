@@ -14,18 +14,22 @@
 // diagonal tile its L.
 //
 // Order and progress: tiles are numbered by columns, diagonal tile first, and
-// a tile reads tiles of smaller numbers only.  Workgroups start in order of
-// their number, so the unfinished one with the smallest number always has a
-// place and everything it waits for; the launch needs no more workgroups
-// resident than fit.  Every wait is bounded by spin_limit polls and reports
-// −1 in *info.
+// a tile reads tiles of smaller numbers only.  A workgroup takes its number by
+// a ticket when it starts, so whatever else runs on the device the unfinished
+// tile with the smallest number is always one that is running, and has
+// everything it waits for; the launch needs no more workgroups resident than
+// fit.  (Numbers by blockIdx, which would hold for a launch that has the device
+// to itself, spread the tiles better: FP64 n = 5001 1.45 ms, 8192 4.56.  By
+// ticket 1.57 and 4.84, and with the diagonal tiles' waves, which the chain
+// goes through, at a higher priority 1.52 and 4.72.)
+// Every wait is bounded by spin_limit polls and reports −1 in *info.
 //
 // Bound: for small n the chain along the diagonal, per 64 columns the tile
 // factor of four 16×16 tiles (≈7 µs), one flag and tile exchange between
 // workgroups (≈2 µs) and the 64-wide solve and update (≈2 µs): FP64 n = 1000
 // takes 0.21 ms (0.53 ms with a launch per factor, solve and update of 128
 // columns).  For large n the products, at about half the MFMA rate (n = 8192
-// FP64: 4.65 ms, 39 TFLOP/s): three workgroups per CU cover each other's
+// FP64: 4.72 ms, 39 TFLOP/s): three workgroups per CU cover each other's
 // waits, which is why a slab is 16 columns (53 KB of LDS); with 32-column
 // slabs and two workgroups per CU n = 8192 took 5.07 ms.  Coherent or plain
 // operand loads took the same time, so the coherent ones stay.
@@ -57,6 +61,7 @@ struct DfP {
     T *L;                 // packed diagonal tiles
     int *prog;            // per tile row: finished tiles left of the diagonal
     int *ldone;           // per tile column: 1 when L(j, j) is published
+    int *ticket;          // workgroups started
     int *info;
     int64_t info_base;
     T *LinvG;             // 16×16 tile inverses, row-major (optional)
@@ -303,7 +308,10 @@ __global__ __launch_bounds__(kDThreads, sizeof(T) == 8 ? 3 : 4) void chol_df_ker
     const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
 
     // this workgroup's tile: column j, then the diagonal tile or row i
-    int j = 0, id = blockIdx.x;
+    __shared__ int place;
+    if (threadIdx.x == 0) place = atomicAdd(p.ticket, 1);
+    lds_barrier();
+    int j = 0, id = __builtin_amdgcn_readfirstlane(place);
     for (; j < p.nt; ++j) {
         const int c = 1 + p.mt - (j + 1 < p.nt ? j + 2 : j + 1);
         if (id < c) break;
@@ -313,6 +321,7 @@ __global__ __launch_bounds__(kDThreads, sizeof(T) == 8 ? 3 : 4) void chol_df_ker
     const int i = diag ? j : id + (j + 1 < p.nt ? j + 1 : j);
     const int jo = diag ? j - 1 : j;                  // the column of acc and of operand X(jo, k)
     const int nk = diag ? (j > 0 ? j - 1 : 0) : j;    // products of 64 columns
+    if (diag) __builtin_amdgcn_s_setprio(3);          // the chain goes through it
 
     acc_t acc[4], c[3], dg;
 #pragma unroll
@@ -467,7 +476,7 @@ __global__ __launch_bounds__(kDThreads, sizeof(T) == 8 ? 3 : 4) void chol_df_ker
     if (jo >= 0) store_strip<T>(p, i, jo, w, acc);
 }
 
-// Clears the counters and flags of one launch.
+// Clears the counters, flags and ticket of one launch.
 __global__ void df_clear_kernel(int *f, int n)
 {
     const int e = blockIdx.x * blockDim.x + threadIdx.x;
@@ -480,7 +489,7 @@ size_t chol_df_bytes(int64_t m, int64_t n, size_t esz)
 {
     const int64_t mt = cdiv(m, kDT), nt = cdiv(n, kDT);
     return (size_t)(nt * (nt - 1) / 2 + (mt - nt) * nt) * kTE * esz + (size_t)nt * kLE * esz +
-           (size_t)(mt + nt) * sizeof(int) + 256;
+           (size_t)(mt + nt + 1) * sizeof(int) + 256;
 }
 
 // The factor of the m×n block column at A.  h->df holds the packed copies;
@@ -507,11 +516,12 @@ int chol_df(Handle *h, hipStream_t s, int64_t m, int64_t n, T *A, int64_t lda, i
     p.L = p.X + tiles * kTE;
     p.prog = reinterpret_cast<int *>(p.L + (int64_t)p.nt * kLE);
     p.ldone = p.prog + p.mt;
+    p.ticket = p.ldone + p.nt;
     p.info = h->dinfo;
     p.info_base = info_base;
     p.LinvG = LinvG;
     p.spin_limit = h->spin_limit;
-    const int nf = p.mt + p.nt;
+    const int nf = p.mt + p.nt + 1;
     hipLaunchKernelGGL(df_clear_kernel, dim3((unsigned)cdiv(nf, 256)), dim3(256), 0, s, p.prog, nf);
     GLA_LAUNCH_CHECK();
     // one workgroup per tile, the left neighbour of each diagonal tile but
