@@ -22,7 +22,10 @@
 // to itself, spread the tiles better: FP64 n = 5001 1.45 ms, 8192 4.56.  By
 // ticket 1.57 and 4.84, and with the diagonal tiles' waves, which the chain
 // goes through, at a higher priority 1.52 and 4.72.)
-// Every wait is bounded by spin_limit polls and reports −1 in *info.
+// Every wait is bounded by spin_limit polls; one that gives up puts −1 in *info
+// before its workgroup publishes anything.  A workgroup looks there after its
+// own waits, and when it finds −1 leaves NaN for its tile: whatever was formed
+// from data that had not come, at any remove, is NaN in the matrix.
 //
 // Bound: for small n the chain along the diagonal, per 64 columns the tile
 // factor of four 16×16 tiles (≈7 µs), one flag and tile exchange between
@@ -424,6 +427,7 @@ __global__ __launch_bounds__(kDThreads, sizeof(T) == 8 ? 3 : 4) void chol_df_ker
         }
     }
 
+    int state = 0;
     // X = acc L(jo, jo)⁻ᵀ
     T *Ls = buf;                                      // 2560 elements
     T *Xr = buf + kLE;                                // 4096: the solved tile
@@ -433,6 +437,7 @@ __global__ __launch_bounds__(kDThreads, sizeof(T) == 8 ? 3 : 4) void chol_df_ker
         stage<T>(p.L + (int64_t)jo * kLE, Ls, kLE);
         stores_done();
         lds_barrier();
+        state = load_coherent(p.info);                // (looked at in the end)
         solve_strip<T>(Ls, acc);
         if (i < p.nt || jo + 1 < p.nt) {              // someone reads it
             T *xp = x_tile<T>(p, i, jo);
@@ -472,6 +477,17 @@ __global__ __launch_bounds__(kDThreads, sizeof(T) == 8 ? 3 : 4) void chol_df_ker
         // Ls is free: every wave is past its solve (the barrier above; j = 0 has none)
         static_assert(256 + 2 * 16 * kXLD + 2 * 768 <= kLE, "LDS regions");
         factor_diag<T>(p, j, w, c, dg, buf, buf + 256, buf + 256 + 2 * 16 * kXLD);
+    }
+    if (__builtin_amdgcn_readfirstlane(state) < 0) {
+        const T nan = T(__builtin_nan(""));
+#pragma unroll
+        for (int b = 0; b < 4; ++b) acc[b] = acc_t{nan, nan, nan, nan};
+        // (the diagonal tile is in the matrix: factor_diag ended with its stores)
+        if (diag)
+            for (int e = threadIdx.x; e < kTE; e += kDThreads) {
+                const int64_t r = (int64_t)j * kDT + e % kDT, cc = (int64_t)j * kDT + e / kDT;
+                if (r < p.n && cc <= r) p.A[r + cc * p.lda] = nan;
+            }
     }
     if (jo >= 0) store_strip<T>(p, i, jo, w, acc);
 }
