@@ -96,7 +96,12 @@ __global__ void first_zero_diag_k(int64_t n, const T *R, int64_t ldr, int *info)
     if (i < n && R[i + i * ldr] == T(0)) atomicMin(info, (int)(i + 1));
 }
 
-__global__ void set_int_k(int *p, int v) { *p = v; }
+// info: the first zero of the diagonal, and whether a wait has given up
+__global__ void set_info_k(int *p, int v)
+{
+    p[0] = v;
+    p[1] = 0;
+}
 
 // S (rows×cols, ld lds) = 0.
 template <typename T>
@@ -329,8 +334,9 @@ size_t qr_solve_scratch(int64_t m, int64_t n, int64_t nrhs)
 }
 
 // Least squares for m ≥ n: B (m×nrhs) <- Qᵀ B, then B[0:n] <- R⁻¹ B[0:n],
-// with (F, τ) as stored by qrBlocked!/qrUnblocked!.  info: 1 + the first
-// zero diagonal entry of R (device int), n + 1 when R is nonsingular.
+// with (F, τ) as stored by qrBlocked!/qrUnblocked!.  info (device, two ints):
+// 1 + the first zero diagonal entry of R, n + 1 when R is nonsingular; and 1
+// when a wait gave up.
 // Qᵀ B = B − V Tᵀ Vᵀ B with T = (I + D striu(VᵀV))⁻¹ D, D = diag(τ)
 // (src/qr.jl:64-83, src/householder.jl:119-157), so TᵀW = D L⁻¹ W for the
 // unit lower L = I + stril(VᵀV) D: a solve with nrhs rows instead of T's
@@ -343,7 +349,7 @@ int qr_solve_dev(const Handle *h, hipStream_t s, int64_t m, int64_t n, int64_t n
     const size_t nr = (size_t)nrhs * n;
     T *Vw = scratch, *G = Vw + (size_t)m * n, *Gi = G + (size_t)n * n,
       *W = Gi + tile_inverse_elems(n), *Z = W + nr, *W2 = Z + nr, *split = W2 + nr;
-    hipLaunchKernelGGL(set_int_k, dim3(1), dim3(1), 0, s, info, (int)(n + 1));
+    hipLaunchKernelGGL(set_info_k, dim3(1), dim3(1), 0, s, info, (int)(n + 1));
     GLA_LAUNCH_CHECK();
     hipLaunchKernelGGL((first_zero_diag_k<T>), dim3((unsigned)cdiv(n, 256)), dim3(256), 0, s, n, F,
                        ldf, info);
@@ -363,6 +369,7 @@ int qr_solve_dev(const Handle *h, hipStream_t s, int64_t m, int64_t n, int64_t n
         p.n = n;
         p.nrhs = (int)nrhs;
         p.spin_limit = h->spin_limit;
+        p.err = info + 1;
         p.unit = 1;                       // W2 = D L⁻¹ W
         p.M = G;
         p.si = 1;
@@ -481,10 +488,14 @@ int qr_solve_entry(gla_handle_t hh, int64_t m, int64_t n, int64_t nrhs, const T 
     GLA_TRY(gla::qr_solve_dev<T>(h, s, m, n, nrhs, F, ldf, tau, B, ldb, h->dinfo + 8,
                                  reinterpret_cast<T *>(h->ws)));
     if (info) {
-        int hv = 0;
-        GLA_HIP_TRY(hipMemcpyAsync(&hv, h->dinfo + 8, sizeof(int), hipMemcpyDeviceToHost, s));
+        int hv[2] = {0, 0};
+        GLA_HIP_TRY(hipMemcpyAsync(hv, h->dinfo + 8, sizeof(hv), hipMemcpyDeviceToHost, s));
         GLA_HIP_TRY(hipStreamSynchronize(s));
-        *info = hv > n ? 0 : hv;
+        if (hv[1]) {
+            gla::set_error("least squares: a device-side wait gave up after %u polls", h->spin_limit);
+            return GLA_ERR_TIMEOUT;
+        }
+        *info = hv[0] > n ? 0 : hv[0];
     }
     return GLA_OK;
 }

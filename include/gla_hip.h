@@ -13,7 +13,11 @@
  *     argument (LAPACK style), GLA_ERR_HIP for a HIP runtime error,
  *     GLA_ERR_UNSUPPORTED for a shape this build does not handle,
  *     GLA_ERR_TIMEOUT when a bounded device-side wait gave up (the outputs
- *     of that call are then not valid).
+ *     of that call are then not valid).  Only a call that synchronises can
+ *     report that: the QR of real matrices, and those with a host `info`
+ *     pointer given.  The others (gla_symtri_*, gla_bidiag_*, the QR of
+ *     complex matrices, gla_chol_solve_*, gla_ldlt_solve_*, any call
+ *     without `info`) return GLA_OK and leave NaN in their outputs.
  *     gla_last_error_string() describes the last failure on this thread.
  *   - A handle serves one stream at a time: its workspace, grid-barrier
  *     counter, info words and side stream are shared by every call made
@@ -106,9 +110,11 @@ const char *gla_version(void);
  * trailing updates) to a direct-to-LDS kernel with a 4/3/3-deep ring of
  * 8/8/16-wide K slabs, 0 to the register-staged kernel; "gemm_lds1" (process-wide): 1 (default) stages
  * FP64 128×128 tiles through one LDS buffer, 0 through two.  Same results
- * bit for bit in every setting.  "spin_limit": polls (default 2^25, about a
- * second) before a wait of the dataflow Cholesky or a grid-wide wait of the QR panel gives up and the call
- * returns GLA_ERR_TIMEOUT.  "qr_wait_test": 1 makes every wait of a QR
+ * bit for bit in every setting.  "spin_limit": polls (default 2^25, at 0.1
+ * to 2 µs a poll some seconds to a minute) before a device-side wait gives
+ * up: in the QR panels, real and complex, the dataflow Cholesky, the
+ * triangular solves for up to 2048 right-hand sides, symtri! and
+ * bidiagonalize!.  "qr_wait_test": 1 makes every wait of a QR
  * panel, real or complex, one for an arrival that never comes (a test of
  * waits that give up; the kernels still finish, after spin_limit polls per
  * wait, the complex panel's after those of one). */
