@@ -608,7 +608,7 @@ size_t tile_inverse_elems(int64_t n);
 // (a leading stride of 1 is read first); only i ≥ j is read, and with `unit`
 // not the diagonal.  R's element (i, k) at R[i·ri + (k mod 16)·rk +
 // (k div 16)·rp], divided by div[i·ds] if div is given.  Y: tri_solve_elems
-// elements, rows of 16 per pass (element (i, k) at [(k div 16)·npad·16 + 16 i +
+// elements on 16 bytes, rows of 16 per pass (element (i, k) at [(k div 16)·npad·16 + 16 i +
 // k mod 16], npad = n rounded up to 128), and a ticket, both set by
 // tri_solve_prepare.  If `out` is given, out[i·oi + k·ok] = mul[i·ms]·y (mul
 // may be null); if X is, X[i·oi + k·ok] += y.

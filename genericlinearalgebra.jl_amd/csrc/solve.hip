@@ -330,7 +330,7 @@ int ldlt_lmul_dev(hipStream_t s, char uplo, int64_t n, int64_t nrhs, const T *F,
 size_t qr_solve_scratch(int64_t m, int64_t n, int64_t nrhs)
 {
     return (size_t)m * n + (size_t)n * n + tile_inverse_elems(n) + 3 * (size_t)nrhs * n +
-           8 * (size_t)nrhs * n + (nrhs <= kFewRhs ? 2 * tri_solve_elems(n, nrhs) : 0) + 256;
+           8 * (size_t)nrhs * n + (nrhs <= kFewRhs ? 32 + 2 * tri_solve_elems(n, nrhs) : 0) + 256;
 }
 
 // Least squares for m ≥ n: B (m×nrhs) <- Qᵀ B, then B[0:n] <- R⁻¹ B[0:n],
@@ -362,7 +362,7 @@ int qr_solve_dev(const Handle *h, hipStream_t s, int64_t m, int64_t n, int64_t n
     GLA_TRY(gemm<T>(s, 'T', 'N', 0, n, nrhs, m, T(1), Vw, m, B, ldb, T(0), W, n, 0, split, 8 * nr));
     if (nrhs <= kFewRhs) {
         const size_t ye = tri_solve_elems(n, nrhs);
-        T *Y = split + 8 * nr;
+        T *Y = scratch + (split + 8 * nr - scratch + 31) / 32 * 32;   // on 16 bytes (scratch is)
         int *ticket = reinterpret_cast<int *>(Y + 2 * ye);
         GLA_TRY(tri_solve_prepare<T>(s, (int64_t)(2 * ye), Y, ticket, 2));
         TriSolve<T> p{};

@@ -575,6 +575,10 @@ template <typename T>
 int tri_solve(hipStream_t s, TriSolve<T> p)
 {
     if (p.n <= 0 || p.nrhs <= 0) return GLA_OK;
+    if (reinterpret_cast<uintptr_t>(p.Y) % 16 != 0) {   // read 16 bytes at a time
+        set_error("tri_solve: the exchange is not aligned to 16 bytes");
+        return GLA_ERR_UNSUPPORTED;
+    }
     p.npass = (int)cdiv(p.nrhs, kSR);
     const dim3 grid((unsigned)(cdiv(p.n, kSB) * p.npass));
     if (p.si == 1 || p.si == -1)
