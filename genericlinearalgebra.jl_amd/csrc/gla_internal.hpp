@@ -484,7 +484,7 @@ struct Handle {
     int qr_lookahead = 1;
     // Block columns at least this tall are factored by the
     // reconstructed-Householder panel (0: never; -1: any height for block
-    // columns at least 32 wide, 512 rows for those at least 24, none narrower).
+    // columns at least 32 wide, otherwise by width and height: use_hr).
     int64_t qr_hr = -1;
     // Polls before a grid-wide wait of the QR panel gives up (the call then
     // returns GLA_ERR_TIMEOUT).

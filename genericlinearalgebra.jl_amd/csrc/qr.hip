@@ -1515,16 +1515,21 @@ inline int panel_rows(const Handle *h, int w)
 
 // Whether block column mm×w is factored by the reconstructed-Householder
 // path: at least as tall as wide, qr_hr rows or taller, and within the
-// fallback panel's capacity.  Auto: any height for w ≥ 32, 512 rows for
-// w ≥ 24, none for narrower ones — the path takes 125…225 µs whatever the width, the
-// column-by-column panel 4…6 µs a column.  FP64 path / panel, µs: 64×32 136 / 164,
+// fallback panel's capacity.  Auto: any height for w ≥ 32, 512 rows for w ≥ 24,
+// for 18 ≤ w < 24 from 1024 to 4096 (w − 17) rows, none for narrower ones — the
+// path takes 125…225 µs whatever the width and grows with the height, the
+// column-by-column panel 4…7 µs a column.  FP64 path / panel, µs: 64×32 136 / 164,
 // 861×63 160 / 333, 2000×63 224 / 403, 300×24 135 / 134, 861×24 137 / 164,
-// 861×16 129 / 126, 6000×8 162 / 90; FP32 64×32 125 / 131, 861×24 131 / 156.
+// 512×23 135 / 132, 2048×23 135 / 168, 16384×23 158 / 177, 2048×20 135 / 154,
+// 16384×20 157 / 156, 2048×18 134 / 145, 8192×18 148 / 144, 861×16 129 / 126,
+// 6000×8 162 / 90; FP32 64×32 125 / 131, 861×24 131 / 156, 2048×20 124 / 135.
 inline bool use_hr(const Handle *h, int64_t mm, int w)
 {
-    const int64_t minrows = h->qr_hr >= 0 ? h->qr_hr : (w >= 32 ? 1 : (w >= 24 ? 512 : INT64_MAX));
-    if (h->qr_hr == 0 || mm < w || mm < minrows || w > kQrNB) return false;
-    return cdiv(mm, panel_rows(h, w)) <= h->num_cus;
+    if (h->qr_hr == 0 || mm < w || w > kQrNB) return false;
+    const bool pays = h->qr_hr > 0 ? mm >= h->qr_hr
+                    : w >= 24     ? mm >= (w >= 32 ? 1 : 512)
+                                  : mm >= 1024 && mm <= 4096 * (int64_t)(w - 17);
+    return pays && cdiv(mm, panel_rows(h, w)) <= h->num_cus;
 }
 
 // The reconstructed-Householder panel (see hr_gram_kernel … hr_finish_kernel):

@@ -100,7 +100,8 @@ const char *gla_version(void);
  * block reflector to the rest of the trailing matrix; 0 runs the
  * reference's sequential loop.  "qr_hr": block columns at least this
  * many rows tall (−1, default: any height for block columns ≥ 32 wide,
- * 512 rows for those ≥ 24 wide, none narrower; 0: none) are factored by two
+ * 512 rows for those ≥ 24 wide, 1024 to 4096 (w − 17) rows for a width w from
+ * 18 to 23, none narrower; 0: none) are factored by two
  * CholeskyQR passes and a reconstruction of the Householder vectors from
  * the orthonormal factor (the LU of S − Q₁ with the sign choice that
  * reflector! makes), checked on the device and falling back to the
