@@ -29,8 +29,9 @@ sys.path[:0] = [os.path.join(ROOT, "genericlinearalgebra.jl_amd"), os.path.join(
 FP64_PEAK_TFLOPS = 78.6
 N_CHOL = 16384
 M_QR, N_QR, NB_QR = 8192, 4096, 128
-# the look-ahead step width cholRecursive! takes at n = 16384 (handle knob
-# chol_block −1: 1024 from n = 14336 up); the first step's trailing SYRK has K = SYRK_K
+# K of the trailing SYRK timed for the roofline, on n − 2K rows.  (cholRecursive!
+# takes 2048-wide steps at n = 16384, the same kernel with twice this K on 12288
+# rows; the shape here stays the one that earlier figures and counters are of.)
 SYRK_K = 1024
 
 
@@ -364,7 +365,8 @@ def next_rows_section(torch, gla):
     del A, W, F, L
 
     # symtri!: FP64 n = 4096; the dominant kernel is the symmetric product,
-    # which reads the trailing lower triangle once per column: Σ (n−c)²/2·8 B
+    # which reads the trailing lower triangle once per column, Σ (n−c)²/2·8 B, until
+    # the last 2048 rows, which one launch holds in registers
     n = 4096
     G = torch.randn(n, n, dtype=torch.float64, device=dev, generator=g)
     A = G + G.t()
@@ -383,7 +385,7 @@ def next_rows_section(torch, gla):
     import scipy.linalg as _sl
     lam_t = _sl.eigvalsh_tridiagonal(d, e)
     lam_a = torch.linalg.eigvalsh(A).cpu().numpy()
-    symv_bytes = sum((n - c - 1) ** 2 / 2 * 8 for c in range(n - 2))
+    symv_bytes = sum((n - c - 1) ** 2 / 2 * 8 for c in range(n - 2048))
     out["symtri_4096_fp64"] = {"ms": t * 1e3, "tflops": 4 * n ** 3 / 3 / t / 1e12,
                                "symv_bytes": symv_bytes, "symv_gbs_if_alone": symv_bytes / t / 1e9,
                                "eigenvalue_max_abs_diff_rel": float(np.max(np.abs(lam_t - lam_a))
@@ -475,7 +477,7 @@ def main():
                     help="the same with qrUnblocked! of the panel (the column-by-column "
                          "panel kernel, one launch)")
     ap.add_argument("--profile-syrk", action="store_true",
-                    help="only run the trailing SYRK of the Cholesky's first look-ahead step "
+                    help="only run a trailing SYRK of the Cholesky's look-ahead driver "
                          "(C 14336x14336 lower -= X X^T, K=1024) and a plain 64 MiB copy five "
                          "times each, for hardware-counter runs")
     ap.add_argument("--profile-batched", action="store_true",
@@ -643,10 +645,9 @@ def main():
     achieved = panel_bytes / t_panel / 1e9
     # the dominant kernel (largest share of the step's kernel time): the
     # FP64 direct-to-LDS MFMA SYRK gemm_dl_kernel<8,3,lower> of the
-    # look-ahead Cholesky, timed on its first step's shape (C 14336×14336
-    # lower -= X Xᵀ, K = 1024, the step width cholRecursive! takes at
-    # n = 16384; rankUpdate! of that shape is exactly one launch);
-    # algorithmic work mm²·K flop
+    # look-ahead Cholesky, timed on C 14336×14336 lower -= X Xᵀ, K = 1024
+    # (rankUpdate! of that shape is exactly one launch); algorithmic work
+    # mm²·K flop
     kk, mm = SYRK_K, n - 2 * SYRK_K
     Cs = torch.empty_like(A0)[:mm, :mm]
     Xs = A0[2 * kk:, :kk]

@@ -140,15 +140,6 @@ __device__ __forceinline__ void load_row4(__amdgpu_buffer_rsrc_t y, int off, flo
     const f4 a = __builtin_bit_cast(f4, __builtin_amdgcn_raw_buffer_load_b128(y, off, 0, 16));
     v[0] = a[0]; v[1] = a[1]; v[2] = a[2]; v[3] = a[3];
 }
-__device__ __forceinline__ double load_y(__amdgpu_buffer_rsrc_t y, int off, double)
-{
-    return __builtin_bit_cast(double, __builtin_amdgcn_raw_buffer_load_b64(y, off, 0, 16));
-}
-__device__ __forceinline__ float load_y(__amdgpu_buffer_rsrc_t y, int off, float)
-{
-    return __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(y, off, 0, 16));
-}
-
 template <typename T, int MODE>
 __global__ __launch_bounds__(512, 2) void tri_solve_kernel(TriSolve<T> p)
 {
