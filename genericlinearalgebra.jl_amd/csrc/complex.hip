@@ -1499,11 +1499,11 @@ int zqr_entry(gla_handle_t hh, int64_t m, int64_t n, void *Av, int64_t lda, int6
     GLA_HIP_TRY(hipSetDevice(h->device));
     // the panel's workgroups must all be resident, and every one gathers from
     // all; up to 127 of them (16256 rows) hold rows
-    const bool fits = cdiv(m, kZPRows) <= std::min(kZPMaxP, h->num_cus / 2);
     const hipStream_t s = reinterpret_cast<hipStream_t>(stream);
-    GLA_TRY(ensure_workspace(h, std::max(fits ? ZqrWS<T>(nullptr, m, n).elems : 0, zqr_scratch(m, n)) *
+    const bool one = cdiv(m, kZPRows) <= std::min(kZPMaxP, h->num_cus / 2) && !capturing(s);
+    GLA_TRY(ensure_workspace(h, std::max(one ? ZqrWS<T>(nullptr, m, n).elems : 0, zqr_scratch(m, n)) *
                                     sizeof(T)));
-    if (fits && resident_begin(h, s)) {
+    if (one && resident_begin(h, s)) {
         const int rc = zqr_blocked_dev<T>(h, s, m, n, A, lda, tau);
         const int end = resident_end(h, s);
         return rc != GLA_OK ? rc : end;

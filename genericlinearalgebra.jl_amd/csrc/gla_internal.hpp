@@ -508,6 +508,8 @@ int ensure_workspace(Handle *h, size_t bytes);
 // would have to grow while stream s is being captured
 // (the caller then takes a path without it).
 bool ensure_df(Handle *h, hipStream_t s, size_t bytes);
+// Whether s is being captured into a graph.
+bool capturing(hipStream_t s);
 
 // Launches whose workgroups wait for each other and take most of the chip
 // must not share it with another such launch: each could hold places the

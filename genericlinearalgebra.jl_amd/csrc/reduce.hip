@@ -1502,12 +1502,13 @@ __global__ void transpose_kernel(int64_t m, int64_t n, const T *A, int64_t lda, 
 }  // namespace
 
 // Workspace elements of symtri for order n.
-size_t symtri_scratch(int64_t n)
+// (resident: with the resident kernel's exchange, which a captured call never uses)
+size_t symtri_scratch(int64_t n, bool resident)
 {
     const int64_t ldv = (n + 3) / 4 * 4;
     const int64_t nbk = cdiv(n, kTB);
     const int64_t g = cdiv(n, kRPB);
-    const int64_t nr = std::min<int64_t>(n, kTRMax);   // the resident kernel's exchange
+    const int64_t nr = resident ? std::min<int64_t>(n, kTRMax) : 0;
     return 2 * (size_t)ldv * kPanel +
            std::max((size_t)nbk * n + 2 * (size_t)nbk * kPanel + 2 * g, 2 * (size_t)nr * (nr + 8)) + 64;
 }
@@ -1597,7 +1598,7 @@ template int symtri_dev<double>(Handle *, hipStream_t, char, int64_t, double *, 
 template int symtri_dev<float>(Handle *, hipStream_t, char, int64_t, float *, int64_t, float *, float *);
 
 // Workspace elements of bidiagonalize! for m×n.
-size_t bidiag_scratch(int64_t m, int64_t n)
+size_t bidiag_scratch(int64_t m, int64_t n, bool resident)
 {
     const int64_t M = std::max(m, n), N = std::min(m, n);   // the tall problem
     const int64_t ldm = (M + 3) / 4 * 4, ldn = (N + 3) / 4 * 4;
@@ -1605,7 +1606,7 @@ size_t bidiag_scratch(int64_t m, int64_t n)
     // the GEMVs' partials, or the resident kernel's exchange for the largest
     // trailing block that fits it
     size_t pe = std::max((size_t)nrb * N, (size_t)ncb * M), re = 0;
-    for (int64_t k = 0; k < N; k += kPanel)
+    for (int64_t k = 0; resident && k < N; k += kPanel)
         if (bd_resident_fits(M - k, N - k, 256)) {
             re = bd_resident_elems(M - k, N - k);
             break;
@@ -1726,8 +1727,9 @@ int symtri_entry(gla_handle_t hh, char uplo, int64_t n, T *A, int64_t lda, T *ta
     if (!tau && n > 1) { gla::set_error("tau is null"); return -6; }
     if (n == 0) return GLA_OK;
     GLA_HIP_TRY(hipSetDevice(h->device));
-    GLA_TRY(gla::ensure_workspace(h, gla::symtri_scratch(n) * sizeof(T)));
-    return gla::symtri_dev<T>(h, reinterpret_cast<hipStream_t>(stream), uplo, n, A, lda, tau,
+    const hipStream_t s = reinterpret_cast<hipStream_t>(stream);
+    GLA_TRY(gla::ensure_workspace(h, gla::symtri_scratch(n, !gla::capturing(s)) * sizeof(T)));
+    return gla::symtri_dev<T>(h, s, uplo, n, A, lda, tau,
                               reinterpret_cast<T *>(h->ws));
 }
 
@@ -1748,8 +1750,9 @@ int bidiag_entry(gla_handle_t hh, int64_t m, int64_t n, T *A, int64_t lda, T *ta
     if (!taur && nr > 0) { gla::set_error("taur is null"); return -7; }
     if (k == 0) return GLA_OK;
     GLA_HIP_TRY(hipSetDevice(h->device));
-    GLA_TRY(gla::ensure_workspace(h, gla::bidiag_scratch(m, n) * sizeof(T)));
-    return gla::bidiag_dev<T>(h, reinterpret_cast<hipStream_t>(stream), m, n, A, lda, taul, taur,
+    const hipStream_t s = reinterpret_cast<hipStream_t>(stream);
+    GLA_TRY(gla::ensure_workspace(h, gla::bidiag_scratch(m, n, !gla::capturing(s)) * sizeof(T)));
+    return gla::bidiag_dev<T>(h, s, m, n, A, lda, taul, taur,
                               reinterpret_cast<T *>(h->ws));
 }
 

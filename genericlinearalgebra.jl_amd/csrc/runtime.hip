@@ -39,15 +39,20 @@ int ensure_workspace(Handle *h, size_t bytes)
     return GLA_OK;
 }
 
+bool capturing(hipStream_t s)
+{
+    hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(s, &cap) == hipSuccess && cap == hipStreamCaptureStatusNone) return false;
+    (void)hipGetLastError();
+    return true;
+}
+
 bool ensure_df(Handle *h, hipStream_t s, size_t bytes)
 {
     // Neither the wait nor the allocation may fall into a capture, and a
     // buffer that a graph holds stays until the handle goes: then the next is
     // twice as large, so that those kept are together smaller than it.
-    hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
-    const bool eager = hipStreamIsCapturing(s, &cap) == hipSuccess &&
-                       cap == hipStreamCaptureStatusNone;
-    if (!eager) (void)hipGetLastError();
+    const bool eager = !capturing(s);
     if (bytes <= h->df_bytes) {
         h->df_captured |= !eager;
         return true;
@@ -92,14 +97,6 @@ struct ResidentChain {
     PanelCall *queued = nullptr;           // the queued ones, linked by `link`
 };
 ResidentChain g_resident[kMaxDevices];
-
-bool capturing(hipStream_t s)
-{
-    hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
-    if (hipStreamIsCapturing(s, &cap) == hipSuccess && cap == hipStreamCaptureStatusNone) return false;
-    (void)hipGetLastError();
-    return true;
-}
 }  // namespace
 
 bool resident_begin(Handle *h, hipStream_t s)
