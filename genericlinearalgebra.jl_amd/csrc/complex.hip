@@ -785,7 +785,7 @@ int zqr_panel(hipStream_t s, int64_t m, int w, T *A, int64_t lda, T *tau, T *ws)
 // The slots are filled with arrival marks beforehand, so a value announces
 // itself; every column has one of its own, and there are two sets: a panel marks
 // the other set's slots again for the next one.
-// Bound: latency.  4096×64 FP64: 296 µs, 4.6 µs a column, of which the round
+// Bound: latency.  4096×64 FP64: 290 µs, 4.5 µs a column, of which the round
 // trip through the device-coherent level takes about 2 and the chain of sums,
 // square root and update the rest; with each half of a value beside a tag, twice
 // the bytes, 317 µs; the two launches per column it replaced took 14.6 µs a

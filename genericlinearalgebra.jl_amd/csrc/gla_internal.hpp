@@ -486,11 +486,11 @@ struct Handle {
     // reconstructed-Householder panel (0: never; -1: any height for block
     // columns at least 32 wide, otherwise by width and height: use_hr).
     int64_t qr_hr = -1;
-    // Polls before a grid-wide wait of the QR panel gives up (the call then
-    // returns GLA_ERR_TIMEOUT).
+    // Polls before a device-side wait gives up (a call that synchronises then
+    // returns GLA_ERR_TIMEOUT, others leave NaN).
     unsigned spin_limit = 1u << 25;
-    // Test setting: every grid-wide wait of the QR panel targets an arrival
-    // count that never comes, so each gives up after spin_limit polls.
+    // Test setting: every wait of a QR panel, real or complex, is for an arrival
+    // that never comes, so each gives up after spin_limit polls.
     int qr_wait_test = 0;
     // CUs kept free of the look-ahead Cholesky's trailing SYRK (0: none;
     // a new handle takes num_cus/8).  When set, the driver runs its chain on
