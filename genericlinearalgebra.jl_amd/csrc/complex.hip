@@ -1363,10 +1363,10 @@ struct ZqrWS {
 // look-ahead, as qr_blocked_dev).  4096×2048 ComplexF64: 11.7 ms (45.5 with
 // 32-wide block columns, two launches per column and no look-ahead); the
 // chain of panels and next-block updates is what it takes.
-// A panel takes a CU per workgroup (150 registers, FP64), half the chip: two
-// fit beside each other, three or one beside another resident launch need not.
-// The whole call is one link of the device's chain (resident_begin): a link per
-// panel would let other calls' products in between, at two events a panel.
+// A panel takes a CU per workgroup (150 registers, FP64), up to half the chip: two
+// of the tallest fit beside each other, three or one beside another resident launch
+// need not.  The whole call counts as one such launch (resident_begin); each of its
+// panels on its own would take two events a panel.
 template <typename T>
 int zqr_blocked_dev(Handle *h, hipStream_t s0, int64_t m, int64_t n, T *A, int64_t lda, T *tau)
 {
@@ -1503,7 +1503,7 @@ int zqr_entry(gla_handle_t hh, int64_t m, int64_t n, void *Av, int64_t lda, int6
     const bool one = cdiv(m, kZPRows) <= std::min(kZPMaxP, h->num_cus / 2) && !capturing(s);
     GLA_TRY(ensure_workspace(h, std::max(one ? ZqrWS<T>(nullptr, m, n).elems : 0, zqr_scratch(m, n)) *
                                     sizeof(T)));
-    if (one && resident_begin(h, s)) {
+    if (one && resident_begin(h, s, cdiv(m, kZPRows) + 1)) {
         const int rc = zqr_blocked_dev<T>(h, s, m, n, A, lda, tau);
         const int end = resident_end(h, s);
         return rc != GLA_OK ? rc : end;

@@ -511,27 +511,29 @@ bool ensure_df(Handle *h, hipStream_t s, size_t bytes);
 // Whether s is being captured into a graph.
 bool capturing(hipStream_t s);
 
-// Launches whose workgroups wait for each other and take most of the chip
-// must not share it with another such launch: each could hold places the
-// other waits for.  resident_begin makes stream s wait for the last of them on
-// the handle's device, from any stream and thread of the process, and for the
-// PanelCalls in flight; resident_end marks the new one.  Between the two the
-// caller queues its launch; a lock is held meanwhile, so every begin is followed by its end.
+// A launch whose workgroups all wait for each other needs them all on the chip,
+// and two such launches that do not fit together could each hold places the
+// other waits for.  Each counts a whole CU per workgroup here, dealt out to the
+// dies in turn.  resident_begin makes stream s wait, on the device, for the
+// oldest such calls of the process until the new one fits beside the rest, and for
+// the PanelCalls in flight if it does not fit beside them; resident_end marks
+// the new one.  Between the two the caller queues its launches; a lock is
+// held meanwhile, so every begin is followed by its end.
 // False (nothing held): the stream is being captured, where another stream's
 // launch cannot be waited for, or an event failed.
-bool resident_begin(Handle *h, hipStream_t s);
+bool resident_begin(Handle *h, hipStream_t s, int64_t workgroups);
 int resident_end(Handle *h, hipStream_t s);
-// A call that queues panels with grid-wide waits and then waits for its stream:
-// they run beside one another, as many as fit (a panel of the QR takes up to
-// all CUs), but not beside a resident launch.  Made before the first launch;
-// queued() after the last; destroyed when the stream has been waited for.
+// A call that queues panels with grid-wide waits, of up to `workgroups` each, and
+// then waits for its stream: such calls run beside one another, but beside
+// resident calls only where all fit.  Made before the first launch; queued() after
+// the last; destroyed when the stream has been waited for.
 struct PanelCall {
-    PanelCall(Handle *h, hipStream_t s);
+    PanelCall(Handle *h, hipStream_t s, int64_t workgroups);
     void queued();
     ~PanelCall();
     PanelCall(const PanelCall &) = delete;
     hipStream_t s;
-    int device = -1;
+    int device = -1, weight = 0;
     bool is_queued = false;
     PanelCall *link = nullptr;
 };

@@ -1840,7 +1840,9 @@ int qr_entry(gla_handle_t hh, int64_t m, int64_t n, T *A, int64_t lda, int64_t b
     hipStream_t s = reinterpret_cast<hipStream_t>(stream);
     GLA_HIP_TRY(hipSetDevice(h->device));
     if (m == 0 || n == 0) return GLA_OK;
-    PanelCall panels(h, s);
+    // the widest block column's panel has the most workgroups
+    PanelCall panels(h, s, std::min<int64_t>(h->num_cus,
+                                             cdiv(m, panel_rows(h, (int)std::min<int64_t>(n, nb)))));
     GLA_TRY(qr_blocked_dev<T>(h, s, m, n, A, lda, nb, tau, work, ldwork));
     panels.queued();
     // a panel whose grid wait gave up has produced meaningless factors

@@ -398,10 +398,10 @@ __global__ __launch_bounds__(256) void tri_w_kernel(int64_t n, int64_t c, int j,
 // [g][k] in which a workgroup writes one line and a thread reads 32 bytes.
 // Each column has an exchange region of its own, filled beforehand with a
 // signalling-NaN pattern no arithmetic produces: a value is its own arrival
-// mark.  All workgroups must be resident: such launches follow one another on
-// a device, and run beside no QR panel, which waits within a launch too
-// (resident_begin).  Two workgroups fit on a CU.  A wait that gives up makes
-// the result NaN.
+// mark.  All workgroups must be resident: such launches, and the QR panels,
+// which wait within a launch too, run beside one another only where all fit
+// (resident_begin).  Two workgroups fit on a CU, but none beside a panel's.  A
+// wait that gives up makes the result NaN.
 // Bound: latency.  n = 2048 FP64: 10.4 ms, 5.1 µs a column (3.2 at n = 512),
 // about half of it the exchange; the three launches per column of the
 // deferred form took 38 ms.  With p and the row in index order (eight
@@ -692,9 +692,10 @@ inline bool tri_resident_fits(int64_t n, int num_cus)
 template <typename T>
 int tri_resident(Handle *h, hipStream_t s, int64_t n, T *A, int64_t lda, T *tau, T *xch, bool *done)
 {
-    *done = resident_begin(h, s);
+    const int64_t P = cdiv(n, kTRRows);
+    *done = resident_begin(h, s, P);
     if (!*done) return GLA_OK;
-    const int64_t P = cdiv(n, kTRRows), cnt = n * 2 * P * kTRRows;
+    const int64_t cnt = n * 2 * P * kTRRows;
     hipLaunchKernelGGL((mark_kernel<T>), dim3((unsigned)cdiv(cnt, 256)), dim3(256), 0, s, cnt, xch);
     const TriResP<T> q{A, lda, (int)n, tau, xch, h->spin_limit};
     hipLaunchKernelGGL((tri_resident_kernel<T>), dim3((unsigned)P), dim3((unsigned)cdiv(2 * P, 64) * 64),
@@ -1462,7 +1463,7 @@ template <typename T>
 int bd_resident(Handle *h, hipStream_t s, int64_t m, int64_t n, T *A, int64_t lda, T *taul, T *taur,
                 T *ws, bool *done)
 {
-    *done = resident_begin(h, s);
+    *done = resident_begin(h, s, cdiv(m, kBRLoc) * cdiv(n, kBRLoc));
     if (!*done) return GLA_OK;
     BdResP<T> q;
     q.A = A;

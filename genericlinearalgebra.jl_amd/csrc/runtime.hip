@@ -1,4 +1,5 @@
 // Handle, workspace and error reporting of libgla_hip.so.
+#include <algorithm>
 #include <condition_variable>
 #include <cstdarg>
 #include <cstring>
@@ -87,35 +88,114 @@ bool ensure_df(Handle *h, hipStream_t s, size_t bytes)
 
 namespace {
 constexpr int kMaxDevices = 64;
-struct ResidentChain {
+constexpr int kDies = 8;                   // workgroups go to the dies in turn
+struct ResidentCall {                      // the last such call of a stream
+    hipEvent_t done = nullptr;
+    hipStream_t s = nullptr;
+    int weight = 0;
+};
+struct ResidentCalls {
     std::mutex lock;
     std::condition_variable turn;
-    hipEvent_t last = nullptr;             // the last resident launch, once recorded
-    hipEvent_t panels = nullptr;           // (reused for every stream waited for)
     unsigned long next = 0, serving = 0;   // callers take turns in the order they come
-    int queueing = 0;                      // PanelCalls not yet queued
-    PanelCall *queued = nullptr;           // the queued ones, linked by `link`
+    static constexpr int kMax = 32;
+    ResidentCall call[kMax];               // those in flight, oldest first: call[0 … n)
+    int n = 0;
+    PanelCall *queued = nullptr;           // queued PanelCalls, linked by `link`
+    int queueing = 0;                      // those not yet queued
+    int panels = 0;                        // weight of both
+    hipEvent_t panel_done = nullptr;       // (reused for every stream waited for)
+    int mine = 0, replaces = -1;           // of the call that holds the lock: weight, its stream's entry
+
+    void drop(int i)                       // its event goes to a later call
+    {
+        std::rotate(call + i, call + i + 1, call + n);
+        --n;
+    }
+    // Drops what has finished; the weight of the rest.
+    int in_flight()
+    {
+        int w = 0;
+        for (int i = 0; i < n;) {
+            if (hipEventQuery(call[i].done) == hipSuccess) {
+                drop(i);
+            } else {
+                (void)hipGetLastError();
+                w += call[i++].weight;
+            }
+        }
+        return w;
+    }
+    // s waits for the oldest calls until those left weigh `room` at most.
+    hipError_t make_room(hipStream_t s, int room)
+    {
+        hipError_t e = hipSuccess;
+        int w = in_flight();
+        for (int i = 0; i < n && w > room && e == hipSuccess; ++i) {
+            e = hipStreamWaitEvent(s, call[i].done, 0);
+            w -= call[i].weight;
+        }
+        return e;
+    }
 };
-ResidentChain g_resident[kMaxDevices];
+ResidentCalls g_resident[kMaxDevices];
+
+// Another thread's capture in the global mode forbids this one event queries and
+// the like; none of those made here touches a captured stream.
+struct RelaxedCapture {
+    hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+    RelaxedCapture() { (void)hipThreadExchangeStreamCaptureMode(&mode); }
+    ~RelaxedCapture() { (void)hipThreadExchangeStreamCaptureMode(&mode); }
+};
+
+int weight_of(int64_t workgroups) { return (int)cdiv(workgroups, kDies); }
+int room_of(const Handle *h) { return std::max(1, h->num_cus / kDies); }
 }  // namespace
 
-bool resident_begin(Handle *h, hipStream_t s)
+bool resident_begin(Handle *h, hipStream_t s, int64_t workgroups)
 {
     if (h->device < 0 || h->device >= kMaxDevices || capturing(s)) return false;
-    ResidentChain &c = g_resident[h->device];
+    ResidentCalls &c = g_resident[h->device];
+    const RelaxedCapture relaxed;
+    const int room = room_of(h), w = std::min(room, weight_of(workgroups));
     std::unique_lock<std::mutex> lk(c.lock);
     const unsigned long mine = c.next++;
-    c.turn.wait(lk, [&] { return c.serving == mine && c.queueing == 0; });
+    c.turn.wait(lk, [&] {
+        return c.serving == mine && (c.panels + w <= room || c.queueing == 0);
+    });
     hipError_t e = hipSuccess;
-    for (hipEvent_t *ev : {&c.last, &c.panels})
-        if (!*ev && e == hipSuccess) {
-            e = hipEventCreateWithFlags(ev, hipEventDisableTiming);
-            if (e != hipSuccess) *ev = nullptr;
+    if (!c.panel_done) {
+        e = hipEventCreateWithFlags(&c.panel_done, hipEventDisableTiming);
+        if (e != hipSuccess) c.panel_done = nullptr;
+    }
+    int panels = c.panels;
+    if (e == hipSuccess && panels + w > room) {
+        for (const PanelCall *q = c.queued; q && e == hipSuccess; q = q->link) {
+            e = hipEventRecord(c.panel_done, q->s);
+            if (e == hipSuccess) e = hipStreamWaitEvent(s, c.panel_done, 0);
         }
-    if (e == hipSuccess) e = hipStreamWaitEvent(s, c.last, 0);
-    for (const PanelCall *q = c.queued; q; q = q->link) {
-        if (e == hipSuccess) e = hipEventRecord(c.panels, q->s);
-        if (e == hipSuccess) e = hipStreamWaitEvent(s, c.panels, 0);
+        panels = 0;
+    }
+    c.mine = w;
+    if (e == hipSuccess) e = c.make_room(s, room - w - panels);
+    // one entry a stream: the new call follows the stream's last one (waited for
+    // too, should the handle be another stream's by now), and weighs as much as
+    // either until it is done
+    c.replaces = -1;
+    for (int i = 0; i < c.n; ++i)
+        if (c.call[i].s == s) {
+            if (e == hipSuccess) e = hipStreamWaitEvent(s, c.call[i].done, 0);
+            c.mine = std::max(c.mine, c.call[i].weight);
+            c.replaces = i;
+        }
+    if (c.replaces < 0 && c.n == ResidentCalls::kMax) {
+        // no entry left: after all of them, and none beside it
+        for (int i = 0; i < c.n && e == hipSuccess; ++i) e = hipStreamWaitEvent(s, c.call[i].done, 0);
+        if (e == hipSuccess) c.n = 0;
+        c.mine = room;
+    } else if (c.replaces < 0 && !c.call[c.n].done && e == hipSuccess) {
+        e = hipEventCreateWithFlags(&c.call[c.n].done, hipEventDisableTiming);
+        if (e != hipSuccess) c.call[c.n].done = nullptr;
     }
     if (e != hipSuccess) {
         (void)hipGetLastError();
@@ -130,8 +210,13 @@ bool resident_begin(Handle *h, hipStream_t s)
 
 int resident_end(Handle *h, hipStream_t s)
 {
-    ResidentChain &c = g_resident[h->device];
-    const hipError_t e = hipEventRecord(c.last, s);
+    ResidentCalls &c = g_resident[h->device];
+    if (c.replaces >= 0) c.drop(c.replaces);
+    ResidentCall &r = c.call[c.n];
+    const hipError_t e = hipEventRecord(r.done, s);
+    r.s = s;
+    r.weight = c.mine;
+    ++c.n;
     ++c.serving;
     c.lock.unlock();
     c.turn.notify_all();
@@ -139,17 +224,20 @@ int resident_end(Handle *h, hipStream_t s)
     return GLA_OK;
 }
 
-PanelCall::PanelCall(Handle *h, hipStream_t stream) : s(stream)
+PanelCall::PanelCall(Handle *h, hipStream_t stream, int64_t workgroups) : s(stream)
 {
     if (h->device < 0 || h->device >= kMaxDevices || capturing(s)) return;
+    const RelaxedCapture relaxed;
     device = h->device;
-    ResidentChain &c = g_resident[device];
+    ResidentCalls &c = g_resident[device];
+    weight = weight_of(workgroups);
     std::unique_lock<std::mutex> lk(c.lock);
     const unsigned long mine = c.next++;
     c.turn.wait(lk, [&] { return c.serving == mine; });
     ++c.serving;
     ++c.queueing;
-    if (c.last && hipStreamWaitEvent(s, c.last, 0) != hipSuccess) (void)hipGetLastError();
+    c.panels += weight;
+    if (c.make_room(s, room_of(h) - c.panels) != hipSuccess) (void)hipGetLastError();
     lk.unlock();
     c.turn.notify_all();
 }
@@ -157,7 +245,7 @@ PanelCall::PanelCall(Handle *h, hipStream_t stream) : s(stream)
 void PanelCall::queued()
 {
     if (device < 0) return;
-    ResidentChain &c = g_resident[device];
+    ResidentCalls &c = g_resident[device];
     {
         std::lock_guard<std::mutex> lk(c.lock);
         link = c.queued;
@@ -171,7 +259,7 @@ void PanelCall::queued()
 PanelCall::~PanelCall()
 {
     if (device < 0) return;
-    ResidentChain &c = g_resident[device];
+    ResidentCalls &c = g_resident[device];
     {
         std::lock_guard<std::mutex> lk(c.lock);
         if (is_queued) {
@@ -181,6 +269,7 @@ PanelCall::~PanelCall()
         } else {
             --c.queueing;
         }
+        c.panels -= weight;
     }
     c.turn.notify_all();
 }
