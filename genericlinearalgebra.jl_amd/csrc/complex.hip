@@ -1323,6 +1323,9 @@ int zwy_apply_dev(hipStream_t s, char trans, int64_t mA, int64_t nA, int64_t b, 
 // products of a 32-row panel by n columns (or of a 32×32 Gram matrix).
 inline int64_t zqr_part_elems(int64_t n) { return 2 * 16 * (int64_t)kZQ * std::max<int64_t>(n, kZQ); }
 
+template <typename T>
+constexpr int64_t kZLookFrom = sizeof(T) == 8 ? 4500000 : 16000000;
+
 // Workspace of zqr_blocked_dev in elements of T, every part on 32 elements:
 // two (V, T) panel sets and two (W1, W2, split-K) update sets, since the side
 // stream updates with one while the next panel fills the other; the panels'
@@ -1360,7 +1363,12 @@ struct ZqrWS {
 // whatever the block size (the factors do not depend on it): the panel and
 // its T by one launch, then Hᴴ on the next block column, on which the next
 // panel starts while the side stream applies Hᴴ to the rest (depth-1
-// look-ahead, as qr_blocked_dev).  4096×2048 ComplexF64: 11.7 ms (45.5 with
+// look-ahead, as qr_blocked_dev).  Matrices of fewer than kZLookFrom elements go
+// without: the products are then too short to pay for the events, and the
+// handle's streams crowd out other callers'.  On / off: ComplexF64 1500×500 2.72 /
+// 2.55 ms (four streams at once 2.61 / 0.67 a call), 3000×1000 5.55 / 5.43,
+// 2048×2048 12.1 / 12.1, 3000×1500 8.39 / 8.49, 8000×1000 6.48 / 6.79; ComplexF32
+// 3000×3000 16.8 / 16.4, 4096×4096 23.6 / 23.7.  4096×2048 ComplexF64: 11.7 ms (45.5 with
 // 32-wide block columns, two launches per column and no look-ahead); the
 // chain of panels and next-block updates is what it takes.
 // A panel takes a CU per workgroup (150 registers, FP64), up to half the chip: two
@@ -1372,7 +1380,7 @@ int zqr_blocked_dev(Handle *h, hipStream_t s0, int64_t m, int64_t n, T *A, int64
 {
     const int64_t k = std::min(m, n);
     const ZqrWS<T> ws(reinterpret_cast<T *>(h->ws), m, n);   // zqr_entry has made it large enough
-    const bool la = h->qr_lookahead && cdiv(k, (int64_t)kZP) > 2;
+    const bool la = h->qr_lookahead && cdiv(k, (int64_t)kZP) > 2 && m * n >= kZLookFrom<T>;
     const bool masked = la && h->masked != nullptr;
     hipStream_t s = masked ? h->chain : s0, side = masked ? h->masked : h->side;
     hipLaunchKernelGGL((zqr_clear_kernel<T>), dim3((unsigned)cdiv(2 * ws.xch_elems, 256)), dim3(256),

@@ -97,7 +97,8 @@ const char *gla_version(void);
  * 0 factors it in one panel launch; −1 (default) takes 64 for block columns
  * taller than 12288 rows and 0 otherwise.  "qr_lookahead": 1 (default)
  * factors the next QR panel while the side stream applies the current
- * block reflector to the rest of the trailing matrix; 0 runs the
+ * block reflector to the rest of the trailing matrix (complex matrices from
+ * 4.5 million elements, ComplexF32 16 million); 0 runs the
  * reference's sequential loop.  "qr_hr": block columns at least this
  * many rows tall (−1, default: any height for block columns ≥ 32 wide,
  * 512 rows for those ≥ 24 wide, 1024 to 4096 (w − 17) rows for a width w from
